@@ -146,7 +146,7 @@ struct Ctx {
   double *th_q1 = nullptr;     // [ny-1][nx] border solution
   double *th_den = nullptr;    // [nx]
   double *th_last = nullptr;   // [nx] q[n-1] of the current solve
-  unsigned char *th_flag = nullptr;  // [ny-1][nx] zero-pivot flags
+  bool th_zero_pivot = false;  // some factor of th_val is 0: a zero pivot (tdm.c:44-47)
   // partition solver tables
   int part_L = 0, part_P = 0;
   // tuned launch shapes (eif_gpu_autotune); 0 is the built-in default

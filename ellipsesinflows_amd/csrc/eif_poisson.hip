@@ -828,115 +828,208 @@ __global__ __launch_bounds__((1 << LOGN) >> dct_logr<LOGN>(), 4) void k_project_
 }
 
 // ---------------------------------------------------------------------
-// Thomas mode: one lane per wavenumber k, sweeps along j
+// Thomas mode: one lane per wavenumber k, sweeps along j.
+//
+// Each sweep is one dependent chain of ny rows per wavenumber (three FP64
+// operations a row forward, two backward, in the reference's order), so the
+// time is the chain's as long as its operands are there.  A workgroup takes
+// TH_K = 16 wavenumbers (one 128-byte line of every row, so that nx / 16
+// CUs share the traffic): wave 0 walks the chain over tiles of TH_R rows in
+// LDS, and four helper waves move the tiles: while wave 0 is on tile t they
+// store the results of tile t - 1, put tile t + 1 (held in registers since
+// the last phase) in its place and issue the loads of tile t + 2, about two
+// phases (3 us) before they are needed.  A helper thread moves the same
+// elements in both sweeps, so the backward sweep's loads of a row follow
+// that thread's own stores of it.  The last two tiles of the forward sweep
+// stay in LDS for the backward one.
+// FLAG: some pivot of the tables is zero (rv == 0 there: the reference
+// writes 0); without one the chain has no select.
+// One wave per 64 wavenumbers with register look-ahead, all it replaced,
+// waited for its loads: 92 -> 8.6 us at 128x128, 773 -> 43 at 512x1024,
+// 1617 -> 81 at 1024x2048, 3648 -> 157 at 2048x4096 (38 ns a row for both
+// sweeps; the chain alone is about 40 cycles, 17 ns).
 // ---------------------------------------------------------------------
-struct ThomasB {
-  static constexpr int T = 64, M = 0;
-  static __device__ __forceinline__ void run(const VB &vb, int nx, int ny, double *q,
-                                               const double *__restrict__ rv,
-                                               const double *__restrict__ um,
-                                               const unsigned char *__restrict__ flag,
-                                               const double *__restrict__ cdiag,
-                                               const double *__restrict__ den,
-                                               double coef, double *last) {
-  const int k = vb.bx * blockDim.x + threadIdx.x;
-  if (k >= nx) return;
-  const int n1 = ny - 1;  // size of the bordered (n-1) system
-  const double l = coef;  // l = u = 1/dy/dy everywhere
-  // forward sweep (tdm.c:40-53) on rows 0..n-2.  The sweeps are one
-  // dependent chain per wavenumber: the rows' loads are issued a batch of
-  // TH_U rows ahead of the arithmetic (same operations, same order).
-  constexpr int TH_U = 16;
-  double prev = q[k] / cdiag[k];
-  q[k] = prev;
-  {
-    const int iend = n1 - 1;  // last row of the forward sweep
-    double qa[TH_U], ra[TH_U];
-    bool fa[TH_U];
-    auto load = [&](int i0, double *qv, double *rw, bool *fl) {
-#pragma unroll
-      for (int u = 0; u < TH_U; u++) {
-        const int ii = i0 + u;
-        if (ii <= iend) {
-          const long o = (long)ii * nx + k;
-          qv[u] = q[o];
-          rw[u] = rv[o];
-          fl[u] = flag[o] != 0;
-        }
-      }
-    };
-    load(1, qa, ra, fa);
-    for (int i = 1; i <= iend; i += TH_U) {
-      double qb[TH_U] = {}, rb[TH_U] = {};
-      bool fb[TH_U] = {};
-      if (i + TH_U <= iend) load(i + TH_U, qb, rb, fb);  // later rows: not yet written
-#pragma unroll
-      for (int u = 0; u < TH_U; u++) {
-        const int ii = i + u;
-        if (ii > iend) break;
-        const double v = fa[u] ? 0. : ra[u] * (qa[u] - l * prev);
-        q[(long)ii * nx + k] = v;
-        prev = v;
-      }
-#pragma unroll
-      for (int u = 0; u < TH_U; u++) {
-        qa[u] = qb[u];
-        ra[u] = rb[u];
-        fa[u] = fb[u];
-      }
-    }
-  }
-  // backward sweep (:55-57), loads a batch ahead in the same way
-  const double q_last_fwd = prev;  // q0[n-2]
-  double next = prev;
-  {
-    double qa[TH_U], ua[TH_U];
-    auto load = [&](int i0, double *qv, double *uw) {
-#pragma unroll
-      for (int u = 0; u < TH_U; u++) {
-        const int ii = i0 - u;
-        if (ii >= 0) {
-          const long o = (long)ii * nx + k;
-          qv[u] = q[o];
-          uw[u] = um[o];
-        }
-      }
-    };
-    load(n1 - 2, qa, ua);
-    for (int i = n1 - 2; i >= 0; i -= TH_U) {
-      double qb[TH_U] = {}, ub[TH_U] = {};
-      if (i - TH_U >= 0) load(i - TH_U, qb, ub);  // earlier rows: not yet written
-#pragma unroll
-      for (int u = 0; u < TH_U; u++) {
-        const int ii = i - u;
-        if (ii < 0) break;
-        const double v = qa[u] - ua[u] * next;
-        q[(long)ii * nx + k] = v;
-        next = v;
-      }
-#pragma unroll
-      for (int u = 0; u < TH_U; u++) {
-        qa[u] = qb[u];
-        ua[u] = ub[u];
-      }
-    }
-  }
-  // bottom solution (tdm.c:99-102)
-  const double q0_0 = next;
-  const double num = q[(long)(ny - 1) * nx + k] - l * q0_0 - l * q_last_fwd;
-  const double d = den[k];
-  const double xl = fabs(d) < DBL_EPSILON ? 0. : num / d;
-  last[k] = xl;
-}
+constexpr int TH_K = 16;
+constexpr int TH_R = 128;
+constexpr int TH_HELP = 256;                     // helper threads
+constexpr int TH_E = TH_R * TH_K / TH_HELP;      // elements a helper moves per tile
+constexpr int TH_THREADS = 64 + TH_HELP;
+
+struct ThPair {
+  double q, a;  // the right-hand side (then the result) and the table factor
 };
-__global__ __launch_bounds__(64) void k_thomas(int nx, int ny, double *q,
-                                               const double *__restrict__ rv,
-                                               const double *__restrict__ um,
-                                               const unsigned char *__restrict__ flag,
-                                               const double *__restrict__ cdiag,
-                                               const double *__restrict__ den,
-                                               double coef, double *last) {
-  ThomasB::run(VB::here(), nx, ny, q, rv, um, flag, cdiag, den, coef, last);
+
+// N rows of the chain from row r of the tile, operands read ahead of it
+template <bool FLAG, int N>
+__device__ __forceinline__ void th_fwd_rows(ThPair *t, int r, double l, double &prev) {
+  ThPair v[N];
+#pragma unroll
+  for (int u = 0; u < N; u++) v[u] = t[(r + u) * TH_K];
+#pragma unroll
+  for (int u = 0; u < N; u++) {
+    const double w = FLAG && v[u].a == 0. ? 0. : v[u].a * (v[u].q - l * prev);
+    t[(r + u) * TH_K].q = w;
+    prev = w;
+  }
+}
+// rows r, r - 1, ..., r - N + 1
+template <int N>
+__device__ __forceinline__ void th_bwd_rows(ThPair *t, int r, double &next) {
+  ThPair v[N];
+#pragma unroll
+  for (int u = 0; u < N; u++) v[u] = t[(r - u) * TH_K];
+#pragma unroll
+  for (int u = 0; u < N; u++) {
+    const double w = v[u].q - v[u].a * next;
+    t[(r - u) * TH_K].q = w;
+    next = w;
+  }
+}
+
+template <bool FLAG>
+struct ThomasB {
+  static constexpr int T = TH_THREADS, M = 0;
+  static __device__ __forceinline__ void run(const VB &vb, int nx, int ny, double *q,
+                                             const double *__restrict__ rv,
+                                             const double *__restrict__ um,
+                                             const double *__restrict__ cdiag,
+                                             const double *__restrict__ den, double coef,
+                                             double *last) {
+    __shared__ ThPair tile[2][TH_R * TH_K];
+    const int k0 = vb.bx * TH_K;
+    const int rows = ny - 1;          // rows 0 .. ny-2 of the bordered system
+    const int tl = (rows - 1) / TH_R;  // last tile
+    const double l = coef;             // l = u = 1/dy/dy everywhere
+    const bool helper = threadIdx.x >= 64;
+    // helper: element m is row (h >> 4) + 16 m of the tile, wavenumber h & 15
+    const int h = (int)threadIdx.x - 64, hr = h >> 4, hk = k0 + (h & (TH_K - 1));
+    const bool hon = hk < nx;
+    const int hkc = min(hk, nx - 1);
+    constexpr int HS = TH_HELP / TH_K;  // rows between a helper's elements
+    double rq[TH_E], ra[TH_E];
+    auto fetch = [&](int t, const double *__restrict__ tab) {
+#pragma unroll
+      for (int m = 0; m < TH_E; m++) {
+        const long o = (long)min(t * TH_R + hr + HS * m, rows - 1) * nx + hkc;
+        rq[m] = q[o];
+        ra[m] = tab[o];
+      }
+    };
+    auto fetch_a2 = [&]() {
+#pragma unroll
+      for (int m = 0; m < TH_E; m++) {
+        const int i = tl * TH_R + hr + HS * m;
+        ra[m] = um[(long)min(i, rows - 1) * nx + hkc];
+        rq[m] = um[(long)min(max(i - TH_R, 0), rows - 1) * nx + hkc];
+      }
+    };
+    auto place = [&](ThPair *b) {
+#pragma unroll
+      for (int m = 0; m < TH_E; m++) b[h + TH_HELP * m] = ThPair{rq[m], ra[m]};
+    };
+    auto place_a = [&](ThPair *b, const double *v) {
+#pragma unroll
+      for (int m = 0; m < TH_E; m++) b[h + TH_HELP * m].a = v[m];
+    };
+    auto store = [&](int t, const ThPair *b) {
+#pragma unroll
+      for (int m = 0; m < TH_E; m++) {
+        const int i = t * TH_R + hr + HS * m;
+        if (hon && i < rows) q[(long)i * nx + hk] = b[h + TH_HELP * m].q;
+      }
+    };
+    // the chain's lanes
+    const int kk = threadIdx.x, k = k0 + kk;
+    const bool chain = !helper && kk < TH_K;
+    const int kc = min(k, nx - 1);
+    double cd = 1., dn = 1., qb = 0.;
+    if (helper) {
+      fetch(0, rv);
+      place(tile[0]);
+      if (tl > 0) fetch(1, rv);
+    } else if (chain) {
+      cd = cdiag[kc];
+      dn = den[kc];
+      qb = q[(long)rows * nx + kc];
+      __builtin_amdgcn_s_setprio(3);
+    }
+    __syncthreads();
+    // forward sweep (tdm.c:40-53) on rows 0..n-2
+    double prev = 0.;
+    for (int t = 0; t <= tl; t++) {
+      if (helper) {
+        ThPair *b = tile[(t + 1) & 1];
+        if (t > 0 && t - 1 < tl - 1) store(t - 1, b);
+        if (t < tl) place(b);
+        if (t + 2 <= tl)
+          fetch(t + 2, rv);
+        else if (t == tl)  // the backward sweep's factors of the last two tiles
+          fetch_a2();
+      } else if (chain) {
+        ThPair *b = tile[t & 1] + kk;
+        const int n = min(TH_R, rows - t * TH_R);
+        int r = 0;
+        if (t == 0) {
+          prev = b[0].q / cd;
+          b[0].q = prev;
+          r = 1;
+          if (n >= 16) {
+            th_fwd_rows<FLAG, 15>(b, 1, l, prev);
+            r = 16;
+          }
+        }
+        for (; r + 16 <= n; r += 16) th_fwd_rows<FLAG, 16>(b, r, l, prev);
+        for (; r + 4 <= n; r += 4) th_fwd_rows<FLAG, 4>(b, r, l, prev);
+        for (; r < n; r++) th_fwd_rows<FLAG, 1>(b, r, l, prev);
+      }
+      __syncthreads();
+    }
+    // backward sweep (:55-57), the factors in the place of rv; the results
+    // of the last two tiles are still in LDS
+    if (helper) {
+      place_a(tile[tl & 1], ra);
+      if (tl > 0) place_a(tile[(tl - 1) & 1], rq);
+      if (tl > 1) fetch(tl - 2, um);
+    }
+    __syncthreads();
+    const double q_last_fwd = prev;  // q0[n-2]
+    double next = prev;
+    for (int t = tl; t >= 0; t--) {
+      if (helper) {
+        ThPair *b = tile[(t + 1) & 1];
+        if (t < tl) store(t + 1, b);
+        if (t < tl && t >= 1) {
+          place(b);
+          if (t >= 2) fetch(t - 2, um);
+        }
+      } else if (chain) {
+        ThPair *b = tile[t & 1] + kk;
+        int r = min(TH_R, rows - t * TH_R) - 1;
+        if (t == tl) r--;  // the last row holds the forward sweep's value
+        for (; r >= 15; r -= 16) th_bwd_rows<16>(b, r, next);
+        for (; r >= 3; r -= 4) th_bwd_rows<4>(b, r, next);
+        for (; r >= 0; r--) th_bwd_rows<1>(b, r, next);
+      }
+      __syncthreads();
+    }
+    if (helper) {
+      store(0, tile[0]);
+    } else if (chain && k < nx) {
+      // bottom solution (tdm.c:99-102)
+      const double q0_0 = next;
+      const double num = qb - l * q0_0 - l * q_last_fwd;
+      last[k] = fabs(dn) < DBL_EPSILON ? 0. : num / dn;
+    }
+  }
+};
+template <bool FLAG>
+__global__ __launch_bounds__(TH_THREADS) void k_thomas(int nx, int ny, double *q,
+                                                       const double *__restrict__ rv,
+                                                       const double *__restrict__ um,
+                                                       const double *__restrict__ cdiag,
+                                                       const double *__restrict__ den,
+                                                       double coef, double *last) {
+  ThomasB<FLAG>::run(VB::here(), nx, ny, q, rv, um, cdiag, den, coef, last);
 }
 
 // ---------------------------------------------------------------------
@@ -1350,7 +1443,6 @@ int poisson_init(Ctx *c) {
   const int n1 = ny - 1;
   std::vector<double> cdiag(nx), den(nx);
   std::vector<double> rv((size_t)n1 * nx), um((size_t)n1 * nx), q1((size_t)n1 * nx);
-  std::vector<unsigned char> flg((size_t)n1 * nx);
   std::vector<double> uu(n1), qq(n1);
   for (int k = 0; k < nx; k++) {
     // eigenvalue, compute_potential.c:103-106 (pow(., 2.) is a product)
@@ -1367,20 +1459,18 @@ int poisson_init(Ctx *c) {
     qq[0] = qq[0] / cc;
     rv[k] = 0.;
     um[k] = uu[0];
-    flg[k] = 0;
     for (int i = 1; i <= n1 - 1; i++) {
       double val = cc - l * uu[i - 1];
       const size_t o = (size_t)i * nx + k;
       if (fabs(val) < DBL_EPSILON) {
         uu[i] = 0.;
         qq[i] = 0.;
-        flg[o] = 1;
+        c->th_zero_pivot = true;
         rv[o] = 0.;
       } else {
         val = 1. / val;
         uu[i] = val * uu[i];
         qq[i] = val * (qq[i] - l * qq[i - 1]);
-        flg[o] = 0;
         rv[o] = val;
       }
       um[o] = uu[i];
@@ -1392,13 +1482,11 @@ int poisson_init(Ctx *c) {
   EIF_HIP(hipMalloc(&c->th_val, rv.size() * sizeof(double)));
   EIF_HIP(hipMalloc(&c->th_u, um.size() * sizeof(double)));
   EIF_HIP(hipMalloc(&c->th_q1, q1.size() * sizeof(double)));
-  EIF_HIP(hipMalloc(&c->th_flag, flg.size()));
   EIF_HIP(hipMalloc(&c->th_den, 2 * (size_t)nx * sizeof(double)));
   EIF_HIP(hipMalloc(&c->th_last, (size_t)nx * sizeof(double)));
   EIF_HIP(hipMemcpy(c->th_val, rv.data(), rv.size() * sizeof(double), hipMemcpyHostToDevice));
   EIF_HIP(hipMemcpy(c->th_u, um.data(), um.size() * sizeof(double), hipMemcpyHostToDevice));
   EIF_HIP(hipMemcpy(c->th_q1, q1.data(), q1.size() * sizeof(double), hipMemcpyHostToDevice));
-  EIF_HIP(hipMemcpy(c->th_flag, flg.data(), flg.size(), hipMemcpyHostToDevice));
   EIF_HIP(hipMemcpy(c->th_den, den.data(), nx * sizeof(double), hipMemcpyHostToDevice));
   EIF_HIP(hipMemcpy(c->th_den + nx, cdiag.data(), nx * sizeof(double), hipMemcpyHostToDevice));
   return part_init(c);
@@ -1558,9 +1646,13 @@ static int poisson_lines(Ctx *c, int rk, const double *rhs_add, CombineArgs *out
     ca.bnd = c->pt_bnd;
   } else {
     ProfScope ps(c, "thomas");
-    go<ThomasB>(k_thomas, dim3((nx + 63) / 64), dim3(64), 0, c->stream, nx, ny,
-                       c->qhat, c->th_val, c->th_u, c->th_flag, c->th_den + nx,
-                       c->th_den, l, c->th_last);
+    const dim3 g((nx + TH_K - 1) / TH_K);
+    if (c->th_zero_pivot)
+      go<ThomasB<true>>(k_thomas<true>, g, dim3(TH_THREADS), 0, c->stream, nx, ny, c->qhat,
+                        c->th_val, c->th_u, c->th_den + nx, c->th_den, l, c->th_last);
+    else
+      go<ThomasB<false>>(k_thomas<false>, g, dim3(TH_THREADS), 0, c->stream, nx, ny, c->qhat,
+                         c->th_val, c->th_u, c->th_den + nx, c->th_den, l, c->th_last);
     EIF_HIP(hipGetLastError());
     ca.mode = 0;
     ca.q1 = c->th_q1;
