@@ -228,73 +228,227 @@ __device__ inline double rhs_value_add(const Layout &L, const double *ux, const 
   return fac * (div + fac * add[L.p(i + 1, j)]);
 }
 
-// How a one-row kernel transforms a row of n values: logn >= 0, the
-// radix-2 LDS FFT of n = 2^logn; otherwise the Stockham FFT with the stage
-// radices r[0..nr) (n's prime factors in increasing order)
-struct DctPlan {
-  int logn;
-  int nr;
-  int r[24];
+// ---------------------------------------------------------------------
+// Stockham autosort FFT of any length n in LDS (sign -1 forward, +1
+// backward, unnormalised), the stage radices being n's prime factors in
+// increasing order.  In the stage of radix R after radices of product Ns,
+// butterfly j (k = j mod Ns) takes v_r = x[j + r n/R] w^(k r),
+// w = e^(sign 2 pi i / (Ns R)), and stores sum_r v_r e^(sign 2 pi i q r / R)
+// at (j / Ns) Ns R + k + q Ns.  Factors with exponent 0 are not multiplied;
+// the oracle's fft_mixed performs the same operations in the same order.
+//
+// Up to three consecutive stages run on one thread's registers between two
+// visits to LDS: with N = n / (R1 R2 R3), the butterflies j = g + b3 N +
+// b2 N R3 of the first stage feed only the group g's butterflies of the
+// next two, so a row of 768 = 2^8 3 points takes 3 LDS passes instead of 9.
+// Radices above 7 sum over LDS, every thread MIX_BQ outputs at a time.
+// The roots come from the table W[e] = (cos, sin)(2 pi e / n) of the entries
+// of C (the first exactly 1, 0): one load instead of two index foldings.
+// One row per workgroup, its threads the most groups any pass has.
+// Bound by the FP64 sums (R^2 a butterfly, as the oracle has them) and the
+// LDS passes.  DCT-II kernel, against one LDS pass a prime, R-fold repeated
+// twiddles and 64-bit index foldings: 12.9 -> 5.7 us at 48x96, 53 -> 14 at
+// 375x900, 64 -> 27 at 768x1536, 458 -> 116 at 1500x3000, 104700 -> 240 at
+// the prime 499x1000 (DCT-III alike).
+// ---------------------------------------------------------------------
+constexpr int MIX_PASSES = 16;
+constexpr int MIX_BQ = 4;
+constexpr int MIX_T_MAX = 512;
+
+struct MixPlan {
+  int n, np, threads;
+  int sh;     // LDS index p + (p >> sh): keeps the strided stores of a pass apart
+  int words;  // doubles of one padded row
+  short r[MIX_PASSES][3];
 };
 
-// exp(sign 2 pi i e / n) from the table C[m] = cos(pi m / (2n)):
-// cos(2 pi e / n) = C(4e), sin(2 pi e / n) = C(|n - 4e|)
-__device__ inline void unit_root(const double *C, int n, long e, double sign, double &wr,
-                                 double &wi) {
-  const long d = (long)n - 4 * e;
-  wr = cos_lookup(C, n, 4 * e);
-  wi = sign * cos_lookup(C, n, d < 0 ? -d : d);
-}
+__device__ __forceinline__ int mix_pad(const MixPlan &pl, int p) { return p + (p >> pl.sh); }
 
-// Stockham autosort FFT of any length n in LDS (sign -1 forward, +1
-// backward, unnormalised), from (xr, xi) with (yr, yi) as the second
-// buffer; *outr, *outi: the pair that holds the result.  In the stage of
-// radix R after radices of product Ns, butterfly j (k = j mod Ns) takes
-// v_r = x[j + r n/R] w^(k r), w = e^(sign 2 pi i / (Ns R)), and stores
-// sum_r v_r e^(sign 2 pi i q r / R) at (j / Ns) Ns R + k + q Ns.  Factors
-// with exponent 0 are not multiplied; the oracle's fft_mixed performs the
-// same operations in the same order.
-__device__ void lds_fft_mixed(double *xr, double *xi, double *yr, double *yi, int n,
-                              const DctPlan &pl, const double *__restrict__ C, double sign,
-                              double **outr, double **outi) {
-  int Ns = 1;
-  for (int st = 0; st < pl.nr; st++) {
-    const int R = pl.r[st], nR = n / R, tw = n / (Ns * R);
-    for (int j = threadIdx.x; j < nR; j += blockDim.x) {
-      const int k = j % Ns;
-      const int o = (j / Ns) * Ns * R + k;
-      for (int q = 0; q < R; q++) {
-        double sr = 0., si = 0.;
-        for (int r = 0; r < R; r++) {
-          double vr = xr[j + r * nR], vi = xi[j + r * nR];
-          const long e = (long)k * r * tw;
-          if (e != 0) {
-            double wr, wi;
-            unit_root(C, n, e, sign, wr, wi);
-            const double tr = vr * wr - vi * wi, ti = vr * wi + vi * wr;
-            vr = tr;
-            vi = ti;
-          }
-          if (r == 0) {
-            sr = vr;
-            si = vi;
-            continue;
-          }
-          const long e2 = (long)((q * r) % R) * nR;
-          if (e2 == 0) {
-            sr = sr + vr;
-            si = si + vi;
-          } else {
-            double cr, ci;
-            unit_root(C, n, e2, sign, cr, ci);
-            sr = sr + (vr * cr - vi * ci);
-            si = si + (vr * ci + vi * cr);
-          }
+struct MixC {
+  double r, i;
+};
+template <int SIGN>
+__device__ __forceinline__ MixC mix_mul(const MixC &v, const double2 &w) {
+  const double wi = SIGN * w.y;
+  return MixC{v.r * w.x - v.i * wi, v.r * wi + v.i * w.x};
+}
+// the R-point sums in place; root[m] = e^(2 pi i m / R)
+template <int R, int SIGN>
+__device__ __forceinline__ void mix_dft(MixC (&v)[R], const double2 (&root)[R]) {
+  if constexpr (R > 1) {
+    MixC o[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      o[q] = v[0];
+#pragma unroll
+      for (int r = 1; r < R; r++) {
+        if ((q * r) % R == 0) {
+          o[q].r = o[q].r + v[r].r;
+          o[q].i = o[q].i + v[r].i;
+        } else {
+          const double2 w = root[(q * r) % R];
+          const double wi = SIGN * w.y;
+          o[q].r = o[q].r + (v[r].r * w.x - v[r].i * wi);
+          o[q].i = o[q].i + (v[r].r * wi + v[r].i * w.x);
         }
-        yr[o + q * Ns] = sr;
-        yi[o + q * Ns] = si;
       }
     }
+#pragma unroll
+    for (int q = 0; q < R; q++) v[q] = o[q];
+  }
+}
+
+// stages R1, R2, R3 (1: none) of a row, from (xr, xi) to (yr, yi)
+template <int R1, int R2, int R3, int SIGN>
+__device__ __forceinline__ void mix_pass(const MixPlan &pl, int Ns, const double *xr,
+                                         const double *xi, double *yr, double *yi,
+                                         const double2 *__restrict__ W) {
+  const int n = pl.n, N = n / (R1 * R2 * R3);
+  double2 root1[R1], root2[R2], root3[R3];
+#pragma unroll
+  for (int m = 1; m < R1; m++) root1[m] = W[m * (n / R1)];
+#pragma unroll
+  for (int m = 1; m < R2; m++) root2[m] = W[m * (n / R2)];
+#pragma unroll
+  for (int m = 1; m < R3; m++) root3[m] = W[m * (n / R3)];
+  const float inv_ns = 1.f / (float)Ns;
+  const int tw1 = n / (Ns * R1), tw2 = tw1 / R2, tw3 = tw2 / R3;
+  for (int g = threadIdx.x; g < N; g += blockDim.x) {
+    const int q0 = (int)(((float)g + 0.5f) * inv_ns), k = g - q0 * Ns;  // g < 2^13: exact
+    MixC v[R3][R2][R1];
+#pragma unroll
+    for (int c = 0; c < R3; c++)
+#pragma unroll
+      for (int b = 0; b < R2; b++)
+#pragma unroll
+        for (int a = 0; a < R1; a++) {
+          const int p = mix_pad(pl, g + N * (c + R3 * (b + R2 * a)));
+          v[c][b][a] = MixC{xr[p], xi[p]};
+        }
+    // stage 1
+#pragma unroll
+    for (int a = 1; a < R1; a++) {
+      const double2 w = W[k * a * tw1];
+#pragma unroll
+      for (int c = 0; c < R3; c++)
+#pragma unroll
+        for (int b = 0; b < R2; b++) v[c][b][a] = mix_mul<SIGN>(v[c][b][a], w);
+    }
+#pragma unroll
+    for (int c = 0; c < R3; c++)
+#pragma unroll
+      for (int b = 0; b < R2; b++) mix_dft<R1, SIGN>(v[c][b], root1);
+    // stage 2: its butterfly of output q of stage 1 has k2 = k + q Ns
+#pragma unroll
+    for (int a = 0; a < R1; a++) {
+#pragma unroll
+      for (int b = 1; b < R2; b++) {
+        const double2 w = W[(k + a * Ns) * b * tw2];
+#pragma unroll
+        for (int c = 0; c < R3; c++) v[c][b][a] = mix_mul<SIGN>(v[c][b][a], w);
+      }
+#pragma unroll
+      for (int c = 0; c < R3; c++) {
+        MixC u[R2];
+#pragma unroll
+        for (int b = 0; b < R2; b++) u[b] = v[c][b][a];
+        mix_dft<R2, SIGN>(u, root2);
+#pragma unroll
+        for (int b = 0; b < R2; b++) v[c][b][a] = u[b];
+      }
+    }
+    // stage 3
+#pragma unroll
+    for (int b = 0; b < R2; b++)
+#pragma unroll
+      for (int a = 0; a < R1; a++) {
+        MixC u[R3];
+        u[0] = v[0][b][a];
+#pragma unroll
+        for (int c = 1; c < R3; c++)
+          u[c] = mix_mul<SIGN>(v[c][b][a], W[(k + Ns * (a + R1 * b)) * c * tw3]);
+        mix_dft<R3, SIGN>(u, root3);
+#pragma unroll
+        for (int c = 0; c < R3; c++) {
+          const int p = mix_pad(pl, q0 * Ns * (R1 * R2 * R3) + k + Ns * (a + R1 * (b + R2 * c)));
+          yr[p] = u[c].r;
+          yi[p] = u[c].i;
+        }
+      }
+  }
+}
+
+// one stage of a radix too large for registers: the inputs twiddled in
+// place, then every output's sum
+template <int SIGN>
+__device__ __forceinline__ void mix_big(const MixPlan &pl, int Ns, int R, double *xr, double *xi,
+                                        double *yr, double *yi, const double2 *__restrict__ W) {
+  const int n = pl.n, nR = n / R;
+  if (Ns > 1) {
+    const int tw = nR / Ns;
+    for (int t = threadIdx.x; t < n - nR; t += blockDim.x) {
+      const int r = 1 + t / nR, j = t - (r - 1) * nR, p = mix_pad(pl, j + r * nR);
+      const MixC v = mix_mul<SIGN>(MixC{xr[p], xi[p]}, W[(j % Ns) * r * tw]);
+      xr[p] = v.r;
+      xi[p] = v.i;
+    }
+    __syncthreads();
+  }
+  const int Q = (R + MIX_BQ - 1) / MIX_BQ;  // outputs q, q + Q, ... of one thread
+  for (int t = threadIdx.x; t < Q * nR; t += blockDim.x) {
+    const int q = t / nR, j = t - q * nR;
+    MixC s[MIX_BQ];
+    int e[MIX_BQ], step[MIX_BQ];
+    const int p0 = mix_pad(pl, j);
+#pragma unroll
+    for (int b = 0; b < MIX_BQ; b++) {
+      s[b] = MixC{xr[p0], xi[p0]};
+      step[b] = q + b * Q < R ? q + b * Q : 0;
+      e[b] = 0;
+    }
+    for (int r = 1; r < R; r++) {
+      const int p = mix_pad(pl, j + r * nR);
+      const double vr = xr[p], vi = xi[p];
+#pragma unroll
+      for (int b = 0; b < MIX_BQ; b++) {
+        e[b] += step[b];
+        if (e[b] >= R) e[b] -= R;
+        // W[0] is exactly (1, 0): the sum's operations with exponent 0
+        const double2 w = W[e[b] * nR];
+        const double wi = SIGN * w.y;
+        s[b].r = s[b].r + (vr * w.x - vi * wi);
+        s[b].i = s[b].i + (vr * wi + vi * w.x);
+      }
+    }
+    const int k = j % Ns, o = (j / Ns) * Ns * R + k;
+#pragma unroll
+    for (int b = 0; b < MIX_BQ; b++)
+      if (q + b * Q < R) {
+        const int p = mix_pad(pl, o + (q + b * Q) * Ns);
+        yr[p] = s[b].r;
+        yi[p] = s[b].i;
+      }
+  }
+}
+
+// the whole transform; (xr, xi) filled and synchronised by the caller;
+// *outr, *outi: the pair that holds the result (synchronised)
+template <int SIGN>
+__device__ __forceinline__ void mix_fft(const MixPlan &pl, double *xr, double *xi, double *yr,
+                                        double *yi, const double2 *__restrict__ W, double **outr,
+                                        double **outi) {
+  int Ns = 1;
+  for (int p = 0; p < pl.np; p++) {
+    const int a = pl.r[p][0], b = pl.r[p][1], c = pl.r[p][2];
+#define EIF_MIX(A, B, C)                                        \
+  if (a == A && b == B && c == C)                               \
+    mix_pass<A, B, C, SIGN>(pl, Ns, xr, xi, yr, yi, W);         \
+  else
+    EIF_MIX(2, 2, 2) EIF_MIX(2, 2, 3) EIF_MIX(2, 2, 1) EIF_MIX(2, 3, 1) EIF_MIX(2, 5, 1)
+    EIF_MIX(2, 7, 1) EIF_MIX(3, 3, 1) EIF_MIX(3, 5, 1) EIF_MIX(2, 1, 1) EIF_MIX(3, 1, 1)
+    EIF_MIX(5, 1, 1) EIF_MIX(7, 1, 1)
+    mix_big<SIGN>(pl, Ns, a, xr, xi, yr, yi, W);
+#undef EIF_MIX
     __syncthreads();
     double *t = xr;
     xr = yr;
@@ -302,10 +456,88 @@ __device__ void lds_fft_mixed(double *xr, double *xi, double *yr, double *yi, in
     t = xi;
     xi = yi;
     yi = t;
-    Ns *= R;
+    Ns *= a * b * c;
   }
   *outr = xr;
   *outi = xi;
+}
+
+// the passes of a length n (host): consecutive prime factors in increasing
+// order, grouped while the group has a register form above
+static MixPlan mix_plan(int n) {
+  static const short forms[][3] = {{2, 2, 2}, {2, 2, 3}, {2, 2, 1}, {2, 3, 1}, {2, 5, 1},
+                                   {2, 7, 1}, {3, 3, 1}, {3, 5, 1}};
+  std::vector<int> f;
+  for (int p = 2, m = n; m > 1;) {
+    if (m % p == 0) {
+      f.push_back(p);
+      m /= p;
+    } else {
+      p++;
+    }
+  }
+  MixPlan pl{};
+  pl.n = n;
+  pl.sh = n <= 4096 ? 3 : 30;  // unpadded rows where the padding would not fit in LDS
+  pl.words = (n - 1) + ((n - 1) >> pl.sh) + 1;
+  int most = 1;
+  for (size_t i = 0; i < f.size() && pl.np < MIX_PASSES; pl.np++) {
+    short *r = pl.r[pl.np];
+    int use = 1;
+    r[0] = (short)f[i];
+    r[1] = r[2] = 1;
+    for (const auto &form : forms) {
+      const int len = form[2] > 1 ? 3 : 2;
+      bool ok = i + len <= f.size();
+      for (int k = 0; k < len && ok; k++) ok = f[i + k] == form[k];
+      if (ok) {
+        for (int k = 0; k < 3; k++) r[k] = form[k];
+        use = len;
+        break;
+      }
+    }
+    i += use;
+    const int group = r[0] * r[1] * r[2];
+    const int items = group > 15 || (use == 1 && group > 7) ? (n + MIX_BQ - 1) / MIX_BQ : n / group;
+    most = items > most ? items : most;
+  }
+  pl.threads = 64 * ((most + 63) / 64);
+  if (pl.threads > MIX_T_MAX) pl.threads = MIX_T_MAX;
+  return pl;
+}
+
+// RHS (compute_potential.c:70-82) and DCT-II of one row of any length
+struct RhsDct2MixB {
+  static constexpr int T = MIX_T_MAX, M = 0;
+  static __device__ __forceinline__ void run(const VB &vb, Layout L, const double *ux,
+                                             const double *uy, const double *dscal, double ga,
+                                             double dx, double dy, const double *__restrict__ C,
+                                             const double *__restrict__ W, MixPlan pl,
+                                             double *qhat, const double *add) {
+    extern __shared__ double sh[];
+    const int nx = pl.n, j = vb.bx + 1, w = pl.words;
+    double *re = sh, *im = sh + w;
+    const double fac = 1. / (ga * dscal[S_DT]);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < nx; i += blockDim.x) {  // Makhoul order
+      const int m = mix_pad(pl, (i & 1) ? nx - 1 - (i >> 1) : (i >> 1));
+      re[m] = rhs_value_add(L, ux, uy, add, fac, dx, dy, i, j);
+      im[m] = 0.;
+    }
+    __syncthreads();
+    double *Xr, *Xi;
+    mix_fft<-1>(pl, re, im, sh + 2 * w, sh + 3 * w, reinterpret_cast<const double2 *>(W), &Xr,
+                &Xi);
+    double *out = qhat + (long)(j - 1) * nx;
+    for (int k = threadIdx.x; k < nx; k += blockDim.x)
+      out[k] = 2. * (C[k] * Xr[mix_pad(pl, k)] + C[nx - k] * Xi[mix_pad(pl, k)]);
+  }
+};
+__global__ __launch_bounds__(MIX_T_MAX) void k_rhs_dct2_mix(
+    Layout L, const double *ux, const double *uy, const double *dscal, double ga, double dx,
+    double dy, const double *__restrict__ C, const double *__restrict__ W, MixPlan pl,
+    double *qhat, const double *add) {
+  RhsDct2MixB::run(VB::here(), L, ux, uy, dscal, ga, dx, dy, C, W, pl, qhat, add);
 }
 
 struct RhsDct2B {
@@ -313,7 +545,7 @@ struct RhsDct2B {
   static __device__ __forceinline__ void run(const VB &vb, 
     Layout L, const double *ux, const double *uy, const double *dscal, double ga,
     double dx, double dy, const double *__restrict__ C, const double *__restrict__ W,
-    DctPlan pl, int mode, double *qhat, const double *add) {
+    int logn, int mode, double *qhat, const double *add) {
   extern __shared__ double sh[];
   const int nx = L.nx;
   const int j = vb.bx + 1;
@@ -321,19 +553,7 @@ struct RhsDct2B {
   const double dt = dscal[S_DT];
   const double fac = 1. / (ga * dt);
   double *out = qhat + (long)(j - 1) * nx;
-  if (mode == 3) {  // Makhoul order, then the Stockham FFT (4 nx values of LDS)
-    for (int i = threadIdx.x; i < nx; i += blockDim.x) {
-      const int m = (i & 1) ? nx - 1 - (i >> 1) : (i >> 1);
-      re[m] = rhs_value_add(L, ux, uy, add, fac, dx, dy, i, j);
-      im[m] = 0.;
-    }
-    __syncthreads();
-    double *Xr, *Xi;
-    lds_fft_mixed(re, im, sh + 2 * nx, sh + 3 * nx, nx, pl, C, -1., &Xr, &Xi);
-    for (int k = threadIdx.x; k < nx; k += blockDim.x)
-      out[k] = 2. * (C[k] * Xr[k] + C[nx - k] * Xi[k]);
-  } else if (mode == 1) {
-    const int logn = pl.logn;
+  if (mode == 1) {
     for (int i = threadIdx.x; i < nx; i += blockDim.x) {
       const int m = (i & 1) ? nx - 1 - (i >> 1) : (i >> 1);
       const int pos = bitrev(m, logn);
@@ -360,8 +580,8 @@ struct RhsDct2B {
 __global__ __launch_bounds__(1024) void k_rhs_dct2(
     Layout L, const double *ux, const double *uy, const double *dscal, double ga,
     double dx, double dy, const double *__restrict__ C, const double *__restrict__ W,
-    DctPlan pl, int mode, double *qhat, const double *add) {
-  RhsDct2B::run(VB::here(), L, ux, uy, dscal, ga, dx, dy, C, W, pl, mode, qhat, add);
+    int logn, int mode, double *qhat, const double *add) {
+  RhsDct2B::run(VB::here(), L, ux, uy, dscal, ga, dx, dy, C, W, logn, mode, qhat, add);
 }
 
 // ---------------------------------------------------------------------
@@ -398,29 +618,14 @@ struct Dct3PsiB {
   static constexpr int T = 1024, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, 
     Layout L, const double *qhat, CombineArgs ca, const double *__restrict__ C,
-    const double *__restrict__ W, DctPlan pl, int mode, double *psi) {
+    const double *__restrict__ W, int logn, int mode, double *psi) {
   if (halted(ca.halt)) return;
   extern __shared__ double sh[];
   const int nx = L.nx, ny = L.ny;
   const int j0 = vb.bx;
   double *re = sh, *im = sh + nx;
   const double norm = 2. * nx;
-  if (mode == 3) {  // pre-twiddled spectrum, Stockham FFT, Makhoul order back
-    for (int k = threadIdx.x; k < nx; k += blockDim.x) {
-      const double xr = combined(ca, qhat, nx, ny, j0, k);
-      const double xi = k == 0 ? 0. : -combined(ca, qhat, nx, ny, j0, nx - k);
-      re[k] = C[k] * xr - C[nx - k] * xi;
-      im[k] = C[k] * xi + C[nx - k] * xr;
-    }
-    __syncthreads();
-    double *Xr, *Xi;
-    lds_fft_mixed(re, im, sh + 2 * nx, sh + 3 * nx, nx, pl, C, +1., &Xr, &Xi);
-    for (int i = threadIdx.x; i < nx; i += blockDim.x) {
-      const double v = (i & 1) ? Xr[nx - 1 - (i >> 1)] : Xr[i >> 1];
-      psi[L.p(i + 1, j0 + 1)] = v / norm;
-    }
-  } else if (mode == 1) {
-    const int logn = pl.logn;
+  if (mode == 1) {
     for (int k = threadIdx.x; k < nx; k += blockDim.x) {
       const double xr = combined(ca, qhat, nx, ny, j0, k);
       const double xi = k == 0 ? 0. : -combined(ca, qhat, nx, ny, j0, nx - k);
@@ -449,8 +654,57 @@ struct Dct3PsiB {
 };
 __global__ __launch_bounds__(1024) void k_dct3_psi(
     Layout L, const double *qhat, CombineArgs ca, const double *__restrict__ C,
-    const double *__restrict__ W, DctPlan pl, int mode, double *psi) {
-  Dct3PsiB::run(VB::here(), L, qhat, ca, C, W, pl, mode, psi);
+    const double *__restrict__ W, int logn, int mode, double *psi) {
+  Dct3PsiB::run(VB::here(), L, qhat, ca, C, W, logn, mode, psi);
+}
+
+// The DCT-III of one row of any length (mix_fft), with psi's boundary values
+// (the Neumann walls and the periodic halo rows 0 and ny + 1)
+struct Dct3PsiMixB {
+  static constexpr int T = MIX_T_MAX, M = 0;
+  static __device__ __forceinline__ void run(const VB &vb, Layout L, const double *qhat,
+                                             CombineArgs ca, const double *__restrict__ C,
+                                             const double *__restrict__ W, MixPlan pl,
+                                             double *psi) {
+    if (halted(ca.halt)) return;
+    extern __shared__ double sh[];
+    const int nx = pl.n, ny = L.ny, j0 = vb.bx, w = pl.words;
+    double *re = sh, *im = sh + w, *row = sh + 2 * w;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < nx; k += blockDim.x)
+      row[mix_pad(pl, k)] = combined(ca, qhat, nx, ny, j0, k);
+    __syncthreads();
+    for (int k = threadIdx.x; k < nx; k += blockDim.x) {  // pre-twiddled spectrum
+      const int p = mix_pad(pl, k);
+      const double xr = row[p];
+      const double xi = k == 0 ? 0. : -row[mix_pad(pl, nx - k)];
+      re[p] = C[k] * xr - C[nx - k] * xi;
+      im[p] = C[k] * xi + C[nx - k] * xr;
+    }
+    __syncthreads();
+    double *Xr, *Xi;
+    mix_fft<+1>(pl, re, im, sh + 2 * w, sh + 3 * w, reinterpret_cast<const double2 *>(W), &Xr,
+                &Xi);
+    const double norm = 2. * nx;
+    const int j = j0 + 1;
+    // ny >= 3: a row has at most one halo copy
+    const int jh = j == ny ? 0 : (j == 1 ? ny + 1 : -1);
+    for (int i = threadIdx.x; i < nx; i += blockDim.x) {  // Makhoul order back
+      const double v = Xr[mix_pad(pl, (i & 1) ? nx - 1 - (i >> 1) : i >> 1)] / norm;
+      psi[L.p(i + 1, j)] = v;
+      if (jh >= 0) psi[L.p(i + 1, jh)] = v;
+      if (i == 0 || i == nx - 1) {
+        const int iw = i == 0 ? 0 : nx + 1;
+        psi[L.p(iw, j)] = v;
+        if (jh >= 0) psi[L.p(iw, jh)] = v;
+      }
+    }
+  }
+};
+__global__ __launch_bounds__(MIX_T_MAX) void k_dct3_psi_mix(
+    Layout L, const double *qhat, CombineArgs ca, const double *__restrict__ C,
+    const double *__restrict__ W, MixPlan pl, double *psi) {
+  Dct3PsiMixB::run(VB::here(), L, qhat, ca, C, W, pl, psi);
 }
 
 // Register-FFT kernels specialised for nx = 2^LOGN (nx / 2^LOGR threads),
@@ -1423,10 +1677,18 @@ int poisson_init(Ctx *c) {
     EIF_HIP(hipMalloc(&c->ctab3, D.size() * sizeof(double)));
     EIF_HIP(hipMemcpy(c->ctab3, D.data(), D.size() * sizeof(double), hipMemcpyHostToDevice));
   }
-  // per-stage twiddles of the radix-2 transform (copies of C entries)
+  // per-stage twiddles of the radix-2 transform, or the roots of the
+  // transform of any length (copies of C entries)
   {
-    std::vector<double> W(2 * (size_t)(nx > 1 ? nx - 1 : 1), 0.);
-    if ((nx & (nx - 1)) == 0)
+    std::vector<double> W(2 * (size_t)nx, 0.);
+    if (nx & (nx - 1)) {  // the roots of the transform of any length
+      for (int e = 0; e < nx; e++) {
+        auto fold = [&](long m) { return C[m <= 2L * nx ? m : 4L * nx - m]; };
+        const long d = (long)nx - 4 * e;
+        W[2 * (size_t)e] = e ? fold(4L * e) : 1.;
+        W[2 * (size_t)e + 1] = e ? fold(d < 0 ? -d : d) : 0.;
+      }
+    } else
       for (int len = 2; len <= nx; len <<= 1)
         for (int k = 0; k < len / 2; k++) {
           const int m = k * (nx / len);
@@ -1510,21 +1772,6 @@ static int dct_mode(int nx) {
   return nx <= DCT_MIXED_MAX ? 3 : 0;
 }
 
-static DctPlan dct_plan(int n) {
-  DctPlan pl{};
-  pl.logn = ilog2_exact(n);
-  pl.nr = 0;
-  for (int p = 2; n > 1 && pl.nr < 24;) {
-    if (n % p == 0) {
-      pl.r[pl.nr++] = p;
-      n /= p;
-    } else {
-      p++;
-    }
-  }
-  return pl;
-}
-
 // values per thread (2^LOGR) of the register FFT of 2^LG-point rows: the
 // default 8, or the tuner's 4 or 16 where the workgroup keeps 32..1024
 // threads (every choice performs the same butterflies: same bits)
@@ -1588,11 +1835,10 @@ static int poisson_lines(Ctx *c, int rk, const double *rhs_add, CombineArgs *out
   const int nx = c->nx, ny = c->ny;
   const int logn = ilog2_exact(nx);
   // register FFT for 64 <= nx <= 8192, LDS FFT for other powers of two,
-  // the Stockham FFT for other lengths up to DCT_MIXED_MAX (its two buffer
-  // pairs in LDS), the direct sum beyond
+  // the Stockham FFT for other lengths up to DCT_MIXED_MAX, the direct sum
+  // beyond
   const int mode = dct_mode(nx);
-  const DctPlan pl = dct_plan(nx);
-  const size_t shmem = (mode == 3 ? 4 : 2) * (size_t)nx * sizeof(double);
+  const size_t shmem = 2 * (size_t)nx * sizeof(double);
   const int threads = DCT_THREADS;  // of the one-row kernels (modes 0, 1)
   {
     ProfScope ps(c, "rhs_dct2");
@@ -1609,8 +1855,16 @@ static int poisson_lines(Ctx *c, int rk, const double *rhs_add, CombineArgs *out
       EIF_RHS_T(6) EIF_RHS_T(7) EIF_RHS_T(8) EIF_RHS_T(9) EIF_RHS_T(10) EIF_RHS_T(11)
       EIF_RHS_T(12) EIF_RHS_T(13)
       default:
+        if (mode == 3) {
+          const MixPlan pl = mix_plan(nx);
+          go<RhsDct2MixB>(k_rhs_dct2_mix, dim3(ny), dim3(pl.threads),
+                          4 * (size_t)pl.words * sizeof(double), c->stream, c->L, c->ux, c->uy,
+                          c->dscal, c->gamma[rk], c->dx, c->dy, c->ctab, c->twid, pl, c->qhat,
+                          rhs_add);
+          break;
+        }
         go<RhsDct2B>(k_rhs_dct2, dim3(ny), dim3(threads), shmem, c->stream, c->L, c->ux, c->uy,
-                     c->dscal, c->gamma[rk], c->dx, c->dy, c->ctab, c->twid, pl, mode,
+                     c->dscal, c->gamma[rk], c->dx, c->dy, c->ctab, c->twid, logn, mode,
                      c->qhat, rhs_add);
     }
 #undef EIF_RHS_T
@@ -1666,12 +1920,11 @@ int launch_poisson(Ctx *c, int rk, const double *rhs_add) {
   const int nx = c->nx, ny = c->ny;
   const int logn = ilog2_exact(nx);
   const int mode = dct_mode(nx);
-  const DctPlan pl = dct_plan(nx);
-  const size_t shmem = (mode == 3 ? 4 : 2) * (size_t)nx * sizeof(double);
+  const size_t shmem = 2 * (size_t)nx * sizeof(double);
   const int threads = DCT_THREADS;
   CombineArgs ca;
   TRY_P(poisson_lines(c, rk, rhs_add, &ca));
-  bool halo_done = false;  // the register-FFT kernel writes psi's boundary values
+  bool halo_done = false;  // the kernels of modes 2 and 3 write psi's boundary values
   {
     ProfScope ps(c, "dct3_psi");
 #define EIF_DCT3_T(LG)                                                                  \
@@ -1683,8 +1936,16 @@ int launch_poisson(Ctx *c, int rk, const double *rhs_add) {
       EIF_DCT3_T(6) EIF_DCT3_T(7) EIF_DCT3_T(8) EIF_DCT3_T(9) EIF_DCT3_T(10) EIF_DCT3_T(11)
       EIF_DCT3_T(12) EIF_DCT3_T(13)
       default:
+        if (mode == 3) {
+          const MixPlan pl = mix_plan(nx);
+          halo_done = true;
+          go<Dct3PsiMixB>(k_dct3_psi_mix, dim3(ny), dim3(pl.threads),
+                          4 * (size_t)pl.words * sizeof(double), c->stream, c->L, c->qhat, ca,
+                          c->ctab, c->twid, pl, c->psi);
+          break;
+        }
         go<Dct3PsiB>(k_dct3_psi, dim3(ny), dim3(threads), shmem, c->stream, c->L,
-                           c->qhat, ca, c->ctab, c->twid, pl, mode, c->psi);
+                           c->qhat, ca, c->ctab, c->twid, logn, mode, c->psi);
     }
 #undef EIF_DCT3_T
     EIF_HIP(hipGetLastError());

@@ -39,3 +39,16 @@ def potential(nx, ny, ly, mode=eif.POISSON_THOMAS):
 def test_thomas_sweep_bit_exact_at_tile_edges(nx, ny, ly):
     a, b = potential(nx, ny, ly)
     assert np.array_equal(a, b)
+
+
+# row lengths of every pass of the transform of any length: each register
+# form alone and after others (12 = 2 2 3, 14 = 2 7, 20 = 2 2, 5, 30 = 2 3, 5,
+# 90 = 2 3, 3 5, 98 = 2 7, 7, 147 = 3, 7, 7, 375 = 3 5, 5, 5,
+# 768 = 2 2 2, 2 2 2, 2 2 3), radices summed over LDS first, last and
+# repeated (11, 121, 22, 143, 499 prime), more groups than threads, and a row
+# whose buffers exceed 64 KiB
+@pytest.mark.parametrize("nx", [3, 9, 11, 12, 14, 20, 22, 30, 90, 98, 121, 143, 147, 375, 499,
+                                768, 1701, 2500])
+def test_transform_of_any_length_bit_exact(nx):
+    a, b = potential(nx, 6, 0.5)
+    assert np.array_equal(a, b)
