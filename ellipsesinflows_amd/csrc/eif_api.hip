@@ -184,13 +184,13 @@ static void free_ctx(Ctx *c) {
                      &c->th_q1, &c->th_den, &c->th_last, &c->pt_fwd, &c->pt_u,
                      &c->pt_v, &c->pt_w, &c->pt_bnd, &c->pt_red, &c->pt_lvl, &c->pt_ends, &c->pt_g, &c->dscal, &c->dred,
                      &c->prt, &c->pconst, &c->dt_part, &c->sc_fx, &c->sc_fy, &c->sc_dist, &c->sc_pos,
-                     &c->sc_t, &c->res_slots, &c->st_ux1, &c->st_ux2, &c->st_uy1,
+                     &c->res_slots, &c->st_ux1, &c->st_ux2, &c->st_uy1,
                      &c->st_uy2, &c->st_phi, &c->slice_part, &c->slice_part0};
   for (auto b : bufs)
     if (*b) (void)hipFree(*b);
-  void *others[] = {c->boxes, c->box_off, c->tile_cnt, c->tile_list,
+  void *others[] = {c->sc_t, c->boxes, c->box_off, c->tile_cnt, c->tile_list,
                     c->flags, c->rows, c->row_cnt, c->wall_hit,
-                    c->ibm_stats, c->slice_first, c->slice_info, c->ibm_pp, c->slice_owner,
+                    c->ibm_stats, c->slice_first, c->slice_info, c->ibm_pp, c->slice_rec,
                     c->sc_key, c->heads, c->cl_start, c->cl_items, c->cl_cell, c->cl_slot, c->cl_count};
   for (auto o : others)
     if (o) (void)hipFree(o);
@@ -857,8 +857,7 @@ static int stage_start(Ctx *c, int rk, bool pred_queued, bool side_start) {
     // closes: the particle update, this stage's reset and the distances
     // at the new positions run on the side stream beside the predictor
     EIF_HIP(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-    TRY(launch_update_particles(c, c->side));
-    TRY(launch_reset(c, c->side, true));
+    TRY(launch_reset(c, c->side, true, true));
     TRY(launch_ibm_dist(c, c->side));
     EIF_HIP(hipEventRecord(c->ev_i0, c->side));
     TRY(launch_collision(c, 0, c->side));
@@ -872,8 +871,7 @@ static int stage_start(Ctx *c, int rk, bool pred_queued, bool side_start) {
     // behind the predictor (and the batches queued after it): the previous
     // stage's particle update, this stage's reset and the distances at the
     // new positions; collision(0) on the side stream
-    TRY(launch_update_particles(c));
-    TRY(launch_reset(c, c->stream, true));
+    TRY(launch_reset(c, c->stream, true, true));
     TRY(launch_ibm_dist(c));
     EIF_HIP(hipEventRecord(c->ev_fork, c->stream));
     EIF_HIP(hipStreamWaitEvent(c->side, c->ev_fork, 0));

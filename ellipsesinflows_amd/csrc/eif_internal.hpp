@@ -187,12 +187,12 @@ struct Ctx {
   int box_cap_x = 0, box_cap_y = 0;
   double *sc_fx = nullptr, *sc_fy = nullptr;  // per box cell forcing*dt
   double *sc_dist = nullptr;                  // cached tanh(BETA d), d the signed distance
-  double *sc_t = nullptr;                     // foot parameter per box cell
+  float *sc_t = nullptr;                      // foot parameter per box cell
   int *sc_key = nullptr;                      // np x 8: boxes of sc_t
   double *sc_pos = nullptr;                   // np x 3: positions of cache
   int *slice_first = nullptr;  // IBM work slices
   long *slice_info = nullptr;
-  int *slice_owner = nullptr;
+  int4 *slice_rec = nullptr;   // particle, its first slice and slices of each slice
   double *slice_part = nullptr;
   double *slice_part0 = nullptr;  // inertia(0) sums of the fused exchange
   void *heads = nullptr;          // np per-particle pass headers (SliceHead)
@@ -333,8 +333,10 @@ int launch_increment(Ctx *c, int rk, int sub = -1);
 // inertia(1) and collision(1) of sub-iteration `sub`, gated, in one launch
 int launch_substep_forces(Ctx *c, int sub);
 int launch_update_particles(Ctx *c, hipStream_t st = nullptr);
-// clear_tiles: also clear the IBM tile registrations for the next exchange
-int launch_reset(Ctx *c, hipStream_t st = nullptr, bool clear_tiles = false);
+// clear_tiles: also clear the IBM tile registrations for the next exchange;
+// update: the particle update first, in the same launch
+int launch_reset(Ctx *c, hipStream_t st = nullptr, bool clear_tiles = false,
+                 bool update = false);
 int launch_status(Ctx *c, int queued);
 int launch_stage_gate(Ctx *c, int stage, int K);
 int launch_graph_status(Ctx *c);

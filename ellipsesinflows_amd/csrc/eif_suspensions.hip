@@ -12,9 +12,9 @@
 //   increments / update   src/suspensions/increment.c:10-72, update.c:8-34
 //
 // Work decomposition (gfx950):
-//   * one workgroup per particle for the IBM integrals; its three periodic
-//     images' boxes are flattened and strided over the workgroup, and the
-//     per-particle sums are reduced in a fixed tree;
+//   * one wave per slice of 256 cells of a particle's boxes for the IBM
+//     integrals (its three periodic images' boxes flattened), the slices' sums
+//     added per particle in slice order;
 //   * the signed distance of every box cell is cached per particle with the
 //     position it belongs to; the reference evaluates it three times at
 //     identical positions in every RK stage (inertia(0), exchange and the
@@ -133,21 +133,30 @@ __device__ inline double signed_dist(const EllipseShape &e, double grid_size,
 }
 
 // ---------------------------------------------------------------------
-// Foot of the normal for the IBM weights.
+// Foot of the normal.
 //
 // src/ellipse.c:30-65 iterates t <- clamp(t + dt) from t = pi/4 until
 // |dt| < 1e-8, every iteration in FP64 with sin, cos, asin and three
 // square roots.  The iteration converges quadratically to the unique foot
-// on the first-quadrant arc, so here it starts in FP32 (hardware sin/cos,
-// stopped at |dt| < 1e-3, where the FP32 rounding noise takes over) and
-// finishes with the reference's FP64 iteration and stopping rule, which
-// then needs one or two iterations instead of about four.  After the first
-// FP64 step every update of t is below 2^-10, so cos and sin of the new t
-// follow from the old ones by the addition theorem with the Taylor series
-// of cos(delta) and sin(delta) (truncation below 1e-21), and only one FP64
-// sincos is evaluated per cell.  The converged (cos t, sin t) agree with
-// the reference's to a few units in the last place; the distance to the
-// foot is stationary in t, so it agrees to rounding.
+// on the first-quadrant arc, so here it starts in FP32 (stopped at
+// |dt| < 1e-3, where the FP32 rounding noise takes over) and finishes in
+// FP64.
+//
+// The collisions use the foot itself (foot_fp32, foot_fp64): the reference's
+// iteration in t and its stopping rule.
+//
+// The weights use only the distance, which is stationary in t
+// (foot_dist_fp32, foot_dist_fp64): cos t and sin t come from the hardware in
+// FP32, normalised to FP64 once and turned by dt from there; the factors that only set the length of a step come from the
+// hardware reciprocal square root (relative error 2^-23); and it ends at
+// |dt| < 2^-17.  The last step leaves an error e ~ dt^2 / 10 ~ 6e-12 in t,
+// which changes the distance by e^2 (at the evolute, where the convergence
+// slows to linear, the distance's second derivative vanishes too and it
+// changes by dt^3 / 6 < 1e-16).  The foot's parameter is kept per cell in
+// FP32, the start of the cell's next search in the same RK stage.
+// The FP64 and FP32 iterations per evaluated cell went from 1.51 and 0.05 to
+// 1.00 and 0.41 (2048x4096, 1024 ellipses), and an FP64 iteration from 124
+// instructions (and 51 of sincos) to 75.
 // ---------------------------------------------------------------------
 struct EllipseShape32 {
   float a, b, kex, key, a2b2;
@@ -197,6 +206,24 @@ __device__ inline void sincos_q1(double t, double &s, double &c) {
   const double ps = sin_poly(u), pc = cos_poly(u);
   s = low ? ps : pc;
   c = low ? pc : ps;
+}
+
+// sin and cos of a particle's orientation: |x| <= 64 (angles are kept in
+// [0, 2 pi]) reduced by multiples of pi/2 held in two doubles, the same
+// polynomials; other angles through the library
+__device__ inline void sincos_angle(double x, double &s, double &c) {
+  if (!(fabs(x) <= 64.)) {
+    sincos(x, &s, &c);
+    return;
+  }
+  constexpr double PIO2_HI = 1.5707963267948966, PIO2_LO = 6.123233995736766e-17;
+  const double q = rint(x * 0.63661977236758134);
+  const double u = fma(-q, PIO2_LO, fma(-q, PIO2_HI, x));
+  const int m = (int)q;
+  const double ps = sin_poly(u), pc = cos_poly(u);
+  const double a = m & 1 ? pc : ps, b = m & 1 ? ps : pc;
+  s = m & 2 ? -a : a;
+  c = (m + 1) & 2 ? -b : b;
 }
 
 // 1/sqrt(x) from the hardware estimate and one Newton step (relative error
@@ -291,18 +318,115 @@ __device__ inline void foot_fp64(const EllipseShape &e, double px, double py, do
   }
 }
 
-// compute_signed_dist (src/suspensions/auxiliary.c:19-47) with the foot
-// from foot_fp32 / foot_fp64; the unfolding of ellipse.c:62-63 maps
-// (cos t, sin t) of the folded foot to (-cos t, sin t) for x_ < 0 and
-// (cos t, -sin t) for y_ < 0.  The foot iteration starts from the parameter this cell's foot had at the
-// particle's previous evaluation in the same RK stage (warm), which the
-// particle has barely moved from, or else from the FP32 estimate; the root
-// on the first-quadrant arc is unique, so the start changes only the number
-// of iterations.  The new parameter is stored back.
-__device__ inline double signed_dist_warm(const EllipseShape &e, const EllipseShape32 &f,
+// where the FP64 iteration of the weights ends
+constexpr double FOOT_DIST_DT = 0x1p-17;
+
+// hardware cosine and sine of t in [0, pi/2] (absolute error below 1e-6)
+__device__ inline void cossin_hw(float t, float &c, float &s) {
+  const float rev = t * 0.15915494f;
+  c = __builtin_amdgcn_cosf(rev);
+  s = __builtin_amdgcn_sinf(rev);
+}
+
+// FP32 part for the distance: t from its start until |dt| < 1e-3 (at most 8
+// iterations)
+__device__ inline void foot_dist_fp32(const EllipseShape32 &f, float px, float py, float &t,
+                                      int &it32) {
+  for (int n = 0; n < 8; n++) {
+    float c, s;
+    cossin_hw(t, c, s);
+    const float x = f.a * c, y = f.b * s;
+    const float ex = f.kex * (c * c * c), ey = f.key * (s * s * s);
+    const float rx = x - ex, ry = y - ey;
+    const float qx = px - ex, qy = py - ey;
+    const float rr = fmaf(rx, rx, ry * ry), qq = fmaf(qx, qx, qy * qy);
+    float arg = fmaf(rx, qy, -(ry * qx)) * __builtin_amdgcn_rsqf(rr * qq);
+    arg = fminf(fmaxf(arg, -1.f), 1.f);
+    const float den = fmaxf(fmaf(-x, x, fmaf(-y, y, f.a2b2)), 1e-30f);
+    const float a2 = arg * arg;
+    const float as = fmaf(arg * a2, fmaf(a2, fmaf(a2, 0.044642857f, 0.075f), 0.16666667f), arg);
+    const float dt = rr * as * __builtin_amdgcn_rsqf(rr * den);
+    it32++;
+    if (!(fabsf(dt) < 1e30f)) break;  // no usable step: hand over to FP64
+    t = fminf(fmaxf(t + dt, 0.f), 1.5707963f);
+    if (fabsf(dt) < 1e-3f) break;
+  }
+}
+
+// FP64 part for the distance: (c, s) = (cos t, sin t) from the hardware's
+// (normalised here to FP64) until |dt| < FOOT_DIST_DT; t follows in FP32
+__device__ inline void foot_dist_fp64(const EllipseShape &e, double px, double py, float &t,
+                                      double &c, double &s, int &it64) {
+  {
+    float cf, sf;
+    cossin_hw(t, cf, sf);
+    c = (double)cf;
+    s = (double)sf;
+    const double d = fma(c, c, fma(s, s, -1.));  // |d| < 4e-6: (1 + d)^(-1/2) to d^3
+    const double w = fma(d, fma(d, 0.375, -0.5), 1.);
+    c *= w;
+    s *= w;
+  }
+  for (int n = 0;; n++) {
+    const double x = e.a * c, y = e.b * s;
+    const double ex = e.kex * (c * c * c), ey = e.key * (s * s * s);
+    const double rx = x - ex, ry = y - ey;
+    const double qx = px - ex, qy = py - ey;
+    const double rr = fma(ry, ry, rx * rx), qq = fma(qy, qy, qx * qx);
+    const double cross = rx * qy - ry * qx;
+    const double arg = cross * __builtin_amdgcn_rsq(rr * qq);
+    const double a2 = arg * arg;
+    const double as = fma(arg * a2, fma(a2, 0.075, 1. / 6.), arg);
+    const double den = fma(-x, x, fma(-y, y, e.a2b2));
+    const double dt = as * (rr * __builtin_amdgcn_rsq(rr * den));
+    it64++;
+    if (!(fabs(dt) < 1e30)) {  // on the evolute: the reference's clamp goes to pi/2
+      const bool there = c == 0.;
+      c = 0.;
+      s = 1.;
+      t = 1.5707963f;
+      if (there || n > 100) break;
+      continue;
+    }
+    const double d2 = dt * dt;
+    const double hc = d2 * fma(d2, -1. / 24., 0.5);  // 1 - cos(dt), |dt| small
+    const double sd = dt * fma(d2, fma(d2, 1. / 120., -1. / 6.), 1.);
+    const double cn = c - fma(s, sd, c * hc), sn = s + fma(c, sd, -(s * hc));
+    c = cn;
+    s = sn;
+    t += (float)dt;
+    if (fabs(dt) > 0x1p-10) {  // a large step: the series is short, normalise
+      const double w = rsqrt_nr(fma(c, c, s * s));
+      c *= w;
+      s *= w;
+    }
+    if (c < 0.) {
+      c = 0.;
+      s = 1.;
+      t = 1.5707963f;
+    }
+    if (s < 0.) {
+      c = 1.;
+      s = 0.;
+      t = 0.f;
+    }
+    if (fabs(dt) < FOOT_DIST_DT || n > 100) break;
+  }
+}
+
+// compute_signed_dist (src/suspensions/auxiliary.c:19-47); the unfolding of
+// ellipse.c:62-63 maps (cos t, sin t) of the folded foot to (-cos t, sin t)
+// for x_ < 0 and (cos t, -sin t) for y_ < 0.  t: where the foot's search
+// starts, and its parameter on return: pi/4, or the parameter this cell's
+// foot had at the particle's previous evaluation in the same RK stage, which
+// the particle has barely moved from.  search: through FP32 iterations first
+// (from pi/4, or when the particle moved by more than one FP64 step
+// resolves).  The root on the first-quadrant arc is unique, so the start
+// changes only the number of iterations.
+__device__ inline double signed_dist_from(const EllipseShape &e, const EllipseShape32 &f,
                                           double inv_grid, double px, double py, double cr,
-                                          double sr, double x, double y, bool warm,
-                                          double &tslot, int &it32, int &it64) {
+                                          double sr, double x, double y, bool search, float &t,
+                                          int &it32, int &it64) {
   const double ddx = x - px, ddy = y - py;
   const double x_ = cr * ddx - sr * ddy;
   const double y_ = sr * ddx + cr * ddy;
@@ -310,13 +434,10 @@ __device__ inline double signed_dist_warm(const EllipseShape &e, const EllipseSh
   const double f0 = 1. - xa * xa - yb * yb;
   const double sign = f0 > 0. ? +1. : -1.;
   const double ax = fabs(x_), ay = fabs(y_);
-  double t = warm ? tslot : (double)foot_fp32(f, ax, ay, it32);
+  if (search) foot_dist_fp32(f, (float)ax, (float)ay, t, it32);
   double ct, st;
-  foot_fp64(e, ax, ay, t, ct, st, it64);
-  tslot = t;
-  const double fx = x_ < 0. ? -(e.a * ct) : e.a * ct;
-  const double fy = y_ < 0. ? -(e.b * st) : e.b * st;
-  const double ex = fx - x_, ey = fy - y_;
+  foot_dist_fp64(e, ax, ay, t, ct, st, it64);
+  const double ex = copysign(e.a * ct, x_) - x_, ey = copysign(e.b * st, y_) - y_;
   const double dist = sign * sqrt(+ex * ex + ey * ey);
   return dist * inv_grid;
 }
@@ -362,6 +483,25 @@ __device__ inline bool sub_open(const double *res, int sub) {
   return !res || sub == 0 || (!(res[sub - 1] < 1.e-8) && sub <= 101);
 }
 
+// The IBM, deposit and collision kernels give each wave its own slice, tile or
+// particle.  The waves of a workgroup (WG_WAVES) share nothing, so LDS is per
+// wave and ordered within the wave.  One wave a workgroup: four made the
+// collision launch 28 -> 41 us and left the others as they were (2048x4096,
+// 1024 ellipses; the dispatch of 11600 one-wave workgroups takes 3.6 us).
+constexpr int WG_WAVES = 1;
+__device__ inline int wave_lane() { return threadIdx.x & 63; }
+// the wave's place in the launch, known uniform
+__device__ inline int wave_index(const VB &vb) {
+  return __builtin_amdgcn_readfirstlane(vb.bx * WG_WAVES + (threadIdx.x >> 6));
+}
+__device__ inline int wave_in_group() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+// LDS written by the wave's lanes is visible to its other lanes
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 struct SliceHead;
 
 struct IbmArgs {
@@ -379,7 +519,7 @@ struct IbmArgs {
   double *sc_fx, *sc_fy;
   double *sc_dist;  // per box cell: tanh(BETA d) of the signed distance d
   double *sc_pos;
-  double *sc_t;   // per box cell: foot parameter of the last evaluation
+  float *sc_t;    // per box cell: foot parameter of the last evaluation
   int *sc_key;    // per particle: boxes of that evaluation (8 ints)
   int *tile_cnt, *tile_list;
   int ntx, nty;
@@ -387,8 +527,9 @@ struct IbmArgs {
   unsigned long long *stats;  // per particle: cells, cells evaluated, FP64 and FP32 iterations
   double *cpos;               // np x 4: the broad phase's packed positions and radii
   int np;
+  int nslices;
   const int *slice_first;  // np+1: first slice of each particle
-  const int *slice_owner;  // particle of each slice
+  const int4 *slice_rec;   // of each slice: its particle, the particle's first slice and slices
   long *slice_info;        // np x 2: box cells, cells evaluated (this call)
   const double *res;       // sub-iteration residuals (null: not gated)
   int sub;                 // sub-iteration index
@@ -435,7 +576,7 @@ __device__ inline double lane_value(double x, int l) {
 // A slice's partial sums (lane 0); k_ibm_finalize adds them per particle in
 // slice order after the kernel has finished, so no fence or atomic is needed.
 __device__ inline void slice_store(const IbmArgs &a, int slice, const double v[SLICE_VALS]) {
-  if (threadIdx.x == 0)
+  if (wave_lane() == 0)
     for (int k = 0; k < SLICE_VALS; k++) a.slice_part[SLICE_VALS * (long)slice + k] = v[k];
 }
 
@@ -469,24 +610,6 @@ __device__ inline void make_boxes(const IbmArgs &a, double px, double py,
   bs.total = bs.b0.cnt + bs.b1.cnt + bs.b2.cnt;
 }
 
-// boxes of the last distance evaluation (cells map to the same flattened
-// index only when every image's box is unchanged)
-__device__ inline bool same_boxes(const int *key, const BoxSet &bs) {
-  return key[7] != 0 && key[0] == bs.b0.imin && key[1] == bs.b0.jmin &&
-         key[2] == bs.b1.imin && key[3] == bs.b1.jmin && key[4] == bs.b2.imin &&
-         key[5] == bs.b2.jmin && key[6] == bs.total;
-}
-__device__ inline void store_boxes(int *key, const BoxSet &bs) {
-  key[0] = bs.b0.imin;
-  key[1] = bs.b0.jmin;
-  key[2] = bs.b1.imin;
-  key[3] = bs.b1.jmin;
-  key[4] = bs.b2.imin;
-  key[5] = bs.b2.jmin;
-  key[6] = bs.total;
-  key[7] = 1;
-}
-
 __device__ inline Img pick(const BoxSet &bs, int k) {
   Img m = bs.b0;
   if (k == 1) m = bs.b1;
@@ -494,18 +617,26 @@ __device__ inline Img pick(const BoxSet &bs, int k) {
   return m;
 }
 
-// image k and cell (i, j) of flattened box cell t.  The image's fields are
-// blended arithmetically (a select between struct members can be turned
-// into a load from a stack copy), and the quotient by the box width comes
-// from a float reciprocal, corrected once (exact for t < 2^24).
-__device__ inline void cell_of(const BoxSet &bs, int t, int &k, int &i, int &j) {
-  const int c0 = bs.b0.cnt, c01 = c0 + bs.b1.cnt;
-  const int g1 = t >= c0, g2 = t >= c01;
-  k = g1 + g2;
-  const int tk = t - g1 * c0 - g2 * bs.b1.cnt;
-  const int imin = bs.b0.imin + g1 * (bs.b1.imin - bs.b0.imin) + g2 * (bs.b2.imin - bs.b1.imin);
-  const int imax = bs.b0.imax + g1 * (bs.b1.imax - bs.b0.imax) + g2 * (bs.b2.imax - bs.b1.imax);
-  const int jmin = bs.b0.jmin + g1 * (bs.b1.jmin - bs.b0.jmin) + g2 * (bs.b2.jmin - bs.b1.jmin);
+// image k and cell (i, j) of flattened box cell t.  single: the particle has
+// cells in the middle image only, which is the same for the whole wave;
+// otherwise the image's fields are blended arithmetically (a select between
+// struct members can be turned into a load from a stack copy).  The quotient
+// by the box width comes from a float reciprocal, corrected once (exact for
+// t < 2^24).
+__device__ inline bool single_image(const BoxSet &bs) { return bs.b1.cnt == bs.total; }
+__device__ inline void cell_of(const BoxSet &bs, int t, int &k, int &i, int &j,
+                               bool single = false) {
+  int tk = t, imin = bs.b1.imin, imax = bs.b1.imax, jmin = bs.b1.jmin;
+  k = 1;
+  if (!single) {
+    const int c0 = bs.b0.cnt, c01 = c0 + bs.b1.cnt;
+    const int g1 = t >= c0, g2 = t >= c01;
+    k = g1 + g2;
+    tk = t - g1 * c0 - g2 * bs.b1.cnt;
+    imin = bs.b0.imin + g1 * (bs.b1.imin - bs.b0.imin) + g2 * (bs.b2.imin - bs.b1.imin);
+    imax = bs.b0.imax + g1 * (bs.b1.imax - bs.b0.imax) + g2 * (bs.b2.imax - bs.b1.imax);
+    jmin = bs.b0.jmin + g1 * (bs.b1.jmin - bs.b0.jmin) + g2 * (bs.b2.jmin - bs.b1.jmin);
+  }
   const int w = imax - imin + 1;
   int q = (int)((float)tk * __builtin_amdgcn_rcpf((float)w));
   int r = tk - q * w;
@@ -518,6 +649,30 @@ __device__ inline void cell_of(const BoxSet &bs, int t, int &k, int &i, int &j) 
   }
   j = jmin + q;
   i = imin + r;
+}
+// the U cells of a lane of a slice, t0 + lane + 64 u (the last cell, t1 - 1,
+// in the place of those past it)
+template <int U>
+__device__ inline void lane_cells(const BoxSet &bs, int t0, int t1, int lane, int (&k)[U],
+                                  int (&i)[U], int (&j)[U]) {
+  if (single_image(bs)) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      cell_of(bs, min(t0 + lane + 64 * u, t1 - 1), k[u], i[u], j[u], true);
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      cell_of(bs, min(t0 + lane + 64 * u, t1 - 1), k[u], i[u], j[u]);
+  }
+}
+
+// the x and y faces west of and south of cell (i, j) in the velocity arrays
+// (fewer than 2^31 values: the context bounds the grid)
+__device__ inline unsigned face_x(const Layout &L, int i, int j) {
+  return (unsigned)j * (unsigned)(L.nx + 1) + (unsigned)(i - 1);
+}
+__device__ inline unsigned face_y(const Layout &L, int i, int j) {
+  return (unsigned)j * (unsigned)(L.nx + 2) + (unsigned)i;
 }
 
 // What every slice wave of one IBM pass needs of its particle: computed
@@ -535,69 +690,90 @@ struct SliceHead {
   EllipseShape32 f;
   int cached;          // the distance cache holds this position
   int warm;            // the foot parameters hold these boxes
+  int far;             // ... of a position too far for one FP64 step
 };
 
-// same_boxes against the key store_boxes(k) would leave
-__device__ inline bool same_boxset(const BoxSet &k, const BoxSet &bs) {
-  return k.b0.imin == bs.b0.imin && k.b0.jmin == bs.b0.jmin && k.b1.imin == bs.b1.imin &&
-         k.b1.jmin == bs.b1.jmin && k.b2.imin == bs.b2.imin && k.b2.jmin == bs.b2.jmin &&
-         k.total == bs.total;
+// lane l's integer, l the same on every lane of the wave
+__device__ inline int lane_int(int x, int l) { return __builtin_amdgcn_readlane(x, l); }
+
+// The pass whose distances and foot parameters a particle's cache holds, as
+// the lanes of its wave see it: the position on every lane, the box corner
+// of image min(lane, 2)
+struct CachedPass {
+  double px, py, paz;
+  int imin, jmin, total;
+  bool pos, boxes;  // recorded
+};
+// ... from the records (sc_pos, sc_key)
+__device__ inline CachedPass cached_records(const IbmArgs &a, int n, int lane) {
+  const double *cp = a.sc_pos + 4 * (long)n;
+  const int *key = a.sc_key + 8 * (long)n;
+  const int k = min(lane, 2);
+  return {cp[0], cp[1], cp[2], key[2 * k], key[2 * k + 1], key[6], cp[3] != 0., key[7] != 0};
 }
 
-// full: also the parts that depend only on the particle's shape and mass
-// (written at every stage start, so records changed between calls are
-// picked up); otherwise only the position-dependent parts
-// prev: the header whose pass the cache records now describe (known to the
-// caller), else the records are read
-// rad: max(a, b) of the particle, when the caller has it (< 0: read here)
-__device__ inline void write_head(const IbmArgs &a, int n, double px, double py, double paz,
-                                  bool full, const SliceHead *prev = nullptr,
-                                  double rad = -1.) {
-  const double *q = a.prt + (long)n * R_N;
-  SliceHead *h = a.heads + n;
-  if (full) {
-    h->e = make_shape(q[R_A], q[R_B]);
-    h->f = shape32(h->e);
-    h->inv_pm = 1. / p_mass(q);
-    h->inv_pim = 1. / p_moi(q);
-    h->off = a.box_off[n];
-    h->cap = a.box_off[n + 1] - h->off;
-  }
-  h->px = px;
-  h->py = py;
-  h->paz = paz;
+// The position-dependent parts of a particle's header, by the lanes of one
+// wave: lanes 0, 1, 2 make the boxes of the three images.  lo, hi: the
+// particle's semi-axes in order; known: the cache holds prev's pass itself
+// (else how far its position lies is not looked at)
+__device__ inline void write_head(const IbmArgs &a, SliceHead *h, int lane, double px, double py,
+                                  double paz, double lo, double hi, const CachedPass &prev,
+                                  bool known) {
+  const Img m = make_img(a, px, py + a.ly * (min(lane, 2) - 1), hi);
+  const int total = lane_int(m.cnt, 0) + lane_int(m.cnt, 1) + lane_int(m.cnt, 2);
+  const bool same = __ballot(m.imin != prev.imin || m.jmin != prev.jmin) == 0ull &&
+                    total == prev.total;
   double sr, cr;
-  sincos(-paz, &sr, &cr);
-  h->cr = cr;
-  h->sr = sr;
-  BoxSet bs;
-  make_boxes(a, px, py, rad >= 0. ? rad : fmax(q[R_A], q[R_B]), bs);
-  h->bs = bs;
-  if (prev) {  // the cache records were just made from prev
-    h->cached = prev->px == px && prev->py == py && prev->paz == paz;
-    h->warm = same_boxset(prev->bs, bs);
-  } else {
-    const double *cp = a.sc_pos + 4 * (long)n;
-    h->cached = cp[3] != 0. && cp[0] == px && cp[1] == py && cp[2] == paz;
-    h->warm = same_boxes(a.sc_key + 8 * (long)n, bs);
+  sincos_angle(-paz, sr, cr);
+  if (lane < 3) (&h->bs.b0)[lane] = m;
+  if (lane == 0) {
+    h->px = px;
+    h->py = py;
+    h->paz = paz;
+    h->cr = cr;
+    h->sr = sr;
+    h->bs.total = total;
+    h->cached = prev.pos && prev.px == px && prev.py == py && prev.paz == paz;
+    h->warm = prev.boxes && same;
+    // a foot moves by at most the displacement over the smallest radius of
+    // curvature, but for cells near the evolute
+    h->far = !known || (fabs(px - prev.px) + fabs(py - prev.py) + hi * fabs(paz - prev.paz)) * hi >
+                           0.5 * FOOT_DIST_DT * lo * lo;
   }
 }
 
-// heads at the particles' positions, with the increments when with_dx
-struct HeadsB {
-  static constexpr int T = 1024, M = 0;
-  static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, int with_dx) {
-  if (halted(a.halt)) return;
-  const int n = vb.bx * blockDim.x + threadIdx.x;
-  if (n >= a.np) return;
-  const double *q = a.prt + (long)n * R_N;
-  if (with_dx)
-    write_head(a, n, q[R_X] + q[R_DX], q[R_Y] + q[R_DY], q[R_AZ] + q[R_DAZ], true);
-  else
-    write_head(a, n, q[R_X], q[R_Y], q[R_AZ], true);
+// the parts that depend only on the particle's shape and mass (written at
+// every stage start, so records changed between calls are picked up)
+__device__ inline void write_head_shape(const IbmArgs &a, SliceHead *h, int n, int lane,
+                                        const double *q) {
+  if (lane != 0) return;
+  const EllipseShape e = make_shape(q[R_A], q[R_B]);
+  h->e = e;
+  h->f = shape32(e);
+  h->inv_pm = 1. / p_mass(q);
+  h->inv_pim = 1. / p_moi(q);
+  h->off = a.box_off[n];
+  h->cap = a.box_off[n + 1] - h->off;
 }
+
+// heads at the particles' positions, with the increments when with_dx; one
+// wave per particle, four per workgroup
+struct HeadsB {
+  static constexpr int T = 256, M = 0;
+  static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, int with_dx) {
+    if (halted(a.halt)) return;
+    const int n = vb.bx * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (n >= a.np) return;
+    const double *q = a.prt + (long)n * R_N;
+    const double w = with_dx ? 1. : 0.;  // x + 0 is x
+    SliceHead *h = a.heads + n;
+    const CachedPass prev = cached_records(a, n, lane);
+    write_head_shape(a, h, n, lane, q);
+    write_head(a, h, lane, q[R_X] + w * q[R_DX], q[R_Y] + w * q[R_DY], q[R_AZ] + w * q[R_DAZ],
+               fmin(q[R_A], q[R_B]), fmax(q[R_A], q[R_B]), prev, false);
+  }
 };
-__global__ void k_heads(IbmArgs a, int with_dx) {
+__global__ __launch_bounds__(256) void k_heads(IbmArgs a, int with_dx) {
   HeadsB::run(VB::here(), a, with_dx);
 }
 
@@ -608,100 +784,97 @@ __global__ void k_heads(IbmArgs a, int with_dx) {
 // slice's own loads are issued, so the gate's load is not waited for alone
 __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int slice,
                                               bool open = true) {
-  const int n = a.slice_owner[slice];
-  const int s0 = a.slice_first[n], nsl = a.slice_first[n + 1] - s0;
+  const int lane = wave_lane();
+  const int4 rec = a.slice_rec[slice];
+  const int n = rec.x, s0 = rec.y, nsl = rec.z;
   const SliceHead &hd = a.heads[n];
   const BoxSet bs = hd.bs;
   const int total = bs.total;
   if (!open) return;
   if (total > hd.cap || total > nsl * IBM_SLICE) {
-    if (threadIdx.x == 0) atomicOr(&a.flags[0], 1);
+    if (lane == 0) atomicOr(&a.flags[0], 1);
     return;
   }
   const EllipseShape e = hd.e;
   const EllipseShape32 f = hd.f;
   const double px = hd.px, py = hd.py;
   const double inv_pm = hd.inv_pm, inv_pim = hd.inv_pim;
-  const bool cached = hd.cached, warm = hd.warm;
+  const bool cached = hd.cached, warm = hd.warm, search = !warm || hd.far;
   double *dist = a.sc_dist + hd.off;
-  double *tcell = a.sc_t + hd.off;
+  float *tcell = a.sc_t + hd.off;
   const double cr = hd.cr, sr = hd.sr;
   const double dxdy = a.dx * a.dy;
   double acc[3] = {0., 0., 0.};  // iux, iuy, ivz
   int it64 = 0, it32 = 0;
   const int t0 = (slice - s0) * IBM_SLICE;
   const int t1 = t0 + IBM_SLICE < total ? t0 + IBM_SLICE : total;
-  if (cached) {
-    // all loads of the lane's cells first (a cell past t1 loads the last
-    // cell instead and is not added), then the sums in cell order
-    if (t0 < t1) {
-      constexpr int U = IBM_SLICE / 64;
-      double th_[U], x_[U], y_[U], vx0[U], vx1[U], vy0[U], vy1[U];
-      int k_[U];
+  // all loads of the lane's cells first (a cell past t1 loads the last cell
+  // instead and is not added), then the weights and the sums in cell order
+  if (t0 < t1) {
+    constexpr int U = IBM_SLICE / 64;
+    double th_[U], x_[U], y_[U], vx0[U], vx1[U], vy0[U], vy1[U];
+    float tp[U];
+    int k_[U], i_[U], j_[U];
+    lane_cells<U>(bs, t0, t1, lane, k_, i_, j_);
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int t = min(t0 + (int)threadIdx.x + 64 * u, t1 - 1);
-        int k, i, j;
-        cell_of(bs, t, k, i, j);
-        k_[u] = k;
-        x_[u] = a.xc[i];
-        y_[u] = a.yc[j - 1];
-        th_[u] = dist[t];
-        vx0[u] = a.ux[a.L.ux(i, j)];
-        vx1[u] = a.ux[a.L.ux(i + 1, j)];
-        vy0[u] = a.uy[a.L.p(i, j)];
-        vy1[u] = a.uy[a.L.p(i, j + 1)];
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (t0 + (int)threadIdx.x + 64 * u >= t1) continue;
-        const double py_ = py + a.ly * (k_[u] - 1);
-        const double w = v_weight_th(th_[u]);
-        const double valx = w * 0.5 * (vx0[u] + vx1[u]) * dxdy;
-        const double valy = w * 0.5 * (vy0[u] + vy1[u]) * dxdy;
-        acc[0] += valx * inv_pm;
-        acc[2] += -(y_[u] - py_) * valx * inv_pim;
-        acc[1] += valy * inv_pm;
-        acc[2] += +(x_[u] - px) * valy * inv_pim;
-      }
+    for (int u = 0; u < U; u++) {
+      const unsigned fx = face_x(a.L, i_[u], j_[u]), fy = face_y(a.L, i_[u], j_[u]);
+      x_[u] = a.xc[i_[u]];
+      y_[u] = a.yc[j_[u] - 1];
+      vx0[u] = a.ux[fx];
+      vx1[u] = a.ux[fx + 1];
+      vy0[u] = a.uy[fy];
+      vy1[u] = a.uy[fy + (unsigned)(a.nx + 2)];
     }
-  } else
-  for (int t = t0 + (int)threadIdx.x; t < t1; t += 64) {
-    int k, i, j;
-    cell_of(bs, t, k, i, j);
-    const double py_ = py + a.ly * (k - 1);
-    const double x = a.xc[i], y = a.yc[j - 1];
-    // the velocities do not depend on the distance: loaded first
-    const double vx0 = a.ux[a.L.ux(i, j)], vx1 = a.ux[a.L.ux(i + 1, j)];
-    const double vy0 = a.uy[a.L.p(i, j)], vy1 = a.uy[a.L.p(i, j + 1)];
-    const double th = weight_th(signed_dist_warm(e, f, 1. / a.grid_size, px, py_, cr, sr, x,
-                                                 y, warm, tcell[t], it32, it64));
-    dist[t] = th;
-    const double w = v_weight_th(th);
-    const double valx = w * 0.5 * (vx0 + vx1) * dxdy;
-    const double valy = w * 0.5 * (vy0 + vy1) * dxdy;
-    acc[0] += valx * inv_pm;
-    acc[2] += -(y - py_) * valx * inv_pim;
-    acc[1] += valy * inv_pm;
-    acc[2] += +(x - px) * valy * inv_pim;
+    if (cached) {
+#pragma unroll
+      for (int u = 0; u < U; u++) th_[u] = dist[min(t0 + lane + 64 * u, t1 - 1)];
+    } else if (warm) {
+#pragma unroll
+      for (int u = 0; u < U; u++) tp[u] = tcell[min(t0 + lane + 64 * u, t1 - 1)];
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; u++) tp[u] = (float)(0.25 * EIF_PI);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int t = t0 + lane + 64 * u;
+      if (t >= t1) continue;
+      const double py_ = py + a.ly * (k_[u] - 1);
+      const double x = x_[u], y = y_[u];
+      if (!cached) {
+        th_[u] = weight_th(signed_dist_from(e, f, 1. / a.grid_size, px, py_, cr, sr, x, y, search,
+                                            tp[u], it32, it64));
+        tcell[t] = tp[u];
+        dist[t] = th_[u];
+      }
+      const double w = v_weight_th(th_[u]);
+      const double valx = w * 0.5 * (vx0[u] + vx1[u]) * dxdy;
+      const double valy = w * 0.5 * (vy0[u] + vy1[u]) * dxdy;
+      acc[0] += valx * inv_pm;
+      acc[2] += -(y - py_) * valx * inv_pim;
+      acc[1] += valy * inv_pm;
+      acc[2] += +(x - px) * valy * inv_pim;
+    }
   }
   double part[SLICE_VALS] = {wave_sum(acc[0]), wave_sum(acc[1]), wave_sum(acc[2]),
                              wave_sum((double)it64), wave_sum((double)it32)};
   slice_store(a, slice, part);
-  if (slice == s0 && threadIdx.x == 0) {
+  if (slice == s0 && lane == 0) {
     a.slice_info[2 * (long)n] = total;
     a.slice_info[2 * (long)n + 1] = cached ? 0 : total;
   }
 }
 
 struct InertiaB {
-  static constexpr int T = 64, M = 0;
+  static constexpr int T = 64 * WG_WAVES, M = 4;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, int cnstep) {
   if (halted(a.halt)) return;
-  inertia_slice(a, cnstep, vb.bx, sub_open(a.res, a.sub));
+  const int slice = wave_index(vb);
+  if (slice < a.nslices) inertia_slice(a, cnstep, slice, sub_open(a.res, a.sub));
 }
 };
-__global__ __launch_bounds__(64) void k_inertia(IbmArgs a, int cnstep) {
+__global__ __launch_bounds__(64 * WG_WAVES, 4) void k_inertia(IbmArgs a, int cnstep) {
   InertiaB::run(VB::here(), a, cnstep);
 }
 
@@ -727,27 +900,46 @@ __device__ inline void slice_sums(const IbmArgs &a, int s0, int s1, double tot[S
   }
 }
 
-// the cache records of the pass with header hd, and the work counters
-__device__ inline void record_pass(const IbmArgs &a, int n, const SliceHead &hd,
-                                   const double tot[SLICE_VALS]) {
-  double *cw = a.sc_pos + 4 * (long)n;
-  cw[0] = hd.px;
-  cw[1] = hd.py;
-  cw[2] = hd.paz;
-  cw[3] = 1.;
-  store_boxes(a.sc_key + 8 * (long)n, hd.bs);
-  if (n == 0) a.stats[4 * (long)a.np] += 1ull;  // IBM calls
-  unsigned long long *c = a.stats + 4 * (long)n;
-  c[0] += (unsigned long long)a.slice_info[2 * (long)n];
-  c[1] += (unsigned long long)a.slice_info[2 * (long)n + 1];
-  c[2] += (unsigned long long)tot[3];
-  c[3] += (unsigned long long)tot[4];
-}
+// The cache records of the pass with header h and the work counters, by the
+// lanes of one wave: their old values and the pass's boxes are loaded by
+// load(), early, and stored by store()
+struct PassRecord {
+  double px, py, paz;
+  Img img;  // of image min(lane, 2)
+  int total;
+  unsigned long long stat, info;  // lanes 0..3
+  __device__ void load(const IbmArgs &a, int n, int lane) {
+    const SliceHead *h = a.heads + n;
+    px = h->px;
+    py = h->py;
+    paz = h->paz;
+    img = (&h->bs.b0)[min(lane, 2)];
+    total = h->bs.total;
+    stat = a.stats[4 * (long)n + min(lane, 3)];
+    info = (unsigned long long)a.slice_info[2 * (long)n + min(lane, 1)];
+  }
+  __device__ void store(const IbmArgs &a, int n, int lane, const double tot[SLICE_VALS]) const {
+    if (lane < 4) {
+      a.sc_pos[4 * (long)n + lane] = lane == 0 ? px : lane == 1 ? py : lane == 2 ? paz : 1.;
+      a.stats[4 * (long)n + lane] =
+          stat + (lane < 2 ? info : (unsigned long long)(lane == 2 ? tot[3] : tot[4]));
+      int *key = a.sc_key + 8 * (long)n + 2 * lane;
+      key[0] = lane < 3 ? img.imin : total;
+      key[1] = lane < 3 ? img.jmin : 1;
+      if (n == 0 && lane == 0) a.stats[4 * (long)a.np] += 1ull;  // IBM calls
+    }
+  }
+  __device__ CachedPass pass() const { return {px, py, paz, img.imin, img.jmin, total, true, true}; }
+};
 
-__device__ void finalize_particle(const IbmArgs &a, int n, int which, bool record = true) {
+__device__ void finalize_particle(const IbmArgs &a, int n, int which) {
+  const int lane = threadIdx.x & 63;
+  PassRecord pr;
+  pr.load(a, n, lane);
   double tot[SLICE_VALS];
   slice_sums(a, a.slice_first[n], a.slice_first[n + 1], tot);
-  if ((threadIdx.x & 63) != 0) return;
+  pr.store(a, n, lane, tot);
+  if (lane != 0) return;
   double *q = a.prt + (long)n * R_N;
   if (which < 2) {
     q[R_IUX + which] = tot[0];
@@ -758,24 +950,28 @@ __device__ void finalize_particle(const IbmArgs &a, int n, int which, bool recor
     q[R_FUY] = tot[1];
     q[R_TVZ] = tot[2];
   }
-  // the cache records and counters (unless another call's); the pass's
-  // header holds its position and boxes
-  if (record) record_pass(a, n, a.heads[n], tot);
 }
 
 // The exchange's sums of particle n and those of the inertia(0) computed
 // beside it, by one wave; the exchange's call records the distance cache
-// and the counters.
+// and the counters.  The first sub-iteration's pass is at the same
+// positions (the increments are zero), whose distances are now cached.
 __device__ inline void finalize_x0_particle(const IbmArgs &a, int n) {
+  const int lane = threadIdx.x & 63;
   finalize_particle(a, n, 2);
   IbmArgs a0 = a;
   a0.slice_part = a.slice_part0;
-  finalize_particle(a0, n, 0, false);
-  // the first sub-iteration's pass, at the cached stage-start positions
-  if ((threadIdx.x & 63) == 0) {
-    const double *q = a.prt + (long)n * R_N;
-    write_head(a, n, q[R_X] + q[R_DX], q[R_Y] + q[R_DY], q[R_AZ] + q[R_DAZ], false);
-  }
+  double tot[SLICE_VALS];
+  slice_sums(a0, a.slice_first[n], a.slice_first[n + 1], tot);
+  if (lane != 0) return;
+  double *q = a.prt + (long)n * R_N;
+  q[R_IUX] = tot[0];
+  q[R_IUY] = tot[1];
+  q[R_IVZ] = tot[2];
+  SliceHead *h = a.heads + n;
+  h->cached = 1;
+  h->warm = 1;
+  h->far = 0;
 }
 
 // one wave per particle, four per workgroup
@@ -860,18 +1056,19 @@ __device__ inline void register_tile(const IbmArgs &a, int tile, int box_id) {
 // already hold them; sliced like k_inertia.  Used before k_exchange when
 // the cache may be stale.
 struct IbmDistB {
-  static constexpr int T = 64, M = 0;
+  static constexpr int T = 64 * WG_WAVES, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a) {
   if (halted(a.halt)) return;
   if (!sub_open(a.res, a.sub)) return;
-  const int slice = vb.bx;
-  const int n = a.slice_owner[slice];
-  const int s0 = a.slice_first[n], nsl = a.slice_first[n + 1] - s0;
+  const int slice = wave_index(vb), lane = wave_lane();
+  if (slice >= a.nslices) return;
+  const int4 rec = a.slice_rec[slice];
+  const int n = rec.x, s0 = rec.y, nsl = rec.z;
   const SliceHead &hd = a.heads[n];
   const BoxSet bs = hd.bs;
   const int total = bs.total;
   if (total > hd.cap || total > nsl * IBM_SLICE) {
-    if (threadIdx.x == 0) atomicOr(&a.flags[0], 1);
+    if (lane == 0) atomicOr(&a.flags[0], 1);
     return;
   }
   const bool cached = hd.cached;
@@ -880,29 +1077,31 @@ struct IbmDistB {
   if (!cached) {
     const EllipseShape e = hd.e;
     const EllipseShape32 f = hd.f;
-    const bool warm = hd.warm;
+    const bool warm = hd.warm, search = !warm || hd.far, single = single_image(bs);
     double *dist = a.sc_dist + hd.off;
-    double *tcell = a.sc_t + hd.off;
+    float *tcell = a.sc_t + hd.off;
     const double cr = hd.cr, sr = hd.sr;
     const int t0 = (slice - s0) * IBM_SLICE;
     const int t1 = t0 + IBM_SLICE < total ? t0 + IBM_SLICE : total;
-    for (int t = t0 + (int)threadIdx.x; t < t1; t += 64) {
+    for (int t = t0 + lane; t < t1; t += 64) {
       int k, i, j;
-      cell_of(bs, t, k, i, j);
+      cell_of(bs, t, k, i, j, single);
       const double py_ = py + a.ly * (k - 1);
-      dist[t] = weight_th(signed_dist_warm(e, f, 1. / a.grid_size, px, py_, cr, sr, a.xc[i],
-                                           a.yc[j - 1], warm, tcell[t], it32, it64));
+      float tp = warm ? tcell[t] : (float)(0.25 * EIF_PI);
+      dist[t] = weight_th(signed_dist_from(e, f, 1. / a.grid_size, px, py_, cr, sr, a.xc[i],
+                                           a.yc[j - 1], search, tp, it32, it64));
+      tcell[t] = tp;
     }
   }
   const double c64 = wave_sum((double)it64), c32 = wave_sum((double)it32);
-  if (threadIdx.x == 0) {
+  if (lane == 0) {
     a.slice_part[SLICE_VALS * (long)slice + 3] = c64;
     a.slice_part[SLICE_VALS * (long)slice + 4] = c32;
     if (slice == s0) a.slice_info[2 * (long)n + 1] = cached ? 0 : total;
   }
 }
 };
-__global__ __launch_bounds__(64) void k_ibm_dist(IbmArgs a) {
+__global__ __launch_bounds__(64 * WG_WAVES) void k_ibm_dist(IbmArgs a) {
   IbmDistB::run(VB::here(), a);
 }
 
@@ -914,12 +1113,13 @@ __global__ __launch_bounds__(64) void k_ibm_dist(IbmArgs a) {
 // distance work.
 // The heads hold the particles' positions without increments.
 struct ExchangeB {
-  static constexpr int T = 64, M = 0;
+  static constexpr int T = 64 * WG_WAVES, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, int own_counts) {
   if (halted(a.halt)) return;
-  const int slice = vb.bx;
-  const int n = a.slice_owner[slice];
-  const int s0 = a.slice_first[n], nsl = a.slice_first[n + 1] - s0;
+  const int slice = wave_index(vb), lane = wave_lane();
+  if (slice >= a.nslices) return;
+  const int4 rec = a.slice_rec[slice];
+  const int n = rec.x, s0 = rec.y, nsl = rec.z;
   const double *q = a.prt + (long)n * R_N;
   const SliceHead &hd = a.heads[n];
   const double dt = a.dscal[S_DT];
@@ -930,11 +1130,11 @@ struct ExchangeB {
   const BoxSet bs = hd.bs;
   const int total = bs.total;
   if (total > hd.cap || total > nsl * IBM_SLICE) {
-    if (threadIdx.x == 0) atomicOr(&a.flags[0], 1);
+    if (lane == 0) atomicOr(&a.flags[0], 1);
     return;
   }
   if (slice == s0) {
-    if (threadIdx.x == 0) {
+    if (lane == 0) {
       long off = hd.off;
 #pragma unroll
       for (int k = 0; k < 3; k++) {
@@ -965,8 +1165,8 @@ struct ExchangeB {
       const TileRange &rg = tr[r & 1];
       const int cnt = rg.count();
       const int w = rg.tx1 - rg.tx0 + 1;
-      if ((int)threadIdx.x < cnt) tile_[r] = (rg.ty0 + (int)threadIdx.x / w) * a.ntx + rg.tx0 + (int)threadIdx.x % w;
-      for (int e_ = threadIdx.x + 64; e_ < cnt; e_ += 64)
+      if (lane < cnt) tile_[r] = (rg.ty0 + lane / w) * a.ntx + rg.tx0 + lane % w;
+      for (int e_ = lane + 64; e_ < cnt; e_ += 64)
         register_tile(a, (rg.ty0 + e_ / w) * a.ntx + rg.tx0 + e_ % w, n * 3 + r / 2);
     }
 #pragma unroll
@@ -995,30 +1195,28 @@ struct ExchangeB {
     constexpr int U = IBM_SLICE / 64;
     double th_[U], x_[U], y_[U], fx0[U], fx1[U], fy0[U], fy1[U], sx0[U], sx1[U], sy0[U],
         sy1[U];
-    int k_[U];
+    int k_[U], i_[U], j_[U];
+    lane_cells<U>(bs, t0, t1, lane, k_, i_, j_);
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int t = min(t0 + (int)threadIdx.x + 64 * u, t1 - 1);
-      int k, i, j;
-      cell_of(bs, t, k, i, j);
-      k_[u] = k;
-      x_[u] = a.xc[i];
-      y_[u] = a.yc[j - 1];
-      th_[u] = dist[t];
-      fx0[u] = a.ux[a.L.ux(i, j)];
-      fx1[u] = a.ux[a.L.ux(i + 1, j)];
-      fy0[u] = a.uy[a.L.p(i, j)];
-      fy1[u] = a.uy[a.L.p(i, j + 1)];
+      const unsigned fx = face_x(a.L, i_[u], j_[u]), fy = face_y(a.L, i_[u], j_[u]);
+      x_[u] = a.xc[i_[u]];
+      y_[u] = a.yc[j_[u] - 1];
+      th_[u] = dist[min(t0 + lane + 64 * u, t1 - 1)];
+      fx0[u] = a.ux[fx];
+      fx1[u] = a.ux[fx + 1];
+      fy0[u] = a.uy[fy];
+      fy1[u] = a.uy[fy + (unsigned)(a.nx + 2)];
       if (a.us_x) {
-        sx0[u] = a.us_x[a.L.ux(i, j)];
-        sx1[u] = a.us_x[a.L.ux(i + 1, j)];
-        sy0[u] = a.us_y[a.L.p(i, j)];
-        sy1[u] = a.us_y[a.L.p(i, j + 1)];
+        sx0[u] = a.us_x[fx];
+        sx1[u] = a.us_x[fx + 1];
+        sy0[u] = a.us_y[fy];
+        sy1[u] = a.us_y[fy + (unsigned)(a.nx + 2)];
       }
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int t = t0 + (int)threadIdx.x + 64 * u;
+      const int t = t0 + lane + 64 * u;
       if (t >= t1) continue;
       const double py_ = py + a.ly * (k_[u] - 1);
       const double x = x_[u], y = y_[u];
@@ -1050,7 +1248,7 @@ struct ExchangeB {
   const double s0v = wave_sum(acc[0]), s1v = wave_sum(acc[1]), s2v = wave_sum(acc[2]);
   if (a.us_x) {
     const double i0 = wave_sum(ai[0]), i1 = wave_sum(ai[1]), i2 = wave_sum(ai[2]);
-    if (threadIdx.x == 0) {
+    if (lane == 0) {
       double *pp = a.slice_part0 + SLICE_VALS * (long)slice;
       pp[0] = i0;
       pp[1] = i1;
@@ -1059,7 +1257,7 @@ struct ExchangeB {
       pp[4] = 0.;
     }
   }
-  if (threadIdx.x == 0) {
+  if (lane == 0) {
     double *pp = a.slice_part + SLICE_VALS * (long)slice;
     pp[0] = s0v;
     pp[1] = s1v;
@@ -1075,7 +1273,7 @@ struct ExchangeB {
   }
 }
 };
-__global__ __launch_bounds__(64) void k_exchange(IbmArgs a, int own_counts) {
+__global__ __launch_bounds__(64 * WG_WAVES) void k_exchange(IbmArgs a, int own_counts) {
   ExchangeB::run(VB::here(), a, own_counts);
 }
 
@@ -1084,7 +1282,7 @@ __global__ __launch_bounds__(64) void k_exchange(IbmArgs a, int own_counts) {
 // ---------------------------------------------------------------------
 struct TileArgs {
   Layout L;
-  int nx, ny, ntx;
+  int nx, ny, ntx, ntiles;
   const Box *boxes;
   const double *sc_fx, *sc_fy;
   const int *tile_cnt, *tile_list;
@@ -1106,42 +1304,43 @@ __device__ inline double box_value(const Box &b, const double *sc, int i, int j)
 // (particle index, then image; a box registered twice counts once), the
 // boxes are staged in LDS, and every cell sums its boxes' values in that
 // order.
-constexpr int TILE_THREADS = 64;
-static_assert(TILE_X == TILE_THREADS, "one lane per tile column");
-static_assert(TILE_CAP <= TILE_THREADS, "one lane per registration");
+constexpr int TILE_THREADS = 64 * WG_WAVES;
+static_assert(TILE_X == 64, "one lane per tile column");
+static_assert(TILE_CAP <= 64, "one lane per registration");
 
 __device__ __forceinline__ void tile_body(const TileArgs &a, int tile) {
-  __shared__ int raw[TILE_CAP];
-  __shared__ bool rep[TILE_CAP];
-  __shared__ Box sbox[TILE_CAP];
-  __shared__ int nlist;
+  __shared__ int raw_[WG_WAVES][TILE_CAP];
+  __shared__ bool rep_[WG_WAVES][TILE_CAP];
+  __shared__ Box sbox_[WG_WAVES][TILE_CAP];
+  const int wv = wave_in_group();
+  int *raw = raw_[wv];
+  bool *rep = rep_[wv];
+  Box *sbox = sbox_[wv];
   // tiles in grid order, so neighbouring workgroups touch neighbouring
   // memory; tiles no box reaches return at once
   const int cnt = min(a.tile_cnt[tile], TILE_CAP);
   if (cnt == 0) return;
-  const int lane = threadIdx.x;
+  const int lane = wave_lane();
   const Layout L = a.L;
   const int tx = tile % a.ntx, ty = tile / a.ntx;
   const int i0 = tx * TILE_X + 1, j0 = ty * TILE_Y + 1;
   if (lane < cnt) raw[lane] = a.tile_list[(long)tile * TILE_CAP + lane];
-  if (lane == 0) nlist = 0;
-  __syncthreads();
+  wave_sync();
   int v = 0;
+  bool dup = false;
   if (lane < cnt) {
     v = raw[lane];
-    bool dup = false;
     for (int s = 0; s < lane; s++) dup |= raw[s] == v;
     rep[lane] = dup;
   }
-  __syncthreads();
-  if (lane < cnt && !rep[lane]) {
+  wave_sync();
+  if (lane < cnt && !dup) {
     int pos = 0;
     for (int s = 0; s < cnt; s++) pos += raw[s] < v && !rep[s];
     sbox[pos] = a.boxes[v];
-    atomicMax(&nlist, pos + 1);
   }
-  __syncthreads();
-  const int nl = nlist;
+  wave_sync();
+  const int nl = __popcll(__ballot(lane < cnt && !dup));  // every box once
   // column i0-1+lane of DUX and column i0+lane of DUY on rows j0-1 .. j0+3
   // (DUY's row j0-1 = 0 is row jtot), then column i0+lane of the tile.
   // Boxes outermost: the 13 loads of one box are in flight together, and
@@ -1211,7 +1410,8 @@ struct TilesB {
   static constexpr int T = TILE_THREADS, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, TileArgs a) {
   if (halted(a.halt)) return;
-  tile_body(a, vb.bx);
+  const int tile = wave_index(vb);
+  if (tile < a.ntiles) tile_body(a, tile);
 }
 };
 __global__ __launch_bounds__(TILE_THREADS) void k_tiles(TileArgs a) {
@@ -1226,10 +1426,11 @@ struct TilesX0B {
   static constexpr int T = TILE_THREADS, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, TileArgs t, IbmArgs a) {
   if (halted(a.halt)) return;
-  if ((int)vb.bx < a.np)
-    finalize_x0_particle(a, vb.bx);
-  else
-    tile_body(t, vb.bx - a.np);
+  const int k = wave_index(vb);
+  if (k < a.np)
+    finalize_x0_particle(a, k);
+  else if (k - a.np < t.ntiles)
+    tile_body(t, k - a.np);
 }
 };
 __global__ __launch_bounds__(TILE_THREADS) void k_tiles_x0(TileArgs t, IbmArgs a) {
@@ -1333,8 +1534,12 @@ __device__ inline bool pair_candidate(const CollArgs &a, int n0, int n1) {
   const double x0 = p0[0], y0 = p0[1];
   const double x1 = p1[0], y1r = p1[1];
   const double y1 = y1r + min_image_offset(y0, y1r, a.ly);
-  const double norm = fmax(hypot(x1 - x0, y1 - y0), DBL_EPSILON);
-  return !(p0[2] + p1[2] - norm < 0.);
+  const double dx = x1 - x0, dy = y1 - y0, r = p0[2] + p1[2];
+  // far apart by the squares, with a margin far above their rounding: the
+  // exact test would say so too (and NaN goes on to it)
+  if (dx * dx + dy * dy > r * r * (1. + 1e-12)) return false;
+  const double norm = fmax(hypot(dx, dy), DBL_EPSILON);
+  return !(r - norm < 0.);
 }
 
 // the packed positions and radii of the broad phase, from the records
@@ -1386,9 +1591,9 @@ __device__ bool contact_force(const CollArgs &a, int n0, int n1, int wall, int s
   // find_equivalent_circles, collision.c:111-135 (guarded iteration count)
   const EllipseShape sh = make_shape(e.a, e.b);
   const EllipseShape32 f = shape32(sh);
-  double cm, sm, cp, sp;
-  sincos(-e.angle, &sm, &cm);
-  sincos(+e.angle, &sp, &cp);
+  double cp, sp;
+  sincos_angle(e.angle, sp, cp);
+  const double cm = cp, sm = -sp;
   double tw = -1.;
   double cx = e.x, cy = e.y, cr = 0., ix = 0., iy = 0.;
   for (int it = 0;; it++) {
@@ -1473,7 +1678,7 @@ constexpr int COLL_CAND_CAP = 256;  // candidate partners per particle
 // the candidates of particle n among the particles of cell c (in the cell
 // list's order), appended to s_cand
 __device__ inline void cell_candidates(const CollArgs &a, int n, int c, int *s_cand, int &cnt) {
-  const int lane = threadIdx.x;
+  const int lane = wave_lane();
   const int s0 = a.cl_start[c], s1 = a.cl_start[c + 1];
   for (int base = s0; base < s1; base += 64) {
     const int k = base + lane;
@@ -1489,9 +1694,10 @@ __device__ inline void cell_candidates(const CollArgs &a, int n, int c, int *s_c
 }
 
 __device__ void collide_particle(const CollArgs &a, int n) {
-  __shared__ int s_cand[COLL_CAND_CAP];
-  __shared__ int s_sorted[COLL_CAND_CAP];
-  const int lane = threadIdx.x;
+  __shared__ int s_cand_[WG_WAVES][COLL_CAND_CAP];
+  __shared__ int s_sorted_[WG_WAVES][COLL_CAND_CAP];
+  int *s_cand = s_cand_[wave_in_group()], *s_sorted = s_sorted_[wave_in_group()];
+  const int lane = wave_lane();
   int cnt = 0;
   const int *cand = s_cand;
   if (a.use_cells) {
@@ -1510,7 +1716,7 @@ __device__ void collide_particle(const CollArgs &a, int n) {
       if (lane == 0) atomicOr(&a.flags[0], 4);
       cnt = COLL_CAND_CAP;
     }
-    __syncthreads();
+    wave_sync();
     // ascending partner order, as the scan over all particles finds them:
     // each candidate's rank is the number of smaller ones (all distinct)
     for (int k = lane; k < cnt; k += 64) {
@@ -1536,7 +1742,7 @@ __device__ void collide_particle(const CollArgs &a, int n) {
       cnt = COLL_CAND_CAP;
     }
   }
-  __syncthreads();
+  wave_sync();
   double fx = 0., fy = 0., tz = 0.;
   int ncont = 0;
   int *row = a.rows + (long)n * CONTACT_CAP;
@@ -1585,16 +1791,17 @@ __device__ void collide_particle(const CollArgs &a, int n) {
   }
 }
 
-// one 64-lane workgroup per particle
+// one wave per particle
 struct CollideB {
-  static constexpr int T = 64, M = 0;
+  static constexpr int T = 64 * WG_WAVES, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, CollArgs a) {
   if (halted(a.halt)) return;
   if (!sub_open(a.res, a.sub)) return;
-  collide_particle(a, vb.bx);
+  const int n = wave_index(vb);
+  if (n < a.np) collide_particle(a, n);
 }
 };
-__global__ __launch_bounds__(64) void k_collide(CollArgs a) {
+__global__ __launch_bounds__(64 * WG_WAVES) void k_collide(CollArgs a) {
   CollideB::run(VB::here(), a);
 }
 
@@ -1705,23 +1912,24 @@ __global__ __launch_bounds__(256) void k_cell_place(CollArgs a) {
 
 // One launch for a sub-iteration's inertia(1) and collision(1), which read
 // the same positions and write disjoint particle members: the first np
-// workgroups are the collisions (long, started first), the rest the IBM
+// waves are the collisions (long, started first), the rest the IBM
 // slices.  Bounded to 4 waves per SIMD (128 VGPRs): the collision path
 // alone needs more and spills a little, which costs less than the
 // occupancy its registers would take from the slices.
 struct InertiaCollideB {
-  static constexpr int T = 64, M = 4;
+  static constexpr int T = 64 * WG_WAVES, M = 4;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, CollArgs ca, int cnstep) {
   if (halted(a.halt)) return;
   const bool open = sub_open(a.res, a.sub);
-  if ((int)vb.bx < ca.np) {
-    if (open) collide_particle(ca, vb.bx);
-  } else {
-    inertia_slice(a, cnstep, vb.bx - ca.np, open);
+  const int k = wave_index(vb);
+  if (k < ca.np) {
+    if (open) collide_particle(ca, k);
+  } else if (k - ca.np < a.nslices) {
+    inertia_slice(a, cnstep, k - ca.np, open);
   }
 }
 };
-__global__ __launch_bounds__(64, 4) void k_inertia_collide(IbmArgs a, CollArgs ca, int cnstep) {
+__global__ __launch_bounds__(64 * WG_WAVES, 4) void k_inertia_collide(IbmArgs a, CollArgs ca, int cnstep) {
   InertiaCollideB::run(VB::here(), a, ca, cnstep);
 }
 
@@ -1755,107 +1963,118 @@ __global__ void k_zero_residual(double *dscal) {
 
 // src/suspensions/increment.c:10-64
 // fin: also finalises the preceding inertia(1) call (its slice sums and
-// cache records) for this particle first, saving a launch per sub-iteration
-// one wave per particle (its lanes finalise the inertia sums), four per
-// workgroup; lane 0 computes the increment
+// cache records) for this particle first, saving a launch per sub-iteration.
+//
+// One wave per particle, four per workgroup, sixteen from INC_WIDE particles
+// on: every workgroup ends with an atomic maximum on one address, and 1024
+// of those take 8 us (4096 particles 15.4 -> 9.3 us by the wide workgroups;
+// 1024 particles 8.7 -> 9.9, 64 particles 5.2 -> 8.6, where the sixteen waves
+// share a CU's issue).  The launch is as long as one wave's chain of loads and dependent operations, so the wave issues every
+// load before it tests the gate, holds the record one member a lane (read
+// back by readlane), and spreads what is independent over lanes: the three
+// images' boxes, the cache records and the counters.  With its
+// predecessor's chain on lane 0 (and the header copied through scratch) it
+// took 9.7 us at 1024 particles, 7.2 at 64, 16.7 at 4096.
+constexpr int INC_WIDE = 2048;
 struct IncrementB {
-  static constexpr int T = 256, M = 0;
+  static constexpr int T = 1024, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, double *prt, int np, const double *dscal,
                                                    double ga, double Fr, double *res_out,
                                                    IbmArgs ia, int fin) {
-  if (halted(ia.halt)) return;
-  const bool open = sub_open(ia.res, ia.sub);
-  __shared__ double red[4];
+  __shared__ double red[16];
+  const int waves = blockDim.x >> 6;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int n = vb.bx * 4 + w;
-  // the slice range and lane 0's record inputs are loaded before the gate
-  // is tested (all threads of the workgroup see the same gate), so that
-  // their latencies overlap
+  const int n = vb.bx * waves + w, nc = min(n, np - 1);
+  double *p = prt + (long)nc * R_N;
+  const int stop = ia.halt ? *ia.halt : 0;
+  const double res_prev = ia.res && ia.sub > 0 ? ia.res[ia.sub - 1] : 1.;
+  const double dt = dscal[S_DT];
+  const double rec = p[min(lane, R_N - 1)];
   int s0 = 0, s1 = 0;
-  if (n < np && fin) {
-    s0 = ia.slice_first[n];
-    s1 = ia.slice_first[n + 1];
+  PassRecord pr;
+  CachedPass prev;
+  if (fin) {
+    s0 = ia.slice_first[nc];
+    s1 = ia.slice_first[nc + 1];
+    pr.load(ia, nc, lane);
+  } else {
+    prev = cached_records(ia, nc, lane);
   }
-  double dt = 0., den = 0., dux_prev = 0., duy_prev = 0., dvz_prev = 0.;
-  double cfx0 = 0., cfy0 = 0., ctz0 = 0., cfx1 = 0., cfy1 = 0., ctz1 = 0.;
-  double fux = 0., fuy = 0., tvz = 0., iux0 = 0., iuy0 = 0., ivz0 = 0.;
-  double ux0 = 0., uy0 = 0., vz0 = 0., x0 = 0., y0 = 0., az0 = 0., rad = 0.;
-  double iux1 = 0., iuy1 = 0., ivz1 = 0.;
-  SliceHead hd{};
-  double *p = prt + (long)n * R_N;
-  if (n < np && lane == 0) {
-    dt = dscal[S_DT];
-    den = p[R_DEN];
-    dux_prev = p[R_DUX]; duy_prev = p[R_DUY]; dvz_prev = p[R_DVZ];
-    cfx0 = p[R_CFX]; cfy0 = p[R_CFY]; ctz0 = p[R_CTZ];
-    cfx1 = p[R_CFX + 1]; cfy1 = p[R_CFY + 1]; ctz1 = p[R_CTZ + 1];
-    fux = p[R_FUX]; fuy = p[R_FUY]; tvz = p[R_TVZ];
-    iux0 = p[R_IUX]; iuy0 = p[R_IUY]; ivz0 = p[R_IVZ];
-    ux0 = p[R_UX]; uy0 = p[R_UY]; vz0 = p[R_VZ];
-    x0 = p[R_X]; y0 = p[R_Y]; az0 = p[R_AZ];
-    rad = fmax(p[R_A], p[R_B]);
-    if (fin) {
-      hd = ia.heads[n];
-    } else {
-      iux1 = p[R_IUX + 1];
-      iuy1 = p[R_IUY + 1];
-      ivz1 = p[R_IVZ + 1];
-    }
-  }
-  if (!open) return;
+  // all threads of the workgroup see the same gate
+  if (stop || (ia.res && ia.sub > 0 && (res_prev < 1.e-8 || ia.sub > 101))) return;
+  auto member = [&](int m) { return lane_value(rec, m); };
   double res = 0.;
-  double tot[SLICE_VALS];
-  if (n < np && fin) slice_sums(ia, s0, s1, tot);
-  if (n < np && lane == 0) {
+  if (n < np) {
+    double iux1, iuy1, ivz1;
     if (fin) {  // inertia(1) of this sub-iteration: its sums and cache records
+      double tot[SLICE_VALS];
+      slice_sums(ia, s0, s1, tot);
       iux1 = tot[0];
       iuy1 = tot[1];
       ivz1 = tot[2];
-      p[R_IUX + 1] = iux1;
-      p[R_IUY + 1] = iuy1;
-      p[R_IVZ + 1] = ivz1;
-      record_pass(ia, n, hd, tot);
+      pr.store(ia, n, lane, tot);
+      prev = pr.pass();
+    } else {
+      iux1 = member(R_IUX + 1);
+      iuy1 = member(R_IUY + 1);
+      ivz1 = member(R_IVZ + 1);
     }
-    if (ia.res && ia.sub == 0) {  // collision(1) at the stage-start positions
-      cfx1 = cfx0;
-      cfy1 = cfy0;
-      ctz1 = ctz0;
-      p[R_CFX + 1] = cfx1;
-      p[R_CFY + 1] = cfy1;
-      p[R_CTZ + 1] = ctz1;
-    }
-    const double dux = +0.5 * ga * dt * (cfx0 + cfx1) + dt * fux + (iux1 - iux0)
+    const double cfx0 = member(R_CFX), cfy0 = member(R_CFY), ctz0 = member(R_CTZ);
+    // sub-iteration 0: collision(1) at the stage-start positions
+    const bool first = ia.res && ia.sub == 0;
+    const double cfx1 = first ? cfx0 : member(R_CFX + 1);
+    const double cfy1 = first ? cfy0 : member(R_CFY + 1);
+    const double ctz1 = first ? ctz0 : member(R_CTZ + 1);
+    const double den = member(R_DEN);
+    const double dux = +0.5 * ga * dt * (cfx0 + cfx1) + dt * member(R_FUX) + (iux1 - member(R_IUX))
                        + 1.0 * ga * dt * (1. - den) / (Fr * Fr);
-    const double duy = +0.5 * ga * dt * (cfy0 + cfy1) + dt * fuy + (iuy1 - iuy0);
-    const double dvz = +0.5 * ga * dt * (ctz0 + ctz1) + dt * tvz + (ivz1 - ivz0);
-    p[R_DUX] = dux;
-    p[R_DUY] = duy;
-    p[R_DVZ] = dvz;
-    res = fmax(res, fabs(dux - dux_prev));
-    res = fmax(res, fabs(duy - duy_prev));
-    res = fmax(res, fabs(dvz - dvz_prev));
+    const double duy = +0.5 * ga * dt * (cfy0 + cfy1) + dt * member(R_FUY) + (iuy1 - member(R_IUY));
+    const double dvz = +0.5 * ga * dt * (ctz0 + ctz1) + dt * member(R_TVZ) + (ivz1 - member(R_IVZ));
+    res = fmax(res, fabs(dux - member(R_DUX)));
+    res = fmax(res, fabs(duy - member(R_DUY)));
+    res = fmax(res, fabs(dvz - member(R_DVZ)));
+    const double ux0 = member(R_UX), uy0 = member(R_UY), vz0 = member(R_VZ);
     const double ux1 = ux0 + dux, uy1 = uy0 + duy, vz1 = vz0 + dvz;
     const double dxn = 0.5 * ga * dt * (ux0 + ux1);
     const double dyn = 0.5 * ga * dt * (uy0 + uy1);
     const double dazn = 0.5 * ga * dt * (vz0 + vz1);
-    p[R_DX] = dxn;
-    p[R_DY] = dyn;
-    p[R_DAZ] = dazn;
-    // the broad phase's packed position for the next sub-iteration's collisions
-    double *cp = ia.cpos + 4 * (long)n;
-    cp[0] = x0 + dxn;
-    cp[1] = y0 + dyn;
-    cp[2] = rad;
+    const double x = member(R_X) + dxn, y = member(R_Y) + dyn, az = member(R_AZ) + dazn;
+    const double lo = fmin(member(R_A), member(R_B)), hi = fmax(member(R_A), member(R_B));
+    if (lane == 0) {
+      if (fin) {
+        p[R_IUX + 1] = iux1;
+        p[R_IUY + 1] = iuy1;
+        p[R_IVZ + 1] = ivz1;
+      }
+      if (first) {
+        p[R_CFX + 1] = cfx1;
+        p[R_CFY + 1] = cfy1;
+        p[R_CTZ + 1] = ctz1;
+      }
+      p[R_DUX] = dux;
+      p[R_DUY] = duy;
+      p[R_DVZ] = dvz;
+      p[R_DX] = dxn;
+      p[R_DY] = dyn;
+      p[R_DAZ] = dazn;
+      // the broad phase's packed position for the next sub-iteration's collisions
+      double *cp = ia.cpos + 4 * (long)n;
+      cp[0] = x;
+      cp[1] = y;
+      cp[2] = hi;
+    }
     // the next sub-iteration's inertia pass
-    write_head(ia, n, x0 + dxn, y0 + dyn, az0 + dazn, false, fin ? &hd : nullptr, rad);
+    write_head(ia, ia.heads + n, lane, x, y, az, lo, hi, prev, fin != 0);
   }
   if (lane == 0) red[w] = res;
   __syncthreads();
-  if (threadIdx.x == 0)
-    atomic_max_nonneg(res_out, fmax(fmax(red[0], red[1]), fmax(red[2], red[3])));
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < waves; k++) res = fmax(res, red[k]);
+    atomic_max_nonneg(res_out, res);
+  }
 }
 };
-__global__ __launch_bounds__(256) void k_increment(double *prt, int np, const double *dscal,
+__global__ __launch_bounds__(1024) void k_increment(double *prt, int np, const double *dscal,
                                                    double ga, double Fr, double *res_out,
                                                    IbmArgs ia, int fin) {
   IncrementB::run(VB::here(), prt, np, dscal, ga, Fr, res_out, ia, fin);
@@ -1885,34 +2104,74 @@ __global__ void k_update_particles(double *prt, int np, double ly, const int *ha
   UpdateParticlesB::run(VB::here(), prt, np, ly, halt);
 }
 
-// src/suspensions/reset.c:7-18
+// src/suspensions/reset.c:7-18, by one wave per particle, four per workgroup
+// update: the previous stage's particle update (UpdateParticlesB's
+// operations) first, in the same launch
 // res (RES_SLOTS sub-iteration residuals) and tile_cnt (ntiles): cleared
 // when given, for the stage's sub-iterations and the next exchange's tile
 // registrations
 // Also the heads of the stage-start pass (positions without increments).
 struct ResetB {
-  static constexpr int T = 1024, M = 0;
-  static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, double *res, int *tile_cnt, int ntiles) {
-  if (halted(a.halt)) return;
-  const int n = vb.bx * blockDim.x + threadIdx.x;
-  if (res && n < RES_SLOTS) res[n] = 0.;
-  if (tile_cnt && n < ntiles) tile_cnt[n] = 0;
-  if (n >= a.np) return;
-  // foot-point warm starts reach back no further than the stage start, so
-  // that a run restarted from a save repeats the same operations
-  a.sc_key[8 * (long)n + 7] = 0;
-  double *p = a.prt + (long)n * R_N;
-  p[R_DUX] = 0.;
-  p[R_DUY] = 0.;
-  p[R_DVZ] = 0.;
-  p[R_DX] = 0.;
-  p[R_DY] = 0.;
-  p[R_DAZ] = 0.;
-  write_head(a, n, p[R_X], p[R_Y], p[R_AZ], true);
-}
+  static constexpr int T = 256, M = 0;
+  static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, double *res, int *tile_cnt,
+                                             int ntiles, int update) {
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int n = vb.bx * 4 + w, nc = max(min(n, a.np - 1), 0);
+    const int stop = a.halt ? *a.halt : 0;
+    double rec = 0.;
+    CachedPass prev{};
+    double *p = a.prt + (long)nc * R_N;
+    if (a.np > 0) {
+      rec = p[min(lane, R_N - 1)];
+      prev = cached_records(a, nc, lane);
+    }
+    if (stop) return;
+    const int t = vb.bx * blockDim.x + threadIdx.x;
+    if (res && t < RES_SLOTS) res[t] = 0.;
+    if (tile_cnt)
+      for (int k = t; k < ntiles; k += vb.gx * blockDim.x) tile_cnt[k] = 0;
+    if (n >= a.np) return;
+    auto member = [&](int m) { return lane_value(rec, m); };
+    double x = member(R_X), y = member(R_Y), az = member(R_AZ);
+    if (update) {
+      x += member(R_DX);
+      y += member(R_DY);
+      az += member(R_DAZ);
+      if (y < 0.) y += a.ly;
+      if (y > a.ly) y -= a.ly;
+      if (az < 0.) az += 2. * EIF_PI;
+      if (az > 2. * EIF_PI) az -= 2. * EIF_PI;
+    }
+    SliceHead *h = a.heads + n;
+    const double pa = member(R_A), pb = member(R_B);
+    if (lane == 0) {
+      if (update) {
+        p[R_UX] = member(R_UX) + member(R_DUX);
+        p[R_UY] = member(R_UY) + member(R_DUY);
+        p[R_VZ] = member(R_VZ) + member(R_DVZ);
+        p[R_X] = x;
+        p[R_Y] = y;
+        p[R_AZ] = az;
+      }
+      p[R_DUX] = 0.;
+      p[R_DUY] = 0.;
+      p[R_DVZ] = 0.;
+      p[R_DX] = 0.;
+      p[R_DY] = 0.;
+      p[R_DAZ] = 0.;
+      // foot-point warm starts reach back no further than the stage start, so
+      // that a run restarted from a save repeats the same operations
+      a.sc_key[8 * (long)n + 7] = 0;
+    }
+    prev.boxes = false;
+    double q[3] = {member(R_DEN), pa, pb};  // the members that the shape needs
+    write_head_shape(a, h, n, lane, q);
+    write_head(a, h, lane, x, y, az, fmin(pa, pb), fmax(pa, pb), prev, false);
+  }
 };
-__global__ void k_reset(IbmArgs a, double *res, int *tile_cnt, int ntiles) {
-  ResetB::run(VB::here(), a, res, tile_cnt, ntiles);
+__global__ __launch_bounds__(256) void k_reset(IbmArgs a, double *res, int *tile_cnt, int ntiles,
+                                               int update) {
+  ResetB::run(VB::here(), a, res, tile_cnt, ntiles, update);
 }
 
 // ---------------------------------------------------------------------
@@ -1952,8 +2211,9 @@ static IbmArgs ibm_args(Ctx *c) {
   a.stats = c->ibm_pp;
   a.cpos = c->cpos;
   a.np = c->np;
+  a.nslices = c->nslices;
   a.slice_first = c->slice_first;
-  a.slice_owner = c->slice_owner;
+  a.slice_rec = c->slice_rec;
   a.slice_info = c->slice_info;
   a.res = nullptr;
   a.sub = 0;
@@ -1964,6 +2224,9 @@ static IbmArgs ibm_args(Ctx *c) {
   a.halt = c->halt;
   return a;
 }
+
+// workgroups of n waves
+static dim3 wave_grid(long n) { return dim3((unsigned)((n + WG_WAVES - 1) / WG_WAVES)); }
 
 int launch_ref_iterations(Ctx *c, unsigned long long *dout) {
   if (c->np == 0) return EIF_OK;
@@ -1997,11 +2260,12 @@ int susp_init(Ctx *c) {
   EIF_HIP(hipMalloc(&c->slice_first, (c->np + 1) * sizeof(int)));
   EIF_HIP(hipMemcpy(c->slice_first, first.data(), (c->np + 1) * sizeof(int), hipMemcpyHostToDevice));
   {
-    std::vector<int> owner(c->nslices > 0 ? c->nslices : 1, 0);
+    std::vector<int4> rec(c->nslices > 0 ? c->nslices : 1, int4{0, 0, 0, 0});
     for (int n = 0; n < c->np; n++)
-      for (int sl = first[n]; sl < first[n + 1]; sl++) owner[sl] = n;
-    EIF_HIP(hipMalloc(&c->slice_owner, owner.size() * sizeof(int)));
-    EIF_HIP(hipMemcpy(c->slice_owner, owner.data(), owner.size() * sizeof(int), hipMemcpyHostToDevice));
+      for (int sl = first[n]; sl < first[n + 1]; sl++)
+        rec[sl] = int4{n, first[n], first[n + 1] - first[n], 0};
+    EIF_HIP(hipMalloc(&c->slice_rec, rec.size() * sizeof(int4)));
+    EIF_HIP(hipMemcpy(c->slice_rec, rec.data(), rec.size() * sizeof(int4), hipMemcpyHostToDevice));
   }
   EIF_HIP(hipMalloc(&c->slice_info, 2 * (size_t)(c->np > 0 ? c->np : 1) * sizeof(long)));
   EIF_HIP(hipMemset(c->slice_info, 0, 2 * (size_t)(c->np > 0 ? c->np : 1) * sizeof(long)));
@@ -2016,7 +2280,7 @@ int susp_init(Ctx *c) {
   EIF_HIP(hipMalloc(&c->sc_fx, sc));
   EIF_HIP(hipMalloc(&c->sc_fy, sc));
   EIF_HIP(hipMalloc(&c->sc_dist, sc));
-  EIF_HIP(hipMalloc(&c->sc_t, sc));
+  EIF_HIP(hipMalloc(&c->sc_t, sc / 2));
   EIF_HIP(hipMalloc(&c->sc_key, 8 * (size_t)(c->np > 0 ? c->np : 1) * sizeof(int)));
   EIF_HIP(hipMemset(c->sc_key, 0, 8 * (size_t)(c->np > 0 ? c->np : 1) * sizeof(int)));
   EIF_HIP(hipMalloc(&c->sc_pos, 4 * (size_t)(c->np > 0 ? c->np : 1) * sizeof(double)));
@@ -2043,13 +2307,13 @@ int susp_init(Ctx *c) {
   return EIF_OK;
 }
 
-int launch_reset(Ctx *c, hipStream_t st, bool clear_tiles) {
+int launch_reset(Ctx *c, hipStream_t st, bool clear_tiles, bool update) {
   if (!st) st = c->stream;
   // also clears the sub-iteration residuals, so it runs without particles too
   const int ntiles = c->np > 0 && clear_tiles ? c->ntx * c->nty : 0;
-  const int n = std::max(std::max(c->np, ntiles), RES_SLOTS);
-  go<ResetB>(k_reset, dim3((n + 255) / 256), dim3(256), 0, st, ibm_args(c),
-                     c->res_slots, ntiles > 0 ? c->tile_cnt : nullptr, ntiles);
+  const int grid = std::max({(c->np + 3) / 4, (ntiles + 1023) / 1024, 1});
+  go<ResetB>(k_reset, dim3(grid), dim3(256), 0, st, ibm_args(c),
+                     c->res_slots, ntiles > 0 ? c->tile_cnt : nullptr, ntiles, update ? 1 : 0);
   EIF_HIP(hipGetLastError());
   return EIF_OK;
 }
@@ -2059,8 +2323,8 @@ int launch_inertia(Ctx *c, int cnstep, hipStream_t st, bool defer_finalize) {
   if (!st) st = c->stream;
   ProfScope ps(c, "ibm_inertia", st);
   IbmArgs a = ibm_args(c);
-  go<HeadsB>(k_heads, dim3((c->np + 255) / 256), dim3(256), 0, st, a, 1);
-  go<InertiaB>(k_inertia, dim3(c->nslices), dim3(64), 0, st, a, cnstep);
+  go<HeadsB>(k_heads, dim3((c->np + 3) / 4), dim3(256), 0, st, a, 1);
+  go<InertiaB>(k_inertia, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, st, a, cnstep);
   if (!defer_finalize)
     go<IbmFinalizeB>(k_ibm_finalize, dim3((c->np + 3) / 4), dim3(256), 0, st, a, cnstep);
   EIF_HIP(hipGetLastError());
@@ -2076,10 +2340,10 @@ int launch_exchange(Ctx *c, bool cached_known, bool tiles_clear, bool defer_fina
                        c->stream, c->tile_cnt, (int)ntiles);
   }
   IbmArgs a = ibm_args(c);
-  go<HeadsB>(k_heads, dim3((c->np + 255) / 256), dim3(256), 0, c->stream, a, 0);
+  go<HeadsB>(k_heads, dim3((c->np + 3) / 4), dim3(256), 0, c->stream, a, 0);
   if (!cached_known)
-    go<IbmDistB>(k_ibm_dist, dim3(c->nslices), dim3(64), 0, c->stream, a);
-  go<ExchangeB>(k_exchange, dim3(c->nslices), dim3(64), 0, c->stream, a,
+    go<IbmDistB>(k_ibm_dist, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a);
+  go<ExchangeB>(k_exchange, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a,
                      cached_known ? 1 : 0);
   EIF_HIP(hipGetLastError());
   if (!defer_finalize) return launch_exchange_finalize(c, c->stream);
@@ -2090,7 +2354,7 @@ int launch_exchange(Ctx *c, bool cached_known, bool tiles_clear, bool defer_fina
 // positions without increments, into the per-cell cache
 int launch_ibm_dist(Ctx *c, hipStream_t st) {
   if (c->np == 0) return EIF_OK;
-  go<IbmDistB>(k_ibm_dist, dim3(c->nslices), dim3(64), 0, st ? st : c->stream,
+  go<IbmDistB>(k_ibm_dist, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, st ? st : c->stream,
                      ibm_args(c));
   EIF_HIP(hipGetLastError());
   return EIF_OK;
@@ -2106,7 +2370,7 @@ int launch_exchange_inertia0(Ctx *c, const double *us_x, const double *us_y) {
   IbmArgs a = ibm_args(c);
   a.us_x = us_x;
   a.us_y = us_y;
-  go<ExchangeB>(k_exchange, dim3(c->nslices), dim3(64), 0, c->stream, a, 0);
+  go<ExchangeB>(k_exchange, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a, 0);
   EIF_HIP(hipGetLastError());
   return EIF_OK;
 }
@@ -2126,6 +2390,7 @@ static TileArgs tile_args(Ctx *c, int apply) {
   t.nx = c->nx;
   t.ny = c->ny;
   t.ntx = c->ntx;
+  t.ntiles = c->ntx * c->nty;
   t.boxes = c->boxes;
   t.sc_fx = c->sc_fx;
   t.sc_fy = c->sc_fy;
@@ -2140,16 +2405,13 @@ static TileArgs tile_args(Ctx *c, int apply) {
   return t;
 }
 
-static int tile_grid(Ctx *c) {
-  const long ntiles = (long)c->ntx * c->nty;
-  return (int)ntiles;  // one workgroup per tile; idle tiles return at once
-}
+static long tile_count(const Ctx *c) { return (long)c->ntx * c->nty; }
 
 int launch_update_momentum(Ctx *c) {
   if (c->np == 0) return EIF_OK;
   ProfScope ps(c, "ibm_apply");
   TileArgs t = tile_args(c, 1);
-  go<TilesB>(k_tiles, dim3(tile_grid(c)), dim3(TILE_THREADS), 0, c->stream, t);
+  go<TilesB>(k_tiles, wave_grid(tile_count(c)), dim3(TILE_THREADS), 0, c->stream, t);
   EIF_HIP(hipGetLastError());
   return EIF_OK;
 }
@@ -2159,7 +2421,7 @@ int launch_update_momentum_x0(Ctx *c) {
   if (c->np == 0) return EIF_OK;
   ProfScope ps(c, "ibm_apply");
   TileArgs t = tile_args(c, 1);
-  go<TilesX0B>(k_tiles_x0, dim3(c->np + tile_grid(c)), dim3(TILE_THREADS), 0, c->stream,
+  go<TilesX0B>(k_tiles_x0, wave_grid(c->np + tile_count(c)), dim3(TILE_THREADS), 0, c->stream,
                      t, ibm_args(c));
   EIF_HIP(hipGetLastError());
   return EIF_OK;
@@ -2171,7 +2433,7 @@ int launch_materialise_du(Ctx *c) {
   EIF_HIP(hipMemsetAsync(c->duy, 0, bytes, c->stream));
   if (c->np > 0) {
     TileArgs t = tile_args(c, 0);
-    go<TilesB>(k_tiles, dim3(tile_grid(c)), dim3(TILE_THREADS), 0, c->stream,
+    go<TilesB>(k_tiles, wave_grid(tile_count(c)), dim3(TILE_THREADS), 0, c->stream,
                        t);
     EIF_HIP(hipGetLastError());
   }
@@ -2281,7 +2543,7 @@ int launch_collision(Ctx *c, int cnstep, hipStream_t st) {
   const CollArgs a = coll_args(c, cnstep);
   go<CollPackB>(k_coll_pack, dim3((c->np + 255) / 256), dim3(256), 0, st, a);
   launch_cell_list(c, a, st);
-  go<CollideB>(k_collide, dim3(c->np), dim3(64), 0, st, a);
+  go<CollideB>(k_collide, wave_grid(c->np), dim3(64 * WG_WAVES), 0, st, a);
   EIF_HIP(hipGetLastError());
   return EIF_OK;
 }
@@ -2296,7 +2558,7 @@ int launch_substep_forces(Ctx *c, int sub) {
     // after the reset): collision(1) would repeat collision(0) operand for
     // operand, so the increment copies collision(0)'s forces instead
     ProfScope ps(c, "ibm_inertia");
-    go<InertiaB>(k_inertia, dim3(c->nslices), dim3(64), 0, c->stream, a, 1);
+    go<InertiaB>(k_inertia, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a, 1);
     EIF_HIP(hipGetLastError());
     return EIF_OK;
   }
@@ -2306,10 +2568,10 @@ int launch_substep_forces(Ctx *c, int sub) {
   launch_cell_list(c, ca, c->stream);
   hipEvent_t e0, e1;
   if (prof_kernel_events(c, "ibm_substep", &e0, &e1))  // a sampled launch stamps its events
-    hipExtLaunchKernelGGL(k_inertia_collide, dim3(c->np + c->nslices), dim3(64), 0, c->stream,
+    hipExtLaunchKernelGGL(k_inertia_collide, wave_grid(c->np + c->nslices), dim3(64 * WG_WAVES), 0, c->stream,
                           e0, e1, 0, a, ca, 1);
   else
-    go<InertiaCollideB>(k_inertia_collide, dim3(c->np + c->nslices), dim3(64), 0, c->stream, a,
+    go<InertiaCollideB>(k_inertia_collide, wave_grid(c->np + c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a,
                        ca, 1);
   EIF_HIP(hipGetLastError());
   return EIF_OK;
@@ -2325,8 +2587,9 @@ int launch_increment(Ctx *c, int rk, int sub) {
     ia.sub = sub;
     res_out = c->res_slots + sub;
   }
+  const int waves = c->np >= INC_WIDE ? 16 : 4;
   if (c->np > 0)
-    go<IncrementB>(k_increment, dim3((c->np + 3) / 4), dim3(256), 0, c->stream,
+    go<IncrementB>(k_increment, dim3((c->np + waves - 1) / waves), dim3(64 * waves), 0, c->stream,
                        c->prt, c->np, c->dscal, c->gamma[rk], c->cfg.Fr, res_out, ia,
                        sub >= 0 ? 1 : 0);
   EIF_HIP(hipGetLastError());

@@ -52,3 +52,63 @@ def test_thomas_sweep_bit_exact_at_tile_edges(nx, ny, ly):
 def test_transform_of_any_length_bit_exact(nx):
     a, b = potential(nx, 6, 0.5)
     assert np.array_equal(a, b)
+
+
+# bodies whose cells meet the foot search's special places: circles centred on
+# a cell centre (every direction is a foot), thin ellipses (the evolute comes
+# within a cell of the tip), tall ones, one across the periodic boundary, and
+# a body smaller than a cell's diagonal; the sums of the weights' passes agree
+# to the rounding of some 1e4 terms (1e-13 of the largest member)
+@pytest.mark.parametrize("a,b,az", [(0.125, 0.125, 0.0), (0.2, 0.02, 0.0), (0.2, 0.02, 0.7),
+                                    (0.02, 0.2, 1.1), (0.15, 0.149, 2.0), (0.012, 0.01, 0.3)])
+def test_weights_of_special_shapes(a, b, az):
+    nx = ny = 64
+    kw = dict(itot=nx, jtot=ny, ly=1.0, Re=100.0)
+    g, o = eif.Solver(**kw), Oracle(**kw)
+    ux, uy, p = cases.random_fields(nx, ny, 5)
+    parts = dict(den=[1.0, 1.2], a=[a, a], b=[b, b], x=[32.5 / nx, 0.37], y=[32.5 / ny, 0.99],
+                 az=[az, az], ux=[0.3, -0.2], uy=[0.1, 0.4], vz=[0.5, -0.3])
+    for s in (g, o):
+        s.upload(ux, uy, p)
+        s.update_boundaries()
+        s.set_dt(1e-3)
+        s.set_particles(**parts)
+        s.reset_particle_increments()
+        s.compute_inertia(0)
+        s.exchange_momentum()
+        # the warm starts, near and far: a small and a large increment
+        rec = s.particles()
+        rec[:, 6:9] = 1e-9
+        s.set_particle_records(rec)
+        s.compute_inertia(1)
+        rec = s.particles()
+        rec[:, 6:9] = [0.004, -0.003, 0.01]
+        s.set_particle_records(rec)
+        s.compute_inertia(1)
+    x, y = g.particles(), o.particles()
+    for cols in ((18, 19), (20, 21), (22, 23), (15, 16), (17,)):
+        c = list(cols)
+        assert np.max(np.abs(x[:, c] - y[:, c])) <= 1e-13 * max(np.max(np.abs(y[:, c])), 1.0), cols
+    g.close()
+
+
+# particle counts on either side of the wide workgroups of the increment, and
+# partial workgroups
+@pytest.mark.parametrize("n", [1, 5, 2047, 2048, 2065])
+def test_increment_bit_exact_at_its_workgroup_sizes(n):
+    kw = dict(itot=32, jtot=64, ly=2.0, Re=100.0, Fr=2.0)
+    g, o = eif.Solver(**kw), Oracle(**kw)
+    rng = np.random.default_rng(n)
+    parts = dict(den=rng.uniform(1, 2, n), a=np.full(n, 0.003), b=np.full(n, 0.002),
+                 x=rng.uniform(0.1, 0.9, n), y=rng.uniform(0, 2, n), az=rng.uniform(0, 3, n))
+    for s in (g, o):
+        s.set_dt(1e-2)
+        s.set_particles(**parts)
+        rec = s.particles()
+        rec[:, 9:30] = np.random.default_rng(7).standard_normal((n, 21))
+        s.set_particle_records(rec)
+        res = s.increment_particles(1)
+        s.res = res
+    assert g.res == o.res
+    assert np.array_equal(g.particles(), o.particles())
+    g.close()
