@@ -1628,8 +1628,7 @@ int eif_gpu_step_fixed_dt(eif_ctx *c, double dt, int record) {
   // integrate() itself at the given dt; recorded: with the stage records
   // copied as it goes (rec_*)
   c->hscal[S_DT] = dt;
-  EIF_HIP(hipMemcpyAsync(c->dscal + S_DT, c->hscal + S_DT, sizeof(double),
-                         hipMemcpyHostToDevice, c->stream));
+  TRY(launch_set_dt(c, dt));
   c->recording = record != 0;
   const int rc = integrate_from(c, 0, 0, nullptr);
   c->recording = false;

@@ -794,6 +794,16 @@ __global__ void k_dt_final(const double *dred, const double *part, const double 
   DtFinalB::run(VB::here(), dred, part, prt, np, sf0, sf2, dt_dif_x, dt_dif_y, delta, dscal, nparts, halt);
 }
 
+// dt given by the host, through the launch's arguments (a copy from the
+// context's pinned scalars could be overtaken by the next call's value)
+__global__ void k_set_dt(double *dscal, double dt) { dscal[S_DT] = dt; }
+
+int launch_set_dt(Ctx *c, double dt) {
+  hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, c->stream, c->dscal, dt);
+  EIF_HIP(hipGetLastError());
+  return EIF_OK;
+}
+
 int launch_decide_dt(Ctx *c) {
   ProfScope ps(c, "decide_dt");
   const int nparts = c->dt_adv_valid ? c->dt_adv_parts : 0;

@@ -281,6 +281,7 @@ int launch_predictor_probe(Ctx *c);
 // choice); returns EIF_ERR_ARG when L does not split jtot within the limits
 int partition_setup(Ctx *c, int L);
 int launch_decide_dt(Ctx *c);
+int launch_set_dt(Ctx *c, double dt);
 int launch_diagnostics(Ctx *c, int which, double *out);
 int launch_wall_shear(Ctx *c, double *out);
 // the same sums into caller device memory, partials in the static scratch

@@ -217,12 +217,13 @@ __device__ inline double rhs_value(const Layout &L, const double *ux, const doub
 
 // the right-hand side with an additive cell field (the adjoint projection's
 // pressure cotangent): fac * (div u + fac * add(i, j)); add == null is the
-// forward right-hand side, operation for operation
-template <bool P2 = false>
+// forward right-hand side, operation for operation (NONNULL: it is not, and
+// no test keeps the loads apart)
+template <bool P2 = false, bool NONNULL = false>
 __device__ inline double rhs_value_add(const Layout &L, const double *ux, const double *uy,
                                        const double *add, double fac, double dx, double dy,
                                        int i, int j) {
-  if (!add) return rhs_value<P2>(L, ux, uy, fac, dx, dy, i, j);
+  if (!NONNULL && !add) return rhs_value<P2>(L, ux, uy, fac, dx, dy, i, j);
   const double div = qdiv<P2>(ux[L.ux(i + 2, j)] - ux[L.ux(i + 1, j)], dx, 1. / dx)
                      + qdiv<P2>(uy[L.p(i + 1, j + 1)] - uy[L.p(i + 1, j)], dy, 1. / dy);
   return fac * (div + fac * add[L.p(i + 1, j)]);
@@ -740,9 +741,9 @@ struct RhsDct2TB {
     const int i = threadIdx.x + s * T;
     const int m = (i & 1) ? nx - 1 - (i >> 1) : i >> 1;
     const int q = sw(bitrev(m, LOGN));
-    const double vb = ADD ? rhs_value_add<P2>(L, ux, uy, add, fac, dx, dy, i, jbl)
+    const double vb = ADD ? rhs_value_add<P2, true>(L, ux, uy, add, fac, dx, dy, i, jbl)
                           : rhs_value<P2>(L, ux, uy, fac, dx, dy, i, jbl);
-    re[q] = ADD ? rhs_value_add<P2>(L, ux, uy, add, fac, dx, dy, i, ja)
+    re[q] = ADD ? rhs_value_add<P2, true>(L, ux, uy, add, fac, dx, dy, i, ja)
                 : rhs_value<P2>(L, ux, uy, fac, dx, dy, i, ja);
     im[q] = hasb ? vb : 0.;
   }

@@ -112,3 +112,68 @@ def test_increment_bit_exact_at_its_workgroup_sizes(n):
     assert g.res == o.res
     assert np.array_equal(g.particles(), o.particles())
     g.close()
+
+
+def objective(s, dts):
+    """mean over the steps of the wall shear and the drag of the last exchange"""
+    j = 0.0
+    for dt in dts:
+        s.step_fixed_dt(dt)
+        rec = s.particles()
+        j += s.wall_shear() - float(np.sum(rec[:, 0] * np.pi * rec[:, 1] * rec[:, 2] * rec[:, 16]))
+    return j / len(dts)
+
+
+# the gathered transposed stencils and the reversed weights on grids whose
+# rows, columns and spacings are of every kind (two columns, odd, more columns
+# than a workgroup), against central differences along a random direction of
+# the velocity and of the particles: h = 1e-6 leaves h^2 J''' and round-off of
+# about 1e-16 J / h = 1e-10 J, held here to 1e-7 of the derivative's scale
+@pytest.mark.parametrize("nx,ny,ly", [(16, 12, 0.8), (33, 20, 1.0), (64, 31, 0.5), (270, 16, 0.06)])
+def test_adjoint_along_a_direction(nx, ny, ly):
+    kw = dict(itot=nx, jtot=ny, ly=ly, Re=40.0, extfrcy=0.2)
+    rng = np.random.default_rng(nx)
+    r = min(0.2 * ly, 0.15)
+    parts = dict(den=[1.3], a=[r], b=[0.7 * r], x=[0.45], y=[0.02 * ly], az=[0.4], ux=[0.1],
+                 uy=[-0.2], vz=[0.3])
+    ux, uy, p = cases.random_fields(nx, ny, 11, amp=0.3)
+    p[:] = 0.0
+    dts = [2e-4, 2.5e-4]
+    dux, duy = np.zeros_like(ux), np.zeros_like(uy)
+    dux[1:-1, 1:-1] = rng.standard_normal((ny, nx - 1))
+    duy[1:-1, 1:-1] = rng.standard_normal((ny, nx))
+    dvel = rng.standard_normal(3)
+
+    def solver(h):
+        s = eif.Solver(**kw)
+        s.upload(ux + h * dux, uy + h * duy, p)
+        s.update_boundaries()
+        q = {k: np.array(v, dtype=float) for k, v in parts.items()}
+        for k, d in zip(("ux", "uy", "vz"), dvel):
+            q[k] = q[k] + h * d
+        s.set_particles(**q)
+        return s
+
+    h = 1e-6
+    fd = (objective(solver(h), dts) - objective(solver(-h), dts)) / (2 * h)
+    s = solver(0.0)
+    s.tape_begin()
+    for dt in dts:
+        s.step_fixed_dt(dt, record=True)
+    rec, w = s.particles(), 1.0 / len(dts)
+    seed = np.zeros((1, 3))
+    seed[:, 1] = -rec[:, 0] * np.pi * rec[:, 1] * rec[:, 2] * w
+    for _ in dts:
+        s.adjoint_add_wall_shear(w)
+        s.adjoint_add(s.ADJ_FORCE, seed)
+        for _ in range(3):
+            s.stage_adjoint()
+    terms = [s.adjoint_get(s.ADJ_UX) * dux, s.adjoint_get(s.ADJ_UY) * duy,
+             s.adjoint_get(s.ADJ_PARTICLES)[0, 3:] * dvel]
+    got = sum(float(t.sum()) for t in terms)
+    scale = sum(float(np.abs(t).sum()) for t in terms)
+    assert abs(got - fd) <= 1e-7 * scale, (got, fd, scale)
+    halo = s.adjoint_get(s.ADJ_UX)
+    assert not halo[0].any() and not halo[-1].any() and not halo[:, 0].any() and not halo[:, -1].any()
+    halo = s.adjoint_get(s.ADJ_UY)
+    assert not halo[0].any() and not halo[-1].any() and not halo[:, 0].any() and not halo[:, -1].any()
