@@ -197,6 +197,7 @@ struct Ctx {
   double *slice_part0 = nullptr;  // inertia(0) sums of the fused exchange
   void *heads = nullptr;          // np per-particle pass headers (SliceHead)
   int nslices = 0;
+  int slice_len = 256;  // box cells per slice
   int *tile_cnt = nullptr, *tile_list = nullptr;
   int ntx = 0, nty = 0;
   int *flags = nullptr;    // device error flags

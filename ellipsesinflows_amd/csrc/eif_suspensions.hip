@@ -12,9 +12,9 @@
 //   increments / update   src/suspensions/increment.c:10-72, update.c:8-34
 //
 // Work decomposition (gfx950):
-//   * one wave per slice of 256 cells of a particle's boxes for the IBM
+//   * one wave per slice of 64 to 256 cells of a particle's boxes for the IBM
 //     integrals (its three periodic images' boxes flattened), the slices' sums
-//     added per particle in slice order;
+//     added per particle in a fixed tree;
 //   * the signed distance of every box cell is cached per particle with the
 //     position it belongs to; the reference evaluates it three times at
 //     identical positions in every RK stage (inertia(0), exchange and the
@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <type_traits>
 
 namespace eif {
 
@@ -281,7 +282,15 @@ __device__ inline double p_moi(const double *q) {
 // IBM integrals
 // ---------------------------------------------------------------------
 constexpr int IBM_THREADS = 256;
-constexpr int IBM_SLICE = 256;  // box cells per wave in the inertia / exchange kernels
+// Box cells per wave of the inertia / exchange kernels (a.slice): 256, or 128
+// or 64 where longer slices leave fewer than IBM_WAVES waves.  A wave takes
+// its cells four, two or one a lane in turn, so a launch too small to fill
+// the GPU is as long as that turn: with 64 cells k_inertia_collide took 10.0
+// -> 7.0 us and k_ibm_dist 10.2 -> 6.1 at 64 ellipses on 512x1024 (2600
+// waves), 8.5 -> 5.1 and 10.7 -> 5.2 at one on 128x128; at 11600 waves (1024
+// ellipses on 2048x4096) shorter slices only repeat the waves' prologue.
+constexpr int IBM_SLICE = 256;
+constexpr int IBM_WAVES = 2048;
 constexpr int SLICE_VALS = 5;   // per-slice partials: 3 sums, FP64 and FP32 iterations
 
 // Sub-iteration `sub` of a stage's speculatively queued Crank-Nicolson
@@ -338,7 +347,7 @@ struct IbmArgs {
   unsigned long long *stats;  // per particle: cells, cells evaluated, FP64 and FP32 iterations
   double *cpos;               // np x 4: the broad phase's packed positions and radii
   int np;
-  int nslices;
+  int nslices, slice;      // slices, and box cells of each
   const int *slice_first;  // np+1: first slice of each particle
   const int4 *slice_rec;   // of each slice: its particle, the particle's first slice and slices
   long *slice_info;        // np x 2: box cells, cells evaluated (this call)
@@ -384,8 +393,8 @@ __device__ inline double lane_value(double x, int l) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// A slice's partial sums (lane 0); k_ibm_finalize adds them per particle in
-// slice order after the kernel has finished, so no fence or atomic is needed.
+// A slice's partial sums (lane 0); slice_sums adds them per particle after
+// the kernel has finished, so no fence or atomic is needed.
 __device__ inline void slice_store(const IbmArgs &a, int slice, const double v[SLICE_VALS]) {
   if (wave_lane() == 0)
     for (int k = 0; k < SLICE_VALS; k++) a.slice_part[SLICE_VALS * (long)slice + k] = v[k];
@@ -593,6 +602,7 @@ __global__ __launch_bounds__(256) void k_heads(IbmArgs a, int with_dx) {
 // slice of a particle to finish adds the slices' sums in slice order.
 // open: the sub-iteration gate, evaluated by the caller; tested after this
 // slice's own loads are issued, so the gate's load is not waited for alone
+template <int U>
 __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int slice,
                                               bool open = true) {
   const int lane = wave_lane();
@@ -602,7 +612,7 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
   const BoxSet bs = hd.bs;
   const int total = bs.total;
   if (!open) return;
-  if (total > hd.cap || total > nsl * IBM_SLICE) {
+  if (total > hd.cap || total > nsl * (64 * U)) {
     if (lane == 0) atomicOr(&a.flags[0], 1);
     return;
   }
@@ -617,12 +627,11 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
   const double dxdy = a.dx * a.dy;
   double acc[3] = {0., 0., 0.};  // iux, iuy, ivz
   int it64 = 0, it32 = 0;
-  const int t0 = (slice - s0) * IBM_SLICE;
-  const int t1 = t0 + IBM_SLICE < total ? t0 + IBM_SLICE : total;
+  const int t0 = (slice - s0) * (64 * U);
+  const int t1 = t0 + 64 * U < total ? t0 + 64 * U : total;
   // all loads of the lane's cells first (a cell past t1 loads the last cell
   // instead and is not added), then the weights and the sums in cell order
   if (t0 < t1) {
-    constexpr int U = IBM_SLICE / 64;
     double th_[U], x_[U], y_[U], vx0[U], vx1[U], vy0[U], vy1[U];
     float tp[U];
     int k_[U], i_[U], j_[U];
@@ -677,38 +686,31 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
   }
 }
 
+// U: cells a lane, slices of 64 U
+template <int U>
 struct InertiaB {
   static constexpr int T = 64 * WG_WAVES, M = 4;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, int cnstep) {
   if (halted(a.halt)) return;
   const int slice = wave_index(vb);
-  if (slice < a.nslices) inertia_slice(a, cnstep, slice, sub_open(a.res, a.sub));
+  if (slice < a.nslices) inertia_slice<U>(a, cnstep, slice, sub_open(a.res, a.sub));
 }
 };
+template <int U>
 __global__ __launch_bounds__(64 * WG_WAVES, 4) void k_inertia(IbmArgs a, int cnstep) {
-  InertiaB::run(VB::here(), a, cnstep);
+  InertiaB<U>::run(VB::here(), a, cnstep);
 }
 
 // Per-particle totals of the sliced inertia / exchange kernels, by the 64
-// lanes of one wave: the lanes load the slices' partial sums together, and
-// they are added in slice order through lane shuffles.  Lane 0 also
-// records the position whose distances are now cached and the work
-// counters.  which: 0..1 inertia (cnstep), 2 exchange.
-// the particle's slice sums in slice order (every lane gets them)
+// lanes of one wave: lane l adds slices l, l + 64, ... and the lanes' sums are
+// added in a fixed tree (every lane gets them).  In slice order through
+// readlane, three instructions a slice and value one behind the other, 41
+// slices took 3.5 us of the increment.
 __device__ inline void slice_sums(const IbmArgs &a, int s0, int s1, double tot[SLICE_VALS]) {
-  const int lane = threadIdx.x & 63;
-  for (int k = 0; k < SLICE_VALS; k++) tot[k] = 0.;
-  for (int base = s0; base < s1; base += 64) {
-    double v[SLICE_VALS] = {0., 0., 0., 0., 0.};
-    if (base + lane < s1)
-      for (int k = 0; k < SLICE_VALS; k++)
-        v[k] = a.slice_part[SLICE_VALS * (long)(base + lane) + k];
-    const int cnt = min(64, s1 - base);
-    // the slice index is the same on every lane: lane l's values are read
-    // as scalars (no LDS round trip), added in the same order
-    for (int l = 0; l < cnt; l++)
-      for (int k = 0; k < SLICE_VALS; k++) tot[k] += lane_value(v[k], l);
-  }
+  double v[SLICE_VALS] = {0., 0., 0., 0., 0.};
+  for (int s = s0 + wave_lane(); s < s1; s += 64)
+    for (int k = 0; k < SLICE_VALS; k++) v[k] += a.slice_part[SLICE_VALS * (long)s + k];
+  for (int k = 0; k < SLICE_VALS; k++) tot[k] = lane_value(wave_sum(v[k]), 0);
 }
 
 // The cache records of the pass with header h and the work counters, by the
@@ -878,7 +880,7 @@ struct IbmDistB {
   const SliceHead &hd = a.heads[n];
   const BoxSet bs = hd.bs;
   const int total = bs.total;
-  if (total > hd.cap || total > nsl * IBM_SLICE) {
+  if (total > hd.cap || total > nsl * a.slice) {
     if (lane == 0) atomicOr(&a.flags[0], 1);
     return;
   }
@@ -892,8 +894,8 @@ struct IbmDistB {
     double *dist = a.sc_dist + hd.off;
     float *tcell = a.sc_t + hd.off;
     const double cr = hd.cr, sr = hd.sr;
-    const int t0 = (slice - s0) * IBM_SLICE;
-    const int t1 = t0 + IBM_SLICE < total ? t0 + IBM_SLICE : total;
+    const int t0 = (slice - s0) * a.slice;
+    const int t1 = t0 + a.slice < total ? t0 + a.slice : total;
     for (int t = t0 + lane; t < t1; t += 64) {
       int k, i, j;
       cell_of(bs, t, k, i, j, single);
@@ -923,6 +925,7 @@ __global__ __launch_bounds__(64 * WG_WAVES) void k_ibm_dist(IbmArgs a) {
 // own_counts: no k_ibm_dist ran before, so this kernel reports no
 // distance work.
 // The heads hold the particles' positions without increments.
+template <int U>
 struct ExchangeB {
   static constexpr int T = 64 * WG_WAVES, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, int own_counts) {
@@ -940,7 +943,7 @@ struct ExchangeB {
   const double pux = q[R_UX], puy = q[R_UY], pvz = q[R_VZ];
   const BoxSet bs = hd.bs;
   const int total = bs.total;
-  if (total > hd.cap || total > nsl * IBM_SLICE) {
+  if (total > hd.cap || total > nsl * (64 * U)) {
     if (lane == 0) atomicOr(&a.flags[0], 1);
     return;
   }
@@ -998,12 +1001,11 @@ struct ExchangeB {
   const double dxdy = a.dx * a.dy;
   double acc[3] = {0., 0., 0.};  // fux, fuy, tvz
   double ai[3] = {0., 0., 0.};   // inertia(0): iux, iuy, ivz
-  const int t0 = (slice - s0) * IBM_SLICE;
-  const int t1 = t0 + IBM_SLICE < total ? t0 + IBM_SLICE : total;
+  const int t0 = (slice - s0) * (64 * U);
+  const int t1 = t0 + 64 * U < total ? t0 + 64 * U : total;
   // all loads of the lane's cells first (a cell past t1 loads the last cell
   // instead and is skipped), then the forcing and the sums in cell order
   if (t0 < t1) {
-    constexpr int U = IBM_SLICE / 64;
     double th_[U], x_[U], y_[U], fx0[U], fx1[U], fy0[U], fy1[U], sx0[U], sx1[U], sy0[U],
         sy1[U];
     int k_[U], i_[U], j_[U];
@@ -1084,8 +1086,9 @@ struct ExchangeB {
   }
 }
 };
+template <int U>
 __global__ __launch_bounds__(64 * WG_WAVES) void k_exchange(IbmArgs a, int own_counts) {
-  ExchangeB::run(VB::here(), a, own_counts);
+  ExchangeB<U>::run(VB::here(), a, own_counts);
 }
 
 // ---------------------------------------------------------------------
@@ -1727,6 +1730,7 @@ __global__ __launch_bounds__(256) void k_cell_place(CollArgs a) {
 // slices.  Bounded to 4 waves per SIMD (128 VGPRs): the collision path
 // alone needs more and spills a little, which costs less than the
 // occupancy its registers would take from the slices.
+template <int U>
 struct InertiaCollideB {
   static constexpr int T = 64 * WG_WAVES, M = 4;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, CollArgs ca, int cnstep) {
@@ -1736,12 +1740,14 @@ struct InertiaCollideB {
   if (k < ca.np) {
     if (open) collide_particle(ca, k);
   } else if (k - ca.np < a.nslices) {
-    inertia_slice(a, cnstep, k - ca.np, open);
+    inertia_slice<U>(a, cnstep, k - ca.np, open);
   }
 }
 };
-__global__ __launch_bounds__(64 * WG_WAVES, 4) void k_inertia_collide(IbmArgs a, CollArgs ca, int cnstep) {
-  InertiaCollideB::run(VB::here(), a, ca, cnstep);
+template <int U>
+__global__ __launch_bounds__(64 * WG_WAVES, 4) void k_inertia_collide(IbmArgs a, CollArgs ca,
+                                                                      int cnstep) {
+  InertiaCollideB<U>::run(VB::here(), a, ca, cnstep);
 }
 
 struct ZeroIntB {
@@ -2023,6 +2029,7 @@ static IbmArgs ibm_args(Ctx *c) {
   a.cpos = c->cpos;
   a.np = c->np;
   a.nslices = c->nslices;
+  a.slice = c->slice_len;
   a.slice_first = c->slice_first;
   a.slice_rec = c->slice_rec;
   a.slice_info = c->slice_info;
@@ -2039,6 +2046,29 @@ static IbmArgs ibm_args(Ctx *c) {
 // workgroups of n waves
 static dim3 wave_grid(long n) { return dim3((unsigned)((n + WG_WAVES - 1) / WG_WAVES)); }
 
+// f(cells a lane) for the context's slices
+template <class F>
+static void by_slice(const Ctx *c, F f) {
+  switch (c->slice_len) {
+    case 64: f(std::integral_constant<int, 1>{}); break;
+    case 128: f(std::integral_constant<int, 2>{}); break;
+    default: f(std::integral_constant<int, IBM_SLICE / 64>{}); break;
+  }
+}
+static void go_inertia(Ctx *c, const IbmArgs &a, int cnstep, hipStream_t st) {
+  by_slice(c, [&](auto u) {
+    constexpr int U = decltype(u)::value;
+    go<InertiaB<U>>(k_inertia<U>, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, st, a, cnstep);
+  });
+}
+static void go_exchange(Ctx *c, const IbmArgs &a, int own_counts) {
+  by_slice(c, [&](auto u) {
+    constexpr int U = decltype(u)::value;
+    go<ExchangeB<U>>(k_exchange<U>, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a,
+                     own_counts);
+  });
+}
+
 int launch_ref_iterations(Ctx *c, unsigned long long *dout) {
   if (c->np == 0) return EIF_OK;
   IbmArgs a = ibm_args(c);
@@ -2053,18 +2083,24 @@ int susp_init(Ctx *c) {
   std::vector<double> rec((size_t)c->np * R_N);
   EIF_HIP(hipMemcpy(rec.data(), c->prt, rec.size() * sizeof(double), hipMemcpyDeviceToHost));
   std::vector<long> off(c->np + 1, 0);
-  // slices of IBM_SLICE cells per particle: the boxes of at most two images
+  // slices of slice_len cells per particle: the boxes of at most two images
   // meet the domain when ly > 2r + 8 dy, and two clipped images together
   // are at most two rows taller than one box; otherwise allow three images
   std::vector<int> first(c->np + 1, 0);
+  std::vector<long> box(c->np, 0);
+  long all = 0;
   for (int n = 0; n < c->np; n++) {
     const double r = fmax(rec[(size_t)n * R_N + R_A], rec[(size_t)n * R_N + R_B]);
     const long cx = (long)(2. * r / c->dx) + 10, cy = (long)(2. * r / c->dy) + 10;
     const long wx = cx < c->nx ? cx : c->nx, wy = cy < c->ny ? cy : c->ny;
     off[n + 1] = off[n] + 3 * wx * wy;
-    const long cells = c->ly > 2. * r + 16. * c->dy ? wx * (wy + 4) : 3 * wx * wy;
-    first[n + 1] = first[n] + (int)((cells + IBM_SLICE - 1) / IBM_SLICE);
+    box[n] = c->ly > 2. * r + 16. * c->dy ? wx * (wy + 4) : 3 * wx * wy;
+    all += box[n];
   }
+  c->slice_len = IBM_SLICE;
+  while (c->slice_len > 64 && all / c->slice_len < IBM_WAVES) c->slice_len /= 2;
+  for (int n = 0; n < c->np; n++)
+    first[n + 1] = first[n] + (int)((box[n] + c->slice_len - 1) / c->slice_len);
   c->scratch_cells = off[c->np];
   c->nslices = first[c->np];
   TRY_S(coll_cells_setup(c, rec.data()));
@@ -2135,7 +2171,7 @@ int launch_inertia(Ctx *c, int cnstep, hipStream_t st, bool defer_finalize) {
   ProfScope ps(c, "ibm_inertia", st);
   IbmArgs a = ibm_args(c);
   go<HeadsB>(k_heads, dim3((c->np + 3) / 4), dim3(256), 0, st, a, 1);
-  go<InertiaB>(k_inertia, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, st, a, cnstep);
+  go_inertia(c, a, cnstep, st);
   if (!defer_finalize)
     go<IbmFinalizeB>(k_ibm_finalize, dim3((c->np + 3) / 4), dim3(256), 0, st, a, cnstep);
   EIF_HIP(hipGetLastError());
@@ -2154,8 +2190,7 @@ int launch_exchange(Ctx *c, bool cached_known, bool tiles_clear, bool defer_fina
   go<HeadsB>(k_heads, dim3((c->np + 3) / 4), dim3(256), 0, c->stream, a, 0);
   if (!cached_known)
     go<IbmDistB>(k_ibm_dist, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a);
-  go<ExchangeB>(k_exchange, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a,
-                     cached_known ? 1 : 0);
+  go_exchange(c, a, cached_known ? 1 : 0);
   EIF_HIP(hipGetLastError());
   if (!defer_finalize) return launch_exchange_finalize(c, c->stream);
   return EIF_OK;
@@ -2181,7 +2216,7 @@ int launch_exchange_inertia0(Ctx *c, const double *us_x, const double *us_y) {
   IbmArgs a = ibm_args(c);
   a.us_x = us_x;
   a.us_y = us_y;
-  go<ExchangeB>(k_exchange, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a, 0);
+  go_exchange(c, a, 0);
   EIF_HIP(hipGetLastError());
   return EIF_OK;
 }
@@ -2369,7 +2404,7 @@ int launch_substep_forces(Ctx *c, int sub) {
     // after the reset): collision(1) would repeat collision(0) operand for
     // operand, so the increment copies collision(0)'s forces instead
     ProfScope ps(c, "ibm_inertia");
-    go<InertiaB>(k_inertia, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a, 1);
+    go_inertia(c, a, 1, c->stream);
     EIF_HIP(hipGetLastError());
     return EIF_OK;
   }
@@ -2378,12 +2413,15 @@ int launch_substep_forces(Ctx *c, int sub) {
   ca.sub = sub;
   launch_cell_list(c, ca, c->stream);
   hipEvent_t e0, e1;
-  if (prof_kernel_events(c, "ibm_substep", &e0, &e1))  // a sampled launch stamps its events
-    hipExtLaunchKernelGGL(k_inertia_collide, wave_grid(c->np + c->nslices), dim3(64 * WG_WAVES), 0, c->stream,
-                          e0, e1, 0, a, ca, 1);
-  else
-    go<InertiaCollideB>(k_inertia_collide, wave_grid(c->np + c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a,
-                       ca, 1);
+  const bool timed = prof_kernel_events(c, "ibm_substep", &e0, &e1);
+  by_slice(c, [&](auto u) {
+    constexpr int U = decltype(u)::value;
+    const dim3 grid = wave_grid(c->np + c->nslices), block(64 * WG_WAVES);
+    if (timed)  // a sampled launch stamps its events
+      hipExtLaunchKernelGGL(k_inertia_collide<U>, grid, block, 0, c->stream, e0, e1, 0, a, ca, 1);
+    else
+      go<InertiaCollideB<U>>(k_inertia_collide<U>, grid, block, 0, c->stream, a, ca, 1);
+  });
   EIF_HIP(hipGetLastError());
   return EIF_OK;
 }
