@@ -1448,48 +1448,65 @@ __global__ __launch_bounds__(64 * PART_KG) void k_part_reduced(
 }
 
 // The same reduced system with both chunk DFTs as FP64 matrix products on
-// the matrix cores (v_mfma_f64_16x16x4f64), for P a multiple of 16 up to
-// 64: a workgroup takes 16 wavenumbers and P/16 waves.  Forward: wave w
-// forms the modes m in [16w, 16w+16) of a0 = C r0 - i S r0 and a1 (C, S:
-// cos and sin of 2 pi m c / P); the 2x2 solves run on the accumulators
-// (every lane holds the four values of its (m, k)); inverse: wave w forms
-// the chunks c in [16w, 16w+16) of b = C x_r - S x_i.  Lane layout of the
-// 16x16x4 product: lane l holds A[l%16][l/16], B[l/16][l%16], and
-// D[4i + l/16][l%16] in element i.  The products are summed in another
-// order than the lane loop of k_part_reduced (rounding only).
+// the matrix cores (v_mfma_f64_16x16x4f64): a workgroup takes 16 wavenumbers
+// and Q/16 waves, Q being P rounded up to a multiple of 16 (chunks and modes
+// past P are zero).  Forward: wave w forms the modes m in [16w, 16w+16) of
+// a0 = C r0 - i S r0 and a1 (C, S: cos and sin of 2 pi m c / P); the 2x2
+// solves run on the accumulators (every lane holds the four values of its
+// (m, k)); inverse: wave w forms the chunks c in [16w, 16w+16) of
+// b = C x_r - S x_i.  Lane layout of the 16x16x4 product: lane l holds
+// A[l%16][l/16], B[l/16][l%16], and D[4i + l/16][l%16] in element i.  The
+// products are summed in another order than the lane loop of k_part_reduced
+// (rounding only).  Bound by the latency of its LDS reads and products:
+// twiddle indices advance by additions and the inverse's four products go
+// into separate accumulators (15.1 -> 11.8 us at P = 64, nx = 2048); it serves
+// every P up to PRM_P_MAX (45 us by the lane loop, 24 here at P = 128,
+// nx = 256; 7.0 and 7.8 at P = 24, nx = 768).
 typedef double pr_d4 __attribute__((ext_vector_type(4)));
 constexpr int PRM_K = 16;
+// P up to here: the tables and the four spectra in LDS (150 KiB), 12 waves
+constexpr int PRM_P_MAX = 192;
+static inline int prm_padded(int P) { return (P + 15) / 16 * 16; }
+static inline size_t prm_lds(int P) { return (size_t)(2 + 6 * PRM_K) * prm_padded(P) * sizeof(double); }
 
 struct PartReducedMfmaB {
-  static constexpr int T = 256, M = 0;
+  static constexpr int T = 4 * PRM_P_MAX, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, 
     int nx, int P, const double *__restrict__ ends, const double *__restrict__ lv,
     const double *__restrict__ twc, const double *__restrict__ tws,
     double *__restrict__ bnd) {
   extern __shared__ double sh[];
-  double *tc = sh, *ts = tc + P;
-  double *r0 = ts + P, *r1 = r0 + P * PRM_K;  // [c][kk]
-  double *xs = r1 + P * PRM_K;                 // [4][m][kk]: x0r, x0i, x1r, x1i
+  const int Q = (P + 15) & ~15;
+  double *tc = sh, *ts = tc + Q;
+  double *r0 = ts + Q, *r1 = r0 + Q * PRM_K;  // [c][kk]
+  double *xs = r1 + Q * PRM_K;                 // [4][m][kk]: x0r, x0i, x1r, x1i
   const int k0 = vb.bx * PRM_K;
   for (int e = threadIdx.x; e < P; e += blockDim.x) {
     tc[e] = twc[e];
     ts[e] = tws[e];
   }
-  for (int e = threadIdx.x; e < P * PRM_K; e += blockDim.x) {
+  for (int e = threadIdx.x; e < Q * PRM_K; e += blockDim.x) {
     const int c = e / PRM_K, kk = e - c * PRM_K, k = k0 + kk;
-    const bool on = k < nx;
-    r0[e] = on ? ends[((long)c * 2 + 1) * nx + k] : 0.;             // y_c[L-1]
-    r1[e] = on ? ends[((long)((c + 1) % P) * 2 + 0) * nx + k] : 0.;  // y_{c+1}[0]
+    const bool on = k < nx && c < P;
+    r0[e] = on ? ends[((long)c * 2 + 1) * nx + k] : 0.;                       // y_c[L-1]
+    r1[e] = on ? ends[((long)(c + 1 < P ? c + 1 : 0) * 2 + 0) * nx + k] : 0.;  // y_{c+1}[0]
   }
   __syncthreads();
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int lo = l & 15, hi = l >> 4;
+  // this lane's row (m forward, c inverse) and the steps of its twiddle
+  // index, row * column mod P, as the column goes hi, hi + 4, ...
+  const int row = 16 * w + lo;
+  const int t0 = (row * hi) % P, dt = (4 * row) % P;
   {
     const int m0 = 16 * w;
     pr_d4 a0r = {0., 0., 0., 0.}, a0i = a0r, a1r = a0r, a1i = a0r;
-    for (int c0 = 0; c0 < P; c0 += 4) {
-      const int t = ((m0 + lo) * (c0 + hi)) % P;
+    int t = t0;
+#pragma unroll 4
+    for (int c0 = 0; c0 < Q; c0 += 4) {
       const double cw = tc[t], sw = -ts[t];
+      t += dt;
+      if (t >= P) t -= P;
       const double v0 = r0[(c0 + hi) * PRM_K + lo], v1 = r1[(c0 + hi) * PRM_K + lo];
       a0r = __builtin_amdgcn_mfma_f64_16x16x4f64(cw, v0, a0r, 0, 0, 0);
       a0i = __builtin_amdgcn_mfma_f64_16x16x4f64(sw, v0, a0i, 0, 0, 0);
@@ -1503,28 +1520,32 @@ struct PartReducedMfmaB {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int m = m0 + 4 * i + hi;
-      double x0r, x0i, x1r, x1i;
-      mode_solve(lv0, lvL, gauge && m == 0, tc[m], ts[m], a0r[i], a0i[i], a1r[i], a1i[i], x0r,
-                 x0i, x1r, x1i);
+      double x0r = 0., x0i = 0., x1r = 0., x1i = 0.;
+      if (m < P)
+        mode_solve(lv0, lvL, gauge && m == 0, tc[m], ts[m], a0r[i], a0i[i], a1r[i], a1i[i], x0r,
+                   x0i, x1r, x1i);
       const int e = m * PRM_K + lo;
       xs[e] = x0r;
-      xs[P * PRM_K + e] = x0i;
-      xs[2 * P * PRM_K + e] = x1r;
-      xs[3 * P * PRM_K + e] = x1i;
+      xs[Q * PRM_K + e] = x0i;
+      xs[2 * Q * PRM_K + e] = x1r;
+      xs[3 * Q * PRM_K + e] = x1i;
     }
   }
   __syncthreads();
   {
     const int cb = 16 * w;
-    pr_d4 b0 = {0., 0., 0., 0.}, b1 = b0;
-    for (int m0 = 0; m0 < P; m0 += 4) {
-      const int t = ((cb + lo) * (m0 + hi)) % P;
+    pr_d4 b0 = {0., 0., 0., 0.}, b1 = b0, d0 = b0, d1 = b0;
+    int t = t0;
+#pragma unroll 4
+    for (int m0 = 0; m0 < Q; m0 += 4) {
       const double cw = tc[t], sw = -ts[t];
+      t += dt;
+      if (t >= P) t -= P;
       const int e = (m0 + hi) * PRM_K + lo;
       b0 = __builtin_amdgcn_mfma_f64_16x16x4f64(cw, xs[e], b0, 0, 0, 0);
-      b0 = __builtin_amdgcn_mfma_f64_16x16x4f64(sw, xs[P * PRM_K + e], b0, 0, 0, 0);
-      b1 = __builtin_amdgcn_mfma_f64_16x16x4f64(cw, xs[2 * P * PRM_K + e], b1, 0, 0, 0);
-      b1 = __builtin_amdgcn_mfma_f64_16x16x4f64(sw, xs[3 * P * PRM_K + e], b1, 0, 0, 0);
+      d0 = __builtin_amdgcn_mfma_f64_16x16x4f64(sw, xs[Q * PRM_K + e], d0, 0, 0, 0);
+      b1 = __builtin_amdgcn_mfma_f64_16x16x4f64(cw, xs[2 * Q * PRM_K + e], b1, 0, 0, 0);
+      d1 = __builtin_amdgcn_mfma_f64_16x16x4f64(sw, xs[3 * Q * PRM_K + e], d1, 0, 0, 0);
     }
     const double invP = 1. / P;
     const int k = k0 + lo;
@@ -1533,14 +1554,15 @@ struct PartReducedMfmaB {
       for (int i = 0; i < 4; i++) {
         // u_c = (beta_c, alpha_{c+1}): chunk c+1's left value, chunk c's right
         const int c = cb + 4 * i + hi;
-        bnd[((long)((c + 1) % P) * 2 + 0) * nx + k] = b0[i] * invP;
-        bnd[((long)c * 2 + 1) * nx + k] = b1[i] * invP;
+        if (c >= P) continue;
+        bnd[((long)(c + 1 < P ? c + 1 : 0) * 2 + 0) * nx + k] = (b0[i] + d0[i]) * invP;
+        bnd[((long)c * 2 + 1) * nx + k] = (b1[i] + d1[i]) * invP;
       }
     }
   }
 }
 };
-__global__ __launch_bounds__(256) void k_part_reduced_mfma(
+__global__ __launch_bounds__(4 * PRM_P_MAX) void k_part_reduced_mfma(
     int nx, int P, const double *__restrict__ ends, const double *__restrict__ lv,
     const double *__restrict__ twc, const double *__restrict__ tws,
     double *__restrict__ bnd) {
@@ -1885,10 +1907,10 @@ static int poisson_lines(Ctx *c, int rk, const double *rhs_add, CombineArgs *out
       case 16: go<PartLocalB<16>>(k_part_local<16>, g1, dim3(PART_LANES), 0, c->stream, nx, c->qhat, c->pt_fwd, c->pt_u, l, c->pt_ends); break;
       default: go<PartLocalB<8>>(k_part_local<8>, g1, dim3(PART_LANES), 0, c->stream, nx, c->qhat, c->pt_fwd, c->pt_u, l, c->pt_ends); break;
     }
-    if (P % 16 == 0 && P <= 64)  // the chunk DFTs on the matrix cores
-      go<PartReducedMfmaB>(k_part_reduced_mfma, dim3((nx + PRM_K - 1) / PRM_K), dim3(4 * P),
-                         (size_t)(2 + 6 * PRM_K) * P * sizeof(double), c->stream, nx, P,
-                         c->pt_ends, c->pt_lvl, c->pt_red, c->pt_w, c->pt_bnd);
+    if (P <= PRM_P_MAX)  // the chunk DFTs on the matrix cores
+      go<PartReducedMfmaB>(k_part_reduced_mfma, dim3((nx + PRM_K - 1) / PRM_K),
+                           dim3(4 * prm_padded(P)), prm_lds(P), c->stream, nx, P, c->pt_ends,
+                           c->pt_lvl, c->pt_red, c->pt_w, c->pt_bnd);
     else
       go<PartReducedB>(k_part_reduced, dim3((nx + PART_KG - 1) / PART_KG), dim3(64 * PART_KG),
                          (size_t)(PART_KG * 6 + 2) * P * sizeof(double), c->stream, nx, P,

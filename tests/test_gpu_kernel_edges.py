@@ -229,3 +229,19 @@ def test_diagnostics_at_odd_sizes(nx, ny):
         for a, b in zip(got, ref):
             assert abs(a - b.sum()) <= 1e-13 * np.abs(b).sum()
     s.close()
+
+
+# chunk counts of the partitioned solve: 2, ones that leave the matrix form's
+# padding of 16 nearly empty or nearly full, its largest (192) and the lane
+# loop past it, with a partial block of wavenumbers; psi less its mean against
+# the sweep's within the conditioning of the line, about (jtot / pi)^2 eps
+@pytest.mark.parametrize("nx,ny", [(20, 16), (16, 24), (32, 120), (33, 136), (64, 1024), (20, 1528),
+                                   (16, 1544), (64, 8192)])
+def test_partition_chunk_counts(nx, ny):
+    ly = 4.0
+    a, b = potential(nx, ny, ly, eif.POISSON_PARTITION)
+    assert eif.partition_layout(ny)[1] >= 2
+    a, b = a[1:-1, 1:-1], b[1:-1, 1:-1]
+    a, b = a - a.mean(), b - b.mean()
+    tol = max(1.0, (ny / np.pi) ** 2) * 2.3e-16 * 100
+    assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b)
