@@ -1773,7 +1773,7 @@ int eif_gpu_autotune(eif_ctx *c, int flags, char *report, int report_len) {
     rep += "; fft_values_per_thread:";
     for (int lr : {3, 2, 4}) {
       if (!fft_logr_valid(c, lr)) continue;
-      c->fft_logr = lr == 3 ? 0 : lr;
+      c->fft_logr = lr;
       double ms = 0.;
       if ((rc = time_launches(c, [&] { return launch_poisson(c, 1); }, 10, &ms))) break;
       snprintf(buf, sizeof(buf), " %d=%.4fms", 1 << lr, ms);

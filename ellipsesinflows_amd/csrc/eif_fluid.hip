@@ -123,7 +123,13 @@ int launch_bc_p(Ctx *c, double *p) {
 // registers and more waves per SIMD.
 // ---------------------------------------------------------------------
 constexpr int PRED_BX = 256;
-constexpr int PRED_ROWS = 16;  // default rows per workgroup (the tuner may pick 8 or 32)
+constexpr int PRED_ROWS = 16;  // most rows per workgroup by default (the tuner may pick 8 or 32)
+// Default rows per workgroup: a workgroup's march is a chain of rows, each
+// waiting for its loads, so a grid that does not fill the GPU is as long as
+// the march.  The rows go down to 2 until there are PRED_GROUPS workgroups
+// (two a CU): 16.7 -> 4.8 us at 128x128 (2 rows), 18.4 -> 10.3 at 512x1024 (4),
+// 28.4 -> 23.1 at 768x1536 (8); from 1024x2048 on 16 rows are the fastest.
+constexpr int PRED_GROUPS = 512;
 enum { PRED_STORE = 0, PRED_PREV = 1, PRED_SRC = 2, PRED_NOB = 3 };
 // bit MODE set: that mode loads a row ahead.  The row loop is unrolled
 // over ROWS, so that the compiler's waits on the loads are per row, not
@@ -425,11 +431,22 @@ static void pred_launch_rows(Ctx *c, const PredArgs &a, hipStream_t st) {
     go<PredictorB<false, MODE, ROWS>>(k_predictor<false, MODE, ROWS>, grid, dim3(PRED_BX), 0, st, a);
 }
 
+static int pred_rows(const Ctx *c) {
+  if (c->pred_rows) return c->pred_rows;
+  int rows = PRED_ROWS;
+  while (rows > 2 &&
+         (long)((c->nx + PRED_BX - 1) / PRED_BX) * ((c->ny + rows - 1) / rows) < PRED_GROUPS)
+    rows /= 2;
+  return rows;
+}
+
 // rows per workgroup from the context (tuned, or the default); every
 // choice performs the same operations per cell
 template <int MODE>
 static void pred_launch(Ctx *c, const PredArgs &a, hipStream_t st) {
-  switch (c->pred_rows) {
+  switch (pred_rows(c)) {
+    case 2: pred_launch_rows<MODE, 2>(c, a, st); break;
+    case 4: pred_launch_rows<MODE, 4>(c, a, st); break;
     case 8: pred_launch_rows<MODE, 8>(c, a, st); break;
     case 32: pred_launch_rows<MODE, 32>(c, a, st); break;
     default: pred_launch_rows<MODE, PRED_ROWS>(c, a, st); break;
@@ -524,7 +541,11 @@ int launch_predictor_prev(Ctx *c, int rk, hipStream_t st) {
 // values of ux, uy and p refreshed by the threads that own the source
 // interior values.
 // ---------------------------------------------------------------------
-constexpr int CP_ROWS = 8;   // default rows per workgroup of k_correct_pressure
+// Default rows per workgroup of k_correct_pressure: 4 (a row's loads are in
+// flight together, more rows only follow one another: 82 -> 78 us at
+// 2048x4096, 9.1 -> 7.6 at 512x1024 against 8), 8 where the
+// workgroups' partial dt minima would not fit in DT_PARTS_CAP
+constexpr int CP_ROWS = 4;
 
 template <bool P2, bool DT, int ROWS = CP_ROWS>
 struct CorrectPressureB {
@@ -541,8 +562,10 @@ struct CorrectPressureB {
   const int i = vb.bx * blockDim.x + threadIdx.x + 1;
   const double dt = dscal[S_DT];
   // with DT: the advective time-step limit of decide_dt.c:26-48 over the
-  // corrected velocities, as one partial minimum per workgroup
-  double m = 5.e-2;
+  // corrected velocities, as one partial minimum per workgroup.  A thread's
+  // column has one DXC and dy, and rounded quotients of one numerator fall as
+  // the denominator grows, so the largest |ux| and |uy| give the minimum
+  double vx = 1.e-8, vy = 1.e-8;
   // rows in chunks of up to 4: the chunk's loads first (threads past nx
   // and rows past ny load clamped addresses inside the arrays, and do not
   // use them), then its updates and stores
@@ -577,7 +600,7 @@ struct CorrectPressureB {
           ux[k] = v;
           if (j == ny) ux[L.ux(i, 0)] = v;
           if (j == 1) ux[L.ux(i, ny + 1)] = v;
-          if (DT) m = fmin(m, dxc_i / fmax(fabs(v), 1.e-8));
+          if (DT) vx = fmax(vx, fabs(v));
         }
         {
           const long k = L.p(i, j);
@@ -585,7 +608,7 @@ struct CorrectPressureB {
           uy[k] = v;
           if (j == ny) uy[L.p(i, 0)] = v;
           if (j == 1) uy[L.p(i, ny + 1)] = v;
-          if (DT) m = fmin(m, dy / fmax(fabs(v), 1.e-8));
+          if (DT) vy = fmax(vy, fabs(v));
         }
       }
       if (do_pressure) {
@@ -608,14 +631,15 @@ struct CorrectPressureB {
     }
   }
   if (DT) {
-    __shared__ double red[256];
-    red[threadIdx.x] = m;
+    // the wave's minimum by shuffles, the four waves' through LDS
+    double m = fmin(5.e-2, dy / vy);
+    if (i >= 2 && i <= nx) m = fmin(m, dxc_i / vx);
+    for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_down(m, off, 64));
+    __shared__ double red[4];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-      if ((int)threadIdx.x < s) red[threadIdx.x] = fmin(red[threadIdx.x], red[threadIdx.x + s]);
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) dt_part[vb.by * vb.gx + vb.bx] = red[0];
+    if (threadIdx.x == 0)
+      dt_part[vb.by * vb.gx + vb.bx] = fmin(fmin(red[0], red[1]), fmin(red[2], red[3]));
   }
 }
 };
@@ -659,10 +683,13 @@ static int cp_launch(Ctx *c, int rk, bool correct, bool pressure, bool dt_fused,
 int launch_correct_pressure_on(Ctx *c, int rk, bool correct, bool pressure, bool dt_fused,
                                double *ux, double *uy, double *p) {
   ProfScope ps(c, "correct_pressure");
-  switch (c->cp_rows) {
+  const long cols = (c->nx + 255) / 256;
+  int rows = c->cp_rows;
+  if (!rows) rows = cols * ((c->ny + CP_ROWS - 1) / CP_ROWS) <= DT_PARTS_CAP ? CP_ROWS : 8;
+  switch (rows) {
     case 4: return cp_launch<4>(c, rk, correct, pressure, dt_fused, ux, uy, p);
     case 16: return cp_launch<16>(c, rk, correct, pressure, dt_fused, ux, uy, p);
-    default: return cp_launch<CP_ROWS>(c, rk, correct, pressure, dt_fused, ux, uy, p);
+    default: return cp_launch<8>(c, rk, correct, pressure, dt_fused, ux, uy, p);
   }
 }
 

@@ -1807,8 +1807,11 @@ bool fft_tunable(const Ctx *c) { return dct_mode(c->nx) == 2; }
 bool fft_logr_valid(const Ctx *c, int lr) {
   return fft_tunable(c) && fft_logr_ok(ilog2_exact(c->nx), lr);
 }
+// untuned: 4 values for rows up to 1024 (twice the waves; DCT-II + y-solve +
+// DCT-III 23.8 -> 19.9 us at 256x512, 51.3 -> 50.0 at 1024x2048), 8 beyond
+// (0.144 ms against 0.146 at 2048x4096)
 static int fft_logr(const Ctx *c, int lg) {
-  const int lr = c->fft_logr;
+  const int lr = c->fft_logr ? c->fft_logr : (lg <= 10 ? 2 : FFT_LOGR_DEFAULT);
   return (lr == 2 || lr == 4) && fft_logr_ok(lg, lr) ? lr : FFT_LOGR_DEFAULT;
 }
 

@@ -245,3 +245,30 @@ def test_partition_chunk_counts(nx, ny):
     a, b = a - a.mean(), b - b.mean()
     tol = max(1.0, (ny / np.pi) ** 2) * 2.3e-16 * 100
     assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b)
+
+
+# grids at which the predictor takes 2, 4, 8 and 16 rows a workgroup, with a
+# partial last workgroup and a partial column block: whole stages (the kept
+# previous velocity's form) and the per-function form, with the time step
+@pytest.mark.parametrize("nx,ny", [(40, 27), (260, 1025), (260, 2050), (260, 4097)])
+def test_predictor_rows_bit_exact(nx, ny):
+    kw = dict(itot=nx, jtot=ny, ly=2.0, Re=100.0, extfrcy=0.1, uy_wall_xp=0.3)
+    g, o = eif.Solver(**kw), Oracle(**kw)
+    ux, uy, p = cases.random_fields(nx, ny, nx + ny, amp=0.3)
+    for s in (g, o):
+        s.upload(ux, uy, p)
+        s.update_boundaries()
+    assert g.decide_dt() == o.decide_dt()
+    for s in (g, o):
+        s.integrate()
+    a, b = g.download(), o.download()
+    for k in ("ux", "uy", "p"):
+        assert np.array_equal(a[k], b[k]), k
+    assert g.decide_dt() == o.decide_dt()
+    for s in (g, o):
+        s.update_velocity(0)
+        s.update_velocity(1)
+    a, b = g.download(), o.download()
+    for k in ("ux", "uy"):
+        assert np.array_equal(a[k], b[k]), k
+    g.close()
