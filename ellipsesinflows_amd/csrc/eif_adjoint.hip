@@ -892,16 +892,13 @@ int adjoint_access(Ctx *c, int which, double *host, bool add) {
   }
   const size_t nu = c->L.ux_len(), npl = c->L.p_len(), np = (size_t)c->np;
   auto dev = [&](double *d, size_t n) -> int {
+    if (!add) return download(c, host, d, n * sizeof(double));
     std::vector<double> tmp(n);
     EIF_HIP(hipMemcpyAsync(tmp.data(), d, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     EIF_HIP(hipStreamSynchronize(c->stream));
-    if (add) {
-      for (size_t k = 0; k < n; k++) tmp[k] += host[k];
-      EIF_HIP(hipMemcpyAsync(d, tmp.data(), n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-      EIF_HIP(hipStreamSynchronize(c->stream));
-    } else {
-      memcpy(host, tmp.data(), n * sizeof(double));
-    }
+    for (size_t k = 0; k < n; k++) tmp[k] += host[k];
+    EIF_HIP(hipMemcpyAsync(d, tmp.data(), n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    EIF_HIP(hipStreamSynchronize(c->stream));
     return EIF_OK;
   };
   switch (which) {

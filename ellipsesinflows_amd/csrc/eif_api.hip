@@ -194,6 +194,7 @@ static void free_ctx(Ctx *c) {
                     c->sc_key, c->heads, c->cl_start, c->cl_items, c->cl_cell, c->cl_slot, c->cl_count};
   for (auto o : others)
     if (o) (void)hipFree(o);
+  staging_free(c);
   if (c->hscal) (void)hipHostFree(c->hscal);
   if (c->hstat) (void)hipHostFree(c->hstat);
   if (c->gstat) (void)hipHostFree(c->gstat);
@@ -416,11 +417,9 @@ int fluid_gpu_upload(eif_ctx *c, const double *ux, const double *uy, const doubl
 int fluid_gpu_download(eif_ctx *c, double *ux, double *uy, double *p) {
   CHECK_CTX(c);
   const Layout &L = c->L;
-  if (ux) EIF_HIP(hipMemcpyAsync(ux, c->ux, L.ux_len() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  if (uy) EIF_HIP(hipMemcpyAsync(uy, c->uy, L.p_len() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  if (p) EIF_HIP(hipMemcpyAsync(p, c->p, L.p_len() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  EIF_HIP(hipStreamSynchronize(c->stream));
-  return EIF_OK;
+  const size_t nu = L.ux_len() * sizeof(double), np = L.p_len() * sizeof(double);
+  const Download parts[] = {{ux, c->ux, nu}, {uy, c->uy, np}, {p, c->p, np}};
+  return download(c, parts, 3);
 }
 
 static int field_ptr(eif_ctx *c, int which, double **ptr, size_t *n) {
@@ -447,9 +446,7 @@ int fluid_gpu_download_field(eif_ctx *c, int which, double *host) {
   TRY(field_ptr(c, which, &ptr, &n));
   if (which == EIF_FIELD_DUX || which == EIF_FIELD_DUY) TRY(launch_materialise_du(c));
   if (which == EIF_FIELD_SRCUXA || which == EIF_FIELD_SRCUYA) TRY(launch_materialise_src(c));
-  EIF_HIP(hipMemcpyAsync(host, ptr, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  EIF_HIP(hipStreamSynchronize(c->stream));
-  return EIF_OK;
+  return download(c, host, ptr, n * sizeof(double));
 }
 
 int fluid_gpu_upload_field(eif_ctx *c, int which, const double *host) {
@@ -590,12 +587,9 @@ int statistics_gpu_download(eif_ctx *c, double *ux1, double *ux2, double *uy1,
   CHECK_CTX(c);
   TRY(stat_alloc(c));
   const size_t nu = c->L.ux_len() * sizeof(double), np = c->L.p_len() * sizeof(double);
-  if (ux1) EIF_HIP(hipMemcpyAsync(ux1, c->st_ux1, nu, hipMemcpyDeviceToHost, c->stream));
-  if (ux2) EIF_HIP(hipMemcpyAsync(ux2, c->st_ux2, nu, hipMemcpyDeviceToHost, c->stream));
-  if (uy1) EIF_HIP(hipMemcpyAsync(uy1, c->st_uy1, np, hipMemcpyDeviceToHost, c->stream));
-  if (uy2) EIF_HIP(hipMemcpyAsync(uy2, c->st_uy2, np, hipMemcpyDeviceToHost, c->stream));
-  if (phi) EIF_HIP(hipMemcpyAsync(phi, c->st_phi, np, hipMemcpyDeviceToHost, c->stream));
-  EIF_HIP(hipStreamSynchronize(c->stream));
+  const Download parts[] = {{ux1, c->st_ux1, nu}, {ux2, c->st_ux2, nu}, {uy1, c->st_uy1, np},
+                            {uy2, c->st_uy2, np}, {phi, c->st_phi, np}};
+  TRY(download(c, parts, 5));
   if (num) *num = c->st_num;
   return EIF_OK;
 }
@@ -639,9 +633,7 @@ int suspensions_gpu_n_particles(const eif_ctx *c) { return c ? c->np : 0; }
 int suspensions_gpu_download(eif_ctx *c, double *records) {
   CHECK_CTX(c);
   if (c->np == 0) return EIF_OK;
-  EIF_HIP(hipMemcpyAsync(records, c->prt, (size_t)c->np * R_N * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  EIF_HIP(hipStreamSynchronize(c->stream));
-  return EIF_OK;
+  return download(c, records, c->prt, (size_t)c->np * R_N * sizeof(double));
 }
 
 int suspensions_gpu_upload(eif_ctx *c, const double *records) {

@@ -242,6 +242,7 @@ struct Ctx {
   double *st_uy1 = nullptr, *st_uy2 = nullptr, *st_phi = nullptr;  // like uy
   int st_num = 0;
   Profiler *prof = nullptr;
+  struct Staging *staging = nullptr;  // pinned slots of the downloads
 };
 
 // error state
@@ -253,6 +254,17 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
     hipError_t _e = (call);                                               \
     if (_e != hipSuccess) return ::eif::hip_fail(_e, #call, __FILE__, __LINE__); \
   } while (0)
+
+// device arrays to host memory (eif_download.hip)
+struct Download {
+  void *host;  // null: not wanted
+  const void *dev;
+  size_t bytes;
+};
+constexpr int DOWNLOAD_PARTS = 5;  // at most
+int download(Ctx *c, const Download *parts, int n);
+int download(Ctx *c, void *host, const void *dev, size_t bytes);
+void staging_free(Ctx *c);
 
 // profiling helpers (host)
 // prof_begin: whether this launch is timed (then prof_end closes it)

@@ -3,6 +3,7 @@ the oracle (bit for bit where the kernels perform the reference's operations
 in its order)."""
 import numpy as np
 import pytest
+import torch
 
 import cases
 from oracle import Oracle
@@ -271,4 +272,23 @@ def test_predictor_rows_bit_exact(nx, ny):
     a, b = g.download(), o.download()
     for k in ("ux", "uy"):
         assert np.array_equal(a[k], b[k]), k
+    g.close()
+
+
+# downloads through the staging slots: one slot (up to 2 MiB), a thread's
+# strip of many chunks, several strips, with ragged ends; some fields left
+# out; and into pinned memory, which is copied to directly
+@pytest.mark.parametrize("nx,ny", [(6, 3), (300, 290), (301, 292), (500, 700), (1021, 1531)])
+def test_downloads_return_the_fields(nx, ny):
+    g = eif.Solver(nx, ny, ly=1.0)
+    want = dict(zip(("ux", "uy", "p"), cases.random_fields(nx, ny, nx + ny)))
+    g.upload(*want.values())
+    for k, a in g.download().items():
+        assert np.array_equal(a, want[k].reshape(a.shape)), k
+    uy = np.full(g.shapes["uy"], -1.0)
+    g._check(g.lib.fluid_gpu_download(g.h, None, eif._ptr(uy), None))
+    assert np.array_equal(uy, want["uy"].reshape(uy.shape))
+    p = torch.empty(g.shapes["p"], dtype=torch.float64, pin_memory=True).numpy()
+    g._check(g.lib.fluid_gpu_download(g.h, None, None, eif._ptr(p)))
+    assert np.array_equal(p, want["p"].reshape(p.shape))
     g.close()
