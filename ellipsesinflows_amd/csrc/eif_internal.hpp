@@ -56,6 +56,7 @@ constexpr int TILE_Y = 4;
 constexpr int TILE_CAP = 48;     // boxes registered per tile
 constexpr int CONTACT_CAP = 64;  // colliding partners per particle
 constexpr int COLL_CELLS_MIN = 4096;  // particles from which the cell list is chosen
+constexpr int CELL_BUILD_MAX = 8192;  // particles up to which one workgroup builds the cell list
 constexpr int COLL_CELLS_CAP = 14336; // cells at most: their counts and a scan in 60 KiB of LDS
 constexpr int EQC_ITER_CAP = 100000;  // guard of the uncapped fixed point
 constexpr int DT_PARTS_CAP = 16384;   // workgroups of the projection with fused dt
@@ -241,6 +242,11 @@ struct Ctx {
   double *st_ux1 = nullptr, *st_ux2 = nullptr;                   // like ux
   double *st_uy1 = nullptr, *st_uy2 = nullptr, *st_phi = nullptr;  // like uy
   int st_num = 0;
+  // a single case's step is being captured.  Its collision(0) keeps the launch
+  // that packs the positions (k_reset has packed them): replayed without it,
+  // 64 ellipses on 512x1024 took 10.27 ms instead of 9.91, while an eager
+  // pass (one on 128x128) gains 0.1 of 3.7 ms
+  bool capturing = false;
   Profiler *prof = nullptr;
   struct Staging *staging = nullptr;  // pinned slots of the downloads
 };
@@ -351,7 +357,8 @@ int launch_exchange_inertia0(Ctx *c, const double *us_x, const double *us_y);
 int launch_update_momentum(Ctx *c);
 int launch_update_momentum_x0(Ctx *c);
 int launch_materialise_du(Ctx *c);
-int launch_collision(Ctx *c, int cnstep, hipStream_t st = nullptr);
+// packed: cpos holds the particles' current positions (after k_reset)
+int launch_collision(Ctx *c, int cnstep, hipStream_t st = nullptr, bool packed = false);
 // sub >= 0: sub-iteration `sub` of the stage, gated on the residual slots;
 // it also finalises the preceding launch_substep_forces
 int launch_increment(Ctx *c, int rk, int sub = -1);

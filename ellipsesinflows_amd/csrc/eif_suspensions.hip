@@ -1263,10 +1263,11 @@ struct EllD {
 // fixed-point iteration (or the FP32 estimate when tw < 0); the root on
 // the first-quadrant arc is unique, so the start only changes the number
 // of iterations.  (cm, sm) = cos/sin(-angle), (cp, sp) = cos/sin(+angle).
+// (ct, st): cosine and sine of the foot's parameter (ellipse.c:62-63).
 __device__ void evolute_fit_fast(const EllD &e, const EllipseShape &s,
                                  const EllipseShape32 &f, double cm, double sm, double cp,
                                  double sp, double x, double y, double &ex, double &ey,
-                                 double &ix, double &iy, double &r, double &tw) {
+                                 double &ct, double &st, double &tw) {
   double x_, y_;
   {
     const double x__ = x - e.x, y__ = y - e.y;
@@ -1278,25 +1279,28 @@ __device__ void evolute_fit_fast(const EllD &e, const EllipseShape &s,
   if (tw < 0.) tw = (double)foot_fp32(f, px, py, it32);
   double c, sn;
   foot_fp64(s, px, py, tw, c, sn, it64);
-  // unfolded foot (ellipse.c:62-63)
-  const double ct = x_ < 0. ? -c : c;
-  const double st = y_ < 0. ? -sn : sn;
-  {
-    // compute_curvature, ellipse.c:15-25
-    const double ct2 = ct * ct, st2 = st * st;
-    const double a2 = e.a * e.a, b2 = e.b * e.b;
-    const double num = e.a * e.b * (ct2 + st2);
-    const double den = +a2 * st2 + b2 * ct2;
-    r = 1. / fmax(num / (den * sqrt(den)), DBL_EPSILON);
-  }
+  ct = x_ < 0. ? -c : c;
+  st = y_ < 0. ? -sn : sn;
   x_ = s.kex * cube(ct);
   y_ = s.key * cube(st);
   ex = cp * x_ - sp * y_;
   ey = sp * x_ + cp * y_;
   ex = ex + e.x;
   ey = ey + e.y;
-  x_ = e.a * ct;
-  y_ = e.b * st;
+}
+
+// what compute_evolute returns besides the centre: the radius of curvature
+// at the foot and the foot itself, which only the last fit of the
+// fixed-point iteration has to give
+__device__ inline void evolute_radius(const EllD &e, double cp, double sp, double ct, double st,
+                                      double &ix, double &iy, double &r) {
+  // compute_curvature, ellipse.c:15-25
+  const double ct2 = ct * ct, st2 = st * st;
+  const double a2 = e.a * e.a, b2 = e.b * e.b;
+  const double num = e.a * e.b * (ct2 + st2);
+  const double den = +a2 * st2 + b2 * ct2;
+  r = 1. / fmax(num / (den * sqrt(den)), DBL_EPSILON);
+  const double x_ = e.a * ct, y_ = e.b * st;
   ix = cp * x_ - sp * y_;
   iy = sp * x_ + cp * y_;
 }
@@ -1319,7 +1323,7 @@ struct CollArgs {
   int ncx, ncy;
   double hx, hy;
   int *cl_start, *cl_items, *cl_cell, *cl_slot;
-  double *cpos;  // np x 4: x + dx, y + dy, max(a, b) (written by k_coll_pack and k_increment)
+  double *cpos;  // np x 4: x + dx, y + dy, max(a, b) (written by k_reset, k_increment, k_coll_pack)
 };
 
 __device__ inline double harmonic(double v0, double v1) {
@@ -1339,16 +1343,21 @@ __device__ inline double min_image_offset(double p0y, double p1y, double ly) {
   return yoffset;
 }
 
+// a particle's bounding circle, from the packed cpos (the same values as the
+// records give)
+struct Circle {
+  double x, y, r;
+};
+__device__ inline Circle circle_of(const CollArgs &a, int n) {
+  const double *p = a.cpos + 4 * (long)n;
+  return {p[0], p[1], p[2]};
+}
+
 // The early exit of collision.c:156-189 for the pair n0 < n1: the bounding
 // circles (radius max(a, b)) of the minimum image overlap
-// (the positions x + dx, y + dy and radii max(a, b) from the packed cpos,
-// the same values as the records give)
-__device__ inline bool pair_candidate(const CollArgs &a, int n0, int n1) {
-  const double *p0 = a.cpos + 4 * (long)n0, *p1 = a.cpos + 4 * (long)n1;
-  const double x0 = p0[0], y0 = p0[1];
-  const double x1 = p1[0], y1r = p1[1];
-  const double y1 = y1r + min_image_offset(y0, y1r, a.ly);
-  const double dx = x1 - x0, dy = y1 - y0, r = p0[2] + p1[2];
+__device__ inline bool pair_candidate(const Circle &p0, const Circle &p1, double ly) {
+  const double y1 = p1.y + min_image_offset(p0.y, p1.y, ly);
+  const double dx = p1.x - p0.x, dy = y1 - p0.y, r = p0.r + p1.r;
   // far apart by the squares, with a margin far above their rounding: the
   // exact test would say so too (and NaN goes on to it)
   if (dx * dx + dy * dy > r * r * (1. + 1e-12)) return false;
@@ -1409,12 +1418,12 @@ __device__ bool contact_force(const CollArgs &a, int n0, int n1, int wall, int s
   sincos_angle(e.angle, sp, cp);
   const double cm = cp, sm = -sp;
   double tw = -1.;
-  double cx = e.x, cy = e.y, cr = 0., ix = 0., iy = 0.;
+  double cx = e.x, cy = e.y, ct = 0., st = 0.;
   for (int it = 0;; it++) {
     const double ox = __shfl_xor(cx, 1), oy = __shfl_xor(cy, 1);
     const double tx = wall < 0 ? ox : 2. * wallx - cx, ty = wall < 0 ? oy : cy;
     double nx, ny;
-    evolute_fit_fast(e, sh, f, cm, sm, cp, sp, tx, ty, nx, ny, ix, iy, cr, tw);
+    evolute_fit_fast(e, sh, f, cm, sm, cp, sp, tx, ty, nx, ny, ct, st, tw);
     const double dx = nx - cx, dy = ny - cy;
     cx += dx;
     cy += dy;
@@ -1427,10 +1436,17 @@ __device__ bool contact_force(const CollArgs &a, int n0, int n1, int wall, int s
       break;
     }
   }
+  double ix, iy, cr;
+  evolute_radius(e, cp, sp, ct, st, ix, iy, cr);
   const double ocx = __shfl_xor(cx, 1), ocy = __shfl_xor(cy, 1), ocr = __shfl_xor(cr, 1);
   const double oix = __shfl_xor(ix, 1), oiy = __shfl_xor(iy, 1);
   if (wall >= 0) {  // collision.c:268-304
     const double m = p_mass(p0), im = p_moi(p0);
+    double nxv = wallx - cx;
+    const double norm = fabs(nxv);
+    nxv /= norm;
+    const double overlap = cr - norm;
+    if (!(overlap > 0.)) return false;
     double k;
     {
       const double mass = m;
@@ -1438,11 +1454,6 @@ __device__ bool contact_force(const CollArgs &a, int n0, int n1, int wall, int s
       const double reft = pow(r, 1.5);
       k = mass * (EIF_PI * EIF_PI) / (reft * reft);
     }
-    double nxv = wallx - cx;
-    const double norm = fabs(nxv);
-    nxv /= norm;
-    const double overlap = cr - norm;
-    if (!(overlap > 0.)) return false;
     const double cfx = k * overlap * nxv;
     const double cfy = 0.;
     v[0] = 1. / m * (-cfx);
@@ -1454,6 +1465,12 @@ __device__ bool contact_force(const CollArgs &a, int n0, int n1, int wall, int s
   const double c1x = side ? cx : ocx, c1y = side ? cy : ocy, c1r = side ? cr : ocr;
   const double ix0 = side ? oix : ix, iy0 = side ? oiy : iy;
   const double ix1 = side ? ix : oix, iy1 = side ? iy : oiy;
+  double nxv = c1x - c0x, nyv = c1y - c0y;
+  const double norm = fmax(hypot(nxv, nyv), DBL_EPSILON);
+  nxv /= norm;
+  nyv /= norm;
+  const double overlap = c0r + c1r - norm;
+  if (!(overlap > 0.)) return false;
   const double m0 = p_mass(p0), m1 = p_mass(p1);
   const double i0 = p_moi(p0), i1 = p_moi(p1);
   double k;
@@ -1464,12 +1481,6 @@ __device__ bool contact_force(const CollArgs &a, int n0, int n1, int wall, int s
     const double reft = pow(harmonic(r0, r1), 1.5);
     k = mass * (EIF_PI * EIF_PI) / (reft * reft);
   }
-  double nxv = c1x - c0x, nyv = c1y - c0y;
-  const double norm = fmax(hypot(nxv, nyv), DBL_EPSILON);
-  nxv /= norm;
-  nyv /= norm;
-  const double overlap = c0r + c1r - norm;
-  if (!(overlap > 0.)) return false;
   const double cfx = k * overlap * nxv;
   const double cfy = k * overlap * nyv;
   v[0] = 1. / m0 * (-cfx);
@@ -1487,44 +1498,60 @@ __device__ bool contact_force(const CollArgs &a, int n0, int n1, int wall, int s
 // its particles' waves, with the same operands), and the contributions are
 // added in the order of the reference's loops: partners in ascending
 // index, then wall x = 0, then wall x = lx.
+//
+// The launch is as long as one wave's chain of dependent loads and FP64
+// operations, so loads are taken together (four partners a lane; the nine
+// cells as three runs), the wave goes before others on its SIMD, and what
+// only the last fit or an overlap needs is left to the end: k_inertia_collide 38.2 ->
+// 35.3 us at 4096 ellipses on 1024x2048, 33.0 -> 31.6 at 1024 on 2048x4096.
 constexpr int COLL_CAND_CAP = 256;  // candidate partners per particle
 
-// the candidates of particle n among the particles of cell c (in the cell
-// list's order), appended to s_cand
-__device__ inline void cell_candidates(const CollArgs &a, int n, int c, int *s_cand, int &cnt) {
-  const int lane = wave_lane();
-  const int s0 = a.cl_start[c], s1 = a.cl_start[c + 1];
-  for (int base = s0; base < s1; base += 64) {
-    const int k = base + lane;
-    const int m = k < s1 ? a.cl_items[k] : n;
-    const bool hit = m != n && pair_candidate(a, min(n, m), max(n, m));
-    const unsigned long long b = __ballot(hit);
-    if (hit) {
-      const int pos = cnt + __popcll(b & ((1ull << lane) - 1ull));
-      if (pos < COLL_CAND_CAP) s_cand[pos] = m;
-    }
-    cnt += __popcll(b);
+// the lanes' partners that hit, appended to s_cand
+__device__ inline void add_candidates(int lane, int m, bool hit, int *s_cand, int &cnt) {
+  const unsigned long long b = __ballot(hit);
+  if (hit) {
+    const int pos = cnt + __popcll(b & ((1ull << lane) - 1ull));
+    if (pos < COLL_CAND_CAP) s_cand[pos] = m;
   }
+  cnt += __popcll(b);
+}
+
+// whether particle n (circle me) and m may touch
+__device__ inline bool candidate(const CollArgs &a, int n, const Circle &me, int m,
+                                 const Circle &q) {
+  return m != n && pair_candidate(n < m ? me : q, n < m ? q : me, a.ly);
 }
 
 __device__ void collide_particle(const CollArgs &a, int n) {
   __shared__ int s_cand_[WG_WAVES][COLL_CAND_CAP];
   __shared__ int s_sorted_[WG_WAVES][COLL_CAND_CAP];
   int *s_cand = s_cand_[wave_in_group()], *s_sorted = s_sorted_[wave_in_group()];
+  // a long chain of dependent operations beside waves of short ones
+  __builtin_amdgcn_s_setprio(3);
   const int lane = wave_lane();
   int cnt = 0;
   const int *cand = s_cand;
+  const Circle me = circle_of(a, n);
   if (a.use_cells) {
     // the cell and its neighbours (ncy >= 3: the three rows are distinct);
-    // two particles within reach are in the same or adjacent cells
+    // two particles within reach are in the same or adjacent cells.  A row's
+    // neighbouring cells are one run of the items; the three runs are taken
+    // as one list, a partner a lane.
     const int c0 = a.cl_cell[n], cx0 = c0 % a.ncx, cy0 = c0 / a.ncx;
-    for (int dyc = -1; dyc <= 1; dyc++) {
-      const int cy = (cy0 + dyc + a.ncy) % a.ncy;
-      for (int dxc = -1; dxc <= 1; dxc++) {
-        const int cx = cx0 + dxc;
-        if (cx < 0 || cx >= a.ncx) continue;
-        cell_candidates(a, n, cy * a.ncx + cx, s_cand, cnt);
-      }
+    const int xa = max(cx0 - 1, 0), xb = min(cx0 + 1, a.ncx - 1);
+    int r0[3], r1[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const int row = (cy0 + d - 1 + a.ncy) % a.ncy * a.ncx;
+      r0[d] = a.cl_start[row + xa];
+      r1[d] = a.cl_start[row + xb + 1];
+    }
+    const int e0 = r1[0] - r0[0], e1 = e0 + r1[1] - r0[1], e2 = e1 + r1[2] - r0[2];
+    for (int base = 0; base < e2; base += 64) {
+      const int t = base + lane;
+      const int k = t < e0 ? r0[0] + t : t < e1 ? r0[1] + (t - e0) : r0[2] + (t - e1);
+      const int m = t < e2 ? a.cl_items[k] : n;
+      add_candidates(lane, m, candidate(a, n, me, m, circle_of(a, m)), s_cand, cnt);
     }
     if (cnt > COLL_CAND_CAP) {
       if (lane == 0) atomicOr(&a.flags[0], 4);
@@ -1541,15 +1568,16 @@ __device__ void collide_particle(const CollArgs &a, int n) {
     }
     cand = s_sorted;
   } else {
-    for (int base = 0; base < a.np; base += 64) {
-      const int m = base + lane;
-      const bool c = m < a.np && m != n && pair_candidate(a, min(n, m), max(n, m));
-      const unsigned long long b = __ballot(c);
-      if (c) {
-        const int pos = cnt + __popcll(b & ((1ull << lane) - 1ull));
-        if (pos < COLL_CAND_CAP) s_cand[pos] = m;
+    // four partners a lane in flight
+    for (int base = 0; base < a.np; base += 256) {
+      Circle q[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) q[u] = circle_of(a, min(base + 64 * u + lane, a.np - 1));
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int m = base + 64 * u + lane;
+        add_candidates(lane, m, m < a.np && candidate(a, n, me, m, q[u]), s_cand, cnt);
       }
-      cnt += __popcll(b);
     }
     if (cnt > COLL_CAND_CAP) {
       if (lane == 0) atomicOr(&a.flags[0], 4);
@@ -1620,10 +1648,13 @@ __global__ __launch_bounds__(64 * WG_WAVES) void k_collide(CollArgs a) {
 }
 
 // The cell list of the collision broad phase at the particles' current
-// positions (x + dx, y + dy), in three launches:
+// positions (x + dx, y + dy, from cpos).  The order within a cell follows
+// atomics; the broad phase sorts each particle's candidates.  Up to
+// CELL_BUILD_MAX particles one workgroup builds it in one launch, gated like
+// the collisions it serves (CellBuildB: 14.4 -> 8.0 us at 4096).  Above, by
+// three launches:
 //  - count: each particle's cell, and its place in the cell from a device
-//    atomic on the cell's count (the order within a cell follows the
-//    atomics; the broad phase sorts each particle's candidates);
+//    atomic on the cell's count;
 //  - scan: one workgroup turns the counts into offsets and clears them, so
 //    that every build starts from zero counts;
 //  - place: each particle's index stored at its cell's offset plus its place.
@@ -1638,6 +1669,82 @@ __device__ inline int cell_of(const CollArgs &a, double x, double y) {
   const int cx = min(max((int)floor(x * (1. / a.hx)), 0), a.ncx - 1);
   const int cy = min(max((int)floor(yw * (1. / a.hy)), 0), a.ncy - 1);
   return cy * a.ncx + cx;
+}
+
+// cnt (nc counts in LDS) turned into exclusive offsets by the workgroup's
+// threads, part their partial sums; returns the total.  Each thread sums a
+// contiguous run; the runs' sums are scanned within each wave by lane
+// shuffles, the waves' totals by the first wave.
+__device__ inline int cell_offsets(int *cnt, int *part, int nc) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int per = (nc + blockDim.x - 1) / blockDim.x;
+  const int k0 = min(t * per, nc), k1 = min(k0 + per, nc);
+  int sum = 0;
+  for (int k = k0; k < k1; k++) sum += cnt[k];
+  int inc = sum;  // inclusive scan of the wave's run sums
+  for (int d = 1; d < 64; d <<= 1) {
+    const int v = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += v;
+  }
+  if (lane == 63) part[w] = inc;
+  __syncthreads();
+  if (w == 0) {
+    const int nw = blockDim.x >> 6;
+    int tot = lane < nw ? part[lane] : 0;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(tot, d, 64);
+      if (lane >= d) tot += v;
+    }
+    if (lane < nw) part[32 + lane] = tot;  // inclusive totals of waves
+  }
+  __syncthreads();
+  int run = (w > 0 ? part[32 + w - 1] : 0) + inc - sum;  // exclusive offset of this run
+  for (int k = k0; k < k1; k++) {
+    const int v = cnt[k];
+    cnt[k] = run;
+    run += v;
+  }
+  __syncthreads();
+  return part[32 + (blockDim.x >> 6) - 1];
+}
+
+// The whole list in one launch, by one workgroup with the counts in LDS.
+struct CellBuildB {
+  static constexpr int T = 1024, M = 0;
+  static __device__ __forceinline__ void run(const VB &vb, CollArgs a) {
+    if (halted(a.halt)) return;
+    if (!sub_open(a.res, a.sub)) return;
+    extern __shared__ int cl_lds[];
+    const int nc = a.ncx * a.ncy, t = threadIdx.x;
+    int *cnt = cl_lds, *part = cl_lds + nc;
+    int cell[CELL_BUILD_MAX / T], slot[CELL_BUILD_MAX / T];
+#pragma unroll
+    for (int u = 0; u < CELL_BUILD_MAX / T; u++) {
+      const double *p = a.cpos + 4 * (long)min(t + u * T, a.np - 1);
+      cell[u] = cell_of(a, p[0], p[1]);
+    }
+    for (int k = t; k < nc; k += T) cnt[k] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < CELL_BUILD_MAX / T; u++) {
+      const int n = t + u * T;
+      if (n >= a.np) continue;
+      a.cl_cell[n] = cell[u];
+      slot[u] = atomicAdd(&cnt[cell[u]], 1);
+    }
+    __syncthreads();
+    const int total = cell_offsets(cnt, part, nc);
+    for (int k = t; k < nc; k += T) a.cl_start[k] = cnt[k];
+    if (t == 0) a.cl_start[nc] = total;
+#pragma unroll
+    for (int u = 0; u < CELL_BUILD_MAX / T; u++) {
+      const int n = t + u * T;
+      if (n < a.np) a.cl_items[cnt[cell[u]] + slot[u]] = n;
+    }
+  }
+};
+__global__ __launch_bounds__(1024) void k_cell_build(CollArgs a) {
+  CellBuildB::run(VB::here(), a);
 }
 
 struct CellCountB {
@@ -1670,40 +1777,9 @@ struct CellScanB {
       counts[k] = 0;
     }
     __syncthreads();
-    // exclusive scan: each thread sums a contiguous run; the runs' sums
-    // are scanned within each wave by lane shuffles, the waves' totals by
-    // the first wave; each run is offset in LDS, then stored coalesced
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int per = (nc + blockDim.x - 1) / blockDim.x;
-    const int k0 = min(t * per, nc), k1 = min(k0 + per, nc);
-    int sum = 0;
-    for (int k = k0; k < k1; k++) sum += cnt[k];
-    int inc = sum;  // inclusive scan of the wave's run sums
-    for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(inc, d, 64);
-      if (lane >= d) inc += v;
-    }
-    if (lane == 63) part[w] = inc;
-    __syncthreads();
-    if (w == 0) {
-      const int nw = blockDim.x >> 6;
-      int tot = lane < nw ? part[lane] : 0;
-      for (int d = 1; d < 64; d <<= 1) {
-        const int v = __shfl_up(tot, d, 64);
-        if (lane >= d) tot += v;
-      }
-      if (lane < nw) part[32 + lane] = tot;  // inclusive totals of waves
-    }
-    __syncthreads();
-    int run = (w > 0 ? part[32 + w - 1] : 0) + inc - sum;  // exclusive offset of this run
-    for (int k = k0; k < k1; k++) {
-      const int v = cnt[k];
-      cnt[k] = run;
-      run += v;
-    }
-    __syncthreads();
-    for (int k = t; k < nc; k += blockDim.x) a.cl_start[k] = cnt[k];
-    if (t == blockDim.x - 1) a.cl_start[nc] = part[32 + (blockDim.x >> 6) - 1];
+    const int total = cell_offsets(cnt, part, nc);
+    for (int k = threadIdx.x; k < nc; k += blockDim.x) a.cl_start[k] = cnt[k];
+    if (threadIdx.x == 0) a.cl_start[nc] = total;
   }
 };
 __global__ __launch_bounds__(1024) void k_cell_scan(CollArgs a, int *counts) {
@@ -1979,6 +2055,11 @@ struct ResetB {
       // foot-point warm starts reach back no further than the stage start, so
       // that a run restarted from a save repeats the same operations
       a.sc_key[8 * (long)n + 7] = 0;
+      // the broad phase's packed position
+      double *cp = a.cpos + 4 * (long)n;
+      cp[0] = x;
+      cp[1] = y;
+      cp[2] = fmax(pa, pb);
     }
     prev.boxes = false;
     double q[3] = {member(R_DEN), pa, pb};  // the members that the shape needs
@@ -2376,18 +2457,22 @@ static CollArgs coll_args(Ctx *c, int cnstep) {
 static void launch_cell_list(Ctx *c, const CollArgs &a, hipStream_t st) {
   if (!a.use_cells) return;
   const size_t lds = ((size_t)c->cl_ncx * c->cl_ncy + 1024) * sizeof(int);
+  if (c->np <= CELL_BUILD_MAX) {
+    go<CellBuildB>(k_cell_build, dim3(1), dim3(CellBuildB::T), lds, st, a);
+    return;
+  }
   const dim3 g((c->np + 255) / 256);
   go<CellCountB>(k_cell_count, g, dim3(256), 0, st, a, c->cl_count);
   go<CellScanB>(k_cell_scan, dim3(1), dim3(1024), lds, st, a, c->cl_count);
   go<CellPlaceB>(k_cell_place, g, dim3(256), 0, st, a);
 }
 
-int launch_collision(Ctx *c, int cnstep, hipStream_t st) {
+int launch_collision(Ctx *c, int cnstep, hipStream_t st, bool packed) {
   if (c->np == 0) return EIF_OK;
   if (!st) st = c->stream;
   ProfScope ps(c, "collision", st);
   const CollArgs a = coll_args(c, cnstep);
-  go<CollPackB>(k_coll_pack, dim3((c->np + 255) / 256), dim3(256), 0, st, a);
+  if (!packed) go<CollPackB>(k_coll_pack, dim3((c->np + 255) / 256), dim3(256), 0, st, a);
   launch_cell_list(c, a, st);
   go<CollideB>(k_collide, wave_grid(c->np), dim3(64 * WG_WAVES), 0, st, a);
   EIF_HIP(hipGetLastError());

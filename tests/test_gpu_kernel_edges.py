@@ -292,3 +292,27 @@ def test_downloads_return_the_fields(nx, ny):
     g._check(g.lib.fluid_gpu_download(g.h, None, None, eif._ptr(p)))
     assert np.array_equal(p, want["p"].reshape(p.shape))
     g.close()
+
+
+# the cell list by one workgroup (up to 8192 particles, 1024 a turn) and by
+# three launches: the partners of the test of all pairs, in the same order.
+# Circles: the reference's fixed point of overlapping ellipses need not end.
+@pytest.mark.parametrize("n", [1023, 1025, 8192, 8193])
+def test_cell_list_finds_the_pairs_of_all_pairs(n):
+    nx, ny, ly = 128, 256, 2.0
+    k = np.arange(n)
+    rng = np.random.default_rng(n)
+    a = rng.uniform(0.007, 0.0085, n)
+    part = dict(den=np.ones(n), a=a, b=a, x=(k % 64 + 0.5) / 64,
+                y=(k // 64 + 0.5) * ly / 129, az=rng.uniform(0, 2 * np.pi, n), ux=np.zeros(n),
+                uy=rng.uniform(-1, 1, n), vz=np.zeros(n))
+    got = []
+    for search in (eif.COLLISION_ALL_PAIRS, eif.COLLISION_CELLS):
+        g = eif.Solver(nx, ny, ly=ly, poisson_mode=eif.POISSON_PARTITION)
+        g.set_particles(**part)
+        g.set_collision_search(search)
+        g.compute_collision_force(0)
+        got.append((g.colliding_pairs(), g.particles()))
+        g.close()
+    assert got[0][0] == got[1][0] and len(got[0][0]) > 20
+    assert np.array_equal(got[0][1], got[1][1])
