@@ -316,3 +316,24 @@ def test_cell_list_finds_the_pairs_of_all_pairs(n):
         g.close()
     assert got[0][0] == got[1][0] and len(got[0][0]) > 20
     assert np.array_equal(got[0][1], got[1][1])
+
+
+# weights of an ellipse 180 cells wide: distances past the exponential's
+# clamp, its centre (foot on the evolute) and the saturated range.  The sums
+# add 1.4e5 cells in another order than the oracle: at most N eps = 1.6e-11
+# of the sum of the terms' sizes (positive here).
+def test_inertia_of_a_wide_ellipse():
+    kw = dict(itot=512, jtot=512, ly=1.0)
+    part = dict(den=[1.0], a=[0.42], b=[0.36], x=[0.5], y=[0.5], az=[0.3])
+    got = []
+    for s in (eif.Solver(**kw), Oracle(**kw)):
+        s.upload(ux=np.full(s.shapes["ux"], 0.75), uy=np.full(s.shapes["uy"], 1.25))
+        s.update_boundaries()
+        s.set_particles(**part)
+        s.reset_particle_increments()
+        s.compute_inertia(0)
+        got.append(np.array(s.particles())[0])
+        s.close()
+    for m in (18, 20):  # iux, iuy of step 0
+        assert got[1][m] > 0.5
+        assert abs(got[0][m] - got[1][m]) <= 1.6e-11 * got[1][m]
