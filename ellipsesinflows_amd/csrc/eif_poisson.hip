@@ -8,8 +8,8 @@
 // reference's two MPI transposes (:94, :118) have no counterpart.
 //
 // DCT-II / DCT-III (FFTW REDFT10 / REDFT01): Makhoul's n-point complex FFT
-// (radix-2, decimation in time) for powers of two, the direct sum
-// otherwise.  For 64 <= n <= 8192 the FFT runs in registers and two rows
+// (radix-2, decimation in time) for powers of two, mixed radices for other
+// n up to 5120, the direct sum beyond.  For 64 <= n <= 8192 the FFT runs in registers and two rows
 // share one complex transform (real and imaginary part); other powers of
 // two use one row per transform in LDS.  Every trigonometric factor comes
 // from the table C[m] = cos(pi m/(2n)) built on the host.

@@ -625,9 +625,9 @@ __global__ __launch_bounds__(256) void k_heads(IbmArgs a, int with_dx) {
   HeadsB::run(VB::here(), a, with_dx);
 }
 
-// src/suspensions/inertia.c:9-70.  One wave per slice of IBM_SLICE box
-// cells of one particle (its three images' boxes flattened); the last
-// slice of a particle to finish adds the slices' sums in slice order.
+// src/suspensions/inertia.c:9-70.  One wave per slice of 64 U box cells of
+// one particle (its three images' boxes flattened); the increment adds the
+// slices' sums.
 // open: the sub-iteration gate, evaluated by the caller; tested after this
 // slice's own loads are issued, so the gate's load is not waited for alone
 template <int U>
