@@ -1680,8 +1680,8 @@ __global__ __launch_bounds__(64 * WG_WAVES) void k_collide(CollArgs a) {
 // positions (x + dx, y + dy, from cpos).  The order within a cell follows
 // atomics; the broad phase sorts each particle's candidates.  Up to
 // CELL_BUILD_MAX particles one workgroup builds it in one launch, gated like
-// the collisions it serves (CellBuildB: 14.4 -> 8.0 us at 4096).  Above, by
-// three launches:
+// the collisions it serves (CellBuildB: 14.4 -> 8.0 us at 4096 in a step; 7.5
+// against the three launches' 15.2 at 8192).  Above, by three launches:
 //  - count: each particle's cell, and its place in the cell from a device
 //    atomic on the cell's count;
 //  - scan: one workgroup turns the counts into offsets and clears them, so
