@@ -184,11 +184,11 @@ static void free_ctx(Ctx *c) {
                      &c->th_q1, &c->th_den, &c->th_last, &c->pt_fwd, &c->pt_u,
                      &c->pt_v, &c->pt_w, &c->pt_bnd, &c->pt_red, &c->pt_lvl, &c->pt_ends, &c->pt_g, &c->dscal, &c->dred,
                      &c->prt, &c->pconst, &c->dt_part, &c->sc_fx, &c->sc_fy, &c->sc_dist, &c->sc_pos,
-                     &c->res_slots, &c->st_ux1, &c->st_ux2, &c->st_uy1,
+                     &c->sc_t, &c->res_slots, &c->st_ux1, &c->st_ux2, &c->st_uy1,
                      &c->st_uy2, &c->st_phi, &c->slice_part, &c->slice_part0};
   for (auto b : bufs)
     if (*b) (void)hipFree(*b);
-  void *others[] = {c->sc_t, c->boxes, c->box_off, c->tile_cnt, c->tile_list,
+  void *others[] = {c->boxes, c->box_off, c->tile_cnt, c->tile_list,
                     c->flags, c->rows, c->row_cnt, c->wall_hit,
                     c->ibm_stats, c->slice_first, c->slice_info, c->ibm_pp, c->slice_rec,
                     c->sc_key, c->heads, c->cl_start, c->cl_items, c->cl_cell, c->cl_slot, c->cl_count};

@@ -105,139 +105,43 @@ __device__ inline double signed_dist(const EllipseShape &e, double grid_size,
 }
 
 // ---------------------------------------------------------------------
-// Foot of the normal.
+// Foot of the normal for the IBM weights.
 //
 // src/ellipse.c:30-65 iterates t <- clamp(t + dt) from t = pi/4 until
 // |dt| < 1e-8, every iteration in FP64 with sin, cos, asin and three
 // square roots.  The iteration converges quadratically to the unique foot
-// on the first-quadrant arc, so here it starts in FP32 (stopped at
-// |dt| < 1e-3, where the FP32 rounding noise takes over) and finishes in
-// FP64.
+// on the first-quadrant arc, so here it starts in FP32 (foot_fp32: hardware
+// sin/cos, stopped at |dt| < 1e-3, where the FP32 rounding noise takes over)
+// and finishes with the reference's FP64 iteration and stopping rule
+// (foot_fp64), which then needs one or two iterations instead of about four
+// (1.51 per evaluated cell at 2048x4096, 1024 ellipses).  After the first
+// FP64 step every update of t is below 2^-10, so cos and sin of the new t
+// follow from the old ones by the addition theorem with the Taylor series
+// of cos(delta) and sin(delta) (truncation below 1e-21), and only one FP64
+// sincos is evaluated per cell.  The converged (cos t, sin t) agree with
+// the reference's to a few units in the last place.
 //
-// The collisions use the foot itself (foot_fp32, foot_fp64): the reference's
-// iteration in t and its stopping rule.
-//
-// The weights use only the distance, which is stationary in t
-// (foot_dist_fp32, foot_dist_fp64): cos t and sin t come from the hardware in
-// FP32, normalised to FP64 once and turned by dt from there; the factors that only set the length of a step come from the
-// hardware reciprocal square root (relative error 2^-23); and it ends at
-// |dt| < 2^-17.  The last step leaves an error e ~ dt^2 / 10 ~ 6e-12 in t,
-// which changes the distance by e^2 (at the evolute, where the convergence
-// slows to linear, the distance's second derivative vanishes too and it
-// changes by dt^3 / 6 < 1e-16).  The foot's parameter is kept per cell in
-// FP32, the start of the cell's next search in the same RK stage.
-// The FP64 and FP32 iterations per evaluated cell went from 1.51 and 0.05 to
-// 1.00 and 0.41 (2048x4096, 1024 ellipses), and an FP64 iteration from 124
-// instructions (and 51 of sincos) to 75.
+// The weights use only the distance, which is stationary in t for a cell
+// centre off the boundary, but the stopping rule cannot be loosened for that:
+// on the boundary an error of t enters linearly, with a factor that grows as
+// b / a falls.  Ended at |dt| < 2^-17 with the length factors and the
+// starting cos t, sin t in FP32, 60 steps took 119.5 ms instead of 126.6
+// (2048x4096, 1024 ellipses) and 6 steps 12.8 instead of 13.8 (1024x2048,
+// 4096 ellipses), but distances were off by 1e-11 (b/a = 1) to 3e-10 cells
+// (b/a = 0.1) at 20 cells, against 5e-15 here.
 // ---------------------------------------------------------------------
-// where the FP64 iteration of the weights ends
-constexpr double FOOT_DIST_DT = 0x1p-17;
 
-// hardware cosine and sine of t in [0, pi/2] (absolute error below 1e-6)
-__device__ inline void cossin_hw(float t, float &c, float &s) {
-  const float rev = t * 0.15915494f;
-  c = __builtin_amdgcn_cosf(rev);
-  s = __builtin_amdgcn_sinf(rev);
-}
-
-// FP32 part for the distance: t from its start until |dt| < 1e-3 (at most 8
-// iterations)
-__device__ inline void foot_dist_fp32(const EllipseShape32 &f, float px, float py, float &t,
-                                      int &it32) {
-  for (int n = 0; n < 8; n++) {
-    float c, s;
-    cossin_hw(t, c, s);
-    const float x = f.a * c, y = f.b * s;
-    const float ex = f.kex * (c * c * c), ey = f.key * (s * s * s);
-    const float rx = x - ex, ry = y - ey;
-    const float qx = px - ex, qy = py - ey;
-    const float rr = fmaf(rx, rx, ry * ry), qq = fmaf(qx, qx, qy * qy);
-    float arg = fmaf(rx, qy, -(ry * qx)) * __builtin_amdgcn_rsqf(rr * qq);
-    arg = fminf(fmaxf(arg, -1.f), 1.f);
-    const float den = fmaxf(fmaf(-x, x, fmaf(-y, y, f.a2b2)), 1e-30f);
-    const float a2 = arg * arg;
-    const float as = fmaf(arg * a2, fmaf(a2, fmaf(a2, 0.044642857f, 0.075f), 0.16666667f), arg);
-    const float dt = rr * as * __builtin_amdgcn_rsqf(rr * den);
-    it32++;
-    if (!(fabsf(dt) < 1e30f)) break;  // no usable step: hand over to FP64
-    t = fminf(fmaxf(t + dt, 0.f), 1.5707963f);
-    if (fabsf(dt) < 1e-3f) break;
-  }
-}
-
-// FP64 part for the distance: (c, s) = (cos t, sin t) from the hardware's
-// (normalised here to FP64) until |dt| < FOOT_DIST_DT; t follows in FP32
-__device__ inline void foot_dist_fp64(const EllipseShape &e, double px, double py, float &t,
-                                      double &c, double &s, int &it64) {
-  {
-    float cf, sf;
-    cossin_hw(t, cf, sf);
-    c = (double)cf;
-    s = (double)sf;
-    const double d = fma(c, c, fma(s, s, -1.));  // |d| < 4e-6: (1 + d)^(-1/2) to d^3
-    const double w = fma(d, fma(d, 0.375, -0.5), 1.);
-    c *= w;
-    s *= w;
-  }
-  for (int n = 0;; n++) {
-    const double x = e.a * c, y = e.b * s;
-    const double ex = e.kex * (c * c * c), ey = e.key * (s * s * s);
-    const double rx = x - ex, ry = y - ey;
-    const double qx = px - ex, qy = py - ey;
-    const double rr = fma(ry, ry, rx * rx), qq = fma(qy, qy, qx * qx);
-    const double cross = rx * qy - ry * qx;
-    const double arg = cross * __builtin_amdgcn_rsq(rr * qq);
-    const double a2 = arg * arg;
-    const double as = fma(arg * a2, fma(a2, 0.075, 1. / 6.), arg);
-    const double den = fma(-x, x, fma(-y, y, e.a2b2));
-    const double dt = as * (rr * __builtin_amdgcn_rsq(rr * den));
-    it64++;
-    if (!(fabs(dt) < 1e30)) {  // on the evolute: the reference's clamp goes to pi/2
-      const bool there = c == 0.;
-      c = 0.;
-      s = 1.;
-      t = 1.5707963f;
-      if (there || n > 100) break;
-      continue;
-    }
-    const double d2 = dt * dt;
-    const double hc = d2 * fma(d2, -1. / 24., 0.5);  // 1 - cos(dt), |dt| small
-    const double sd = dt * fma(d2, fma(d2, 1. / 120., -1. / 6.), 1.);
-    const double cn = c - fma(s, sd, c * hc), sn = s + fma(c, sd, -(s * hc));
-    c = cn;
-    s = sn;
-    t += (float)dt;
-    if (fabs(dt) > 0x1p-10) {  // a large step: the series is short, normalise
-      const double w = rsqrt_nr(fma(c, c, s * s));
-      c *= w;
-      s *= w;
-    }
-    if (c < 0.) {
-      c = 0.;
-      s = 1.;
-      t = 1.5707963f;
-    }
-    if (s < 0.) {
-      c = 1.;
-      s = 0.;
-      t = 0.f;
-    }
-    if (fabs(dt) < FOOT_DIST_DT || n > 100) break;
-  }
-}
-
-// compute_signed_dist (src/suspensions/auxiliary.c:19-47); the unfolding of
-// ellipse.c:62-63 maps (cos t, sin t) of the folded foot to (-cos t, sin t)
-// for x_ < 0 and (cos t, -sin t) for y_ < 0.  t: where the foot's search
-// starts, and its parameter on return: pi/4, or the parameter this cell's
-// foot had at the particle's previous evaluation in the same RK stage, which
-// the particle has barely moved from.  search: through FP32 iterations first
-// (from pi/4, or when the particle moved by more than one FP64 step
-// resolves).  The root on the first-quadrant arc is unique, so the start
-// changes only the number of iterations.
+// compute_signed_dist (src/suspensions/auxiliary.c:19-47) with the foot
+// from foot_fp32 / foot_fp64; the unfolding of ellipse.c:62-63 maps
+// (cos t, sin t) of the folded foot to (-cos t, sin t) for x_ < 0 and
+// (cos t, -sin t) for y_ < 0.  t: the foot's parameter on return; where the
+// search starts if warm, the parameter this cell's foot had at the particle's
+// previous evaluation in the same RK stage, which the particle has barely
+// moved from (else from the FP32 estimate).  The root on the first-quadrant
+// arc is unique, so the start changes only the number of iterations.
 __device__ inline double signed_dist_from(const EllipseShape &e, const EllipseShape32 &f,
                                           double inv_grid, double px, double py, double cr,
-                                          double sr, double x, double y, bool search, float &t,
+                                          double sr, double x, double y, bool warm, double &t,
                                           int &it32, int &it64) {
   const double ddx = x - px, ddy = y - py;
   const double x_ = cr * ddx - sr * ddy;
@@ -246,10 +150,12 @@ __device__ inline double signed_dist_from(const EllipseShape &e, const EllipseSh
   const double f0 = 1. - xa * xa - yb * yb;
   const double sign = f0 > 0. ? +1. : -1.;
   const double ax = fabs(x_), ay = fabs(y_);
-  if (search) foot_dist_fp32(f, (float)ax, (float)ay, t, it32);
+  if (!warm) t = (double)foot_fp32(f, ax, ay, it32);
   double ct, st;
-  foot_dist_fp64(e, ax, ay, t, ct, st, it64);
-  const double ex = copysign(e.a * ct, x_) - x_, ey = copysign(e.b * st, y_) - y_;
+  foot_fp64(e, ax, ay, t, ct, st, it64);
+  const double fx = x_ < 0. ? -(e.a * ct) : e.a * ct;
+  const double fy = y_ < 0. ? -(e.b * st) : e.b * st;
+  const double ex = fx - x_, ey = fy - y_;
   const double dist = sign * sqrt_pos(+ex * ex + ey * ey);
   return dist * inv_grid;
 }
@@ -348,7 +254,7 @@ struct IbmArgs {
   double *sc_fx, *sc_fy;
   double *sc_dist;  // per box cell: tanh(BETA d) of the signed distance d
   double *sc_pos;
-  float *sc_t;    // per box cell: foot parameter of the last evaluation
+  double *sc_t;   // per box cell: foot parameter of the last evaluation
   int *sc_key;    // per particle: boxes of that evaluation (8 ints)
   int *tile_cnt, *tile_list;
   int ntx, nty;
@@ -538,7 +444,6 @@ struct SliceHead {
   EllipseShape32 f;
   int cached;          // the distance cache holds this position
   int warm;            // the foot parameters hold these boxes
-  int far;             // ... of a position too far for one FP64 step
 };
 
 // lane l's integer, l the same on every lane of the wave
@@ -561,13 +466,11 @@ __device__ inline CachedPass cached_records(const IbmArgs &a, int n, int lane) {
 }
 
 // The position-dependent parts of a particle's header, by the lanes of one
-// wave: lanes 0, 1, 2 make the boxes of the three images.  lo, hi: the
-// particle's semi-axes in order; known: the cache holds prev's pass itself
-// (else how far its position lies is not looked at)
+// wave: lanes 0, 1, 2 make the boxes of the three images.  rad: the
+// particle's larger semi-axis
 __device__ inline void write_head(const IbmArgs &a, SliceHead *h, int lane, double px, double py,
-                                  double paz, double lo, double hi, const CachedPass &prev,
-                                  bool known) {
-  const Img m = make_img(a, px, py + a.ly * (min(lane, 2) - 1), hi);
+                                  double paz, double rad, const CachedPass &prev) {
+  const Img m = make_img(a, px, py + a.ly * (min(lane, 2) - 1), rad);
   const int total = lane_int(m.cnt, 0) + lane_int(m.cnt, 1) + lane_int(m.cnt, 2);
   const bool same = __ballot(m.imin != prev.imin || m.jmin != prev.jmin) == 0ull &&
                     total == prev.total;
@@ -583,10 +486,6 @@ __device__ inline void write_head(const IbmArgs &a, SliceHead *h, int lane, doub
     h->bs.total = total;
     h->cached = prev.pos && prev.px == px && prev.py == py && prev.paz == paz;
     h->warm = prev.boxes && same;
-    // a foot moves by at most the displacement over the smallest radius of
-    // curvature, but for cells near the evolute
-    h->far = !known || (fabs(px - prev.px) + fabs(py - prev.py) + hi * fabs(paz - prev.paz)) * hi >
-                           0.5 * FOOT_DIST_DT * lo * lo;
   }
 }
 
@@ -618,7 +517,7 @@ struct HeadsB {
     const CachedPass prev = cached_records(a, n, lane);
     write_head_shape(a, h, n, lane, q);
     write_head(a, h, lane, q[R_X] + w * q[R_DX], q[R_Y] + w * q[R_DY], q[R_AZ] + w * q[R_DAZ],
-               fmin(q[R_A], q[R_B]), fmax(q[R_A], q[R_B]), prev, false);
+               fmax(q[R_A], q[R_B]), prev);
   }
 };
 __global__ __launch_bounds__(256) void k_heads(IbmArgs a, int with_dx) {
@@ -648,9 +547,9 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
   const EllipseShape32 f = hd.f;
   const double px = hd.px, py = hd.py;
   const double inv_pm = hd.inv_pm, inv_pim = hd.inv_pim;
-  const bool cached = hd.cached, warm = hd.warm, search = !warm || hd.far;
+  const bool cached = hd.cached, warm = hd.warm;
   double *dist = a.sc_dist + hd.off;
-  float *tcell = a.sc_t + hd.off;
+  double *tcell = a.sc_t + hd.off;
   const double cr = hd.cr, sr = hd.sr;
   const double dxdy = a.dx * a.dy;
   double acc[3] = {0., 0., 0.};  // iux, iuy, ivz
@@ -660,8 +559,7 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
   // all loads of the lane's cells first (a cell past t1 loads the last cell
   // instead and is not added), then the weights and the sums in cell order
   if (t0 < t1) {
-    double th_[U], x_[U], y_[U], vx0[U], vx1[U], vy0[U], vy1[U];
-    float tp[U];
+    double th_[U] = {}, x_[U], y_[U], vx0[U], vx1[U], vy0[U], vy1[U];
     int k_[U], i_[U], j_[U];
     lane_cells<U>(bs, t0, t1, lane, k_, i_, j_);
 #pragma unroll
@@ -674,15 +572,11 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
       vy0[u] = a.uy[fy];
       vy1[u] = a.uy[fy + (unsigned)(a.nx + 2)];
     }
-    if (cached) {
+    // th, or the foot's parameter that its search starts from
+    if (cached || warm) {
+      const double *from = cached ? dist : tcell;
 #pragma unroll
-      for (int u = 0; u < U; u++) th_[u] = dist[min(t0 + lane + 64 * u, t1 - 1)];
-    } else if (warm) {
-#pragma unroll
-      for (int u = 0; u < U; u++) tp[u] = tcell[min(t0 + lane + 64 * u, t1 - 1)];
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; u++) tp[u] = (float)(0.25 * EIF_PI);
+      for (int u = 0; u < U; u++) th_[u] = from[min(t0 + lane + 64 * u, t1 - 1)];
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
@@ -691,9 +585,10 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
       const double py_ = py + a.ly * (k_[u] - 1);
       const double x = x_[u], y = y_[u];
       if (!cached) {
-        th_[u] = weight_th(signed_dist_from(e, f, 1. / a.grid_size, px, py_, cr, sr, x, y, search,
-                                            tp[u], it32, it64));
-        tcell[t] = tp[u];
+        double tf = th_[u];
+        th_[u] = weight_th(signed_dist_from(e, f, 1. / a.grid_size, px, py_, cr, sr, x, y, warm,
+                                            tf, it32, it64));
+        tcell[t] = tf;
         dist[t] = th_[u];
       }
       const double w = v_weight_th(th_[u]);
@@ -812,7 +707,6 @@ __device__ inline void finalize_x0_particle(const IbmArgs &a, int n) {
   SliceHead *h = a.heads + n;
   h->cached = 1;
   h->warm = 1;
-  h->far = 0;
 }
 
 // one wave per particle, four per workgroup
@@ -849,7 +743,7 @@ __global__ __launch_bounds__(IBM_THREADS) void k_ref_iterations(IbmArgs a,
   }
   __syncthreads();
   double cr, sr;
-  sincos(-paz, &sr, &cr);
+  sincos_angle(-paz, sr, cr);
   int iters = 0;
   for (long t = threadIdx.x; t < bs.total; t += IBM_THREADS) {
     int k, i, j;
@@ -918,9 +812,9 @@ struct IbmDistB {
   if (!cached) {
     const EllipseShape e = hd.e;
     const EllipseShape32 f = hd.f;
-    const bool warm = hd.warm, search = !warm || hd.far, single = single_image(bs);
+    const bool warm = hd.warm, single = single_image(bs);
     double *dist = a.sc_dist + hd.off;
-    float *tcell = a.sc_t + hd.off;
+    double *tcell = a.sc_t + hd.off;
     const double cr = hd.cr, sr = hd.sr;
     const int t0 = (slice - s0) * a.slice;
     const int t1 = t0 + a.slice < total ? t0 + a.slice : total;
@@ -928,9 +822,9 @@ struct IbmDistB {
       int k, i, j;
       cell_of(bs, t, k, i, j, single);
       const double py_ = py + a.ly * (k - 1);
-      float tp = warm ? tcell[t] : (float)(0.25 * EIF_PI);
+      double tp = warm ? tcell[t] : 0.;
       dist[t] = weight_th(signed_dist_from(e, f, 1. / a.grid_size, px, py_, cr, sr, a.xc[i],
-                                           a.yc[j - 1], search, tp, it32, it64));
+                                           a.yc[j - 1], warm, tp, it32, it64));
       tcell[t] = tp;
     }
   }
@@ -1961,7 +1855,7 @@ struct IncrementB {
     const double dyn = 0.5 * ga * dt * (uy0 + uy1);
     const double dazn = 0.5 * ga * dt * (vz0 + vz1);
     const double x = member(R_X) + dxn, y = member(R_Y) + dyn, az = member(R_AZ) + dazn;
-    const double lo = fmin(member(R_A), member(R_B)), hi = fmax(member(R_A), member(R_B));
+    const double rad = fmax(member(R_A), member(R_B));
     if (lane == 0) {
       if (fin) {
         p[R_IUX + 1] = iux1;
@@ -1983,10 +1877,10 @@ struct IncrementB {
       double *cp = ia.cpos + 4 * (long)n;
       cp[0] = x;
       cp[1] = y;
-      cp[2] = hi;
+      cp[2] = rad;
     }
     // the next sub-iteration's inertia pass
-    write_head(ia, ia.heads + n, lane, x, y, az, lo, hi, prev, fin != 0);
+    write_head(ia, ia.heads + n, lane, x, y, az, rad, prev);
   }
   if (lane == 0) red[w] = res;
   __syncthreads();
@@ -2093,7 +1987,7 @@ struct ResetB {
     prev.boxes = false;
     double q[3] = {member(R_DEN), pa, pb};  // the members that the shape needs
     write_head_shape(a, h, n, lane, q);
-    write_head(a, h, lane, x, y, az, fmin(pa, pb), fmax(pa, pb), prev, false);
+    write_head(a, h, lane, x, y, az, fmax(pa, pb), prev);
   }
 };
 __global__ __launch_bounds__(256) void k_reset(IbmArgs a, double *res, int *tile_cnt, int ntiles,
@@ -2237,7 +2131,7 @@ int susp_init(Ctx *c) {
   EIF_HIP(hipMalloc(&c->sc_fx, sc));
   EIF_HIP(hipMalloc(&c->sc_fy, sc));
   EIF_HIP(hipMalloc(&c->sc_dist, sc));
-  EIF_HIP(hipMalloc(&c->sc_t, sc / 2));
+  EIF_HIP(hipMalloc(&c->sc_t, sc));
   EIF_HIP(hipMalloc(&c->sc_key, 8 * (size_t)(c->np > 0 ? c->np : 1) * sizeof(int)));
   EIF_HIP(hipMemset(c->sc_key, 0, 8 * (size_t)(c->np > 0 ? c->np : 1) * sizeof(int)));
   EIF_HIP(hipMalloc(&c->sc_pos, 4 * (size_t)(c->np > 0 ? c->np : 1) * sizeof(double)));

@@ -337,3 +337,42 @@ def test_inertia_of_a_wide_ellipse():
     for m in (18, 20):  # iux, iuy of step 0
         assert got[1][m] > 0.5
         assert abs(got[0][m] - got[1][m]) <= 1.6e-11 * got[1][m]
+
+
+# cell centres on the boundary of an ellipse whose axes are 325 and 65 cells
+# (5 p, q cells from its centre, p^2 + q^2 = 65^2): there an error of the foot's
+# parameter enters the distance linearly.  One velocity at a time reads the
+# weights of two cells.  Ten roundings of coordinates below 0.5 are 6e-16, over
+# the spacing of 1 / 1024 a distance of 6e-13 cells, and a weight changes by
+# as much as the distance; from a cold start and from the foot of a body 1/64
+# of a cell away.
+@pytest.mark.parametrize("warm", [False, True])
+def test_weights_on_the_boundary_of_a_thin_ellipse(warm):
+    nx, ny, h = 1024, 512, 1.0 / 1024
+    kw = dict(itot=nx, jtot=ny, ly=0.5, Re=100.0)
+    a, b, shift = 325 * h, 65 * h, h / 64 if warm else 0.0
+    part = dict(den=[1.0], a=[a], b=[b], x=[512.5 * h - shift], y=[256.5 * h], az=[0.0])
+    legs = [(16, 63), (25, 60), (33, 56), (39, 52), (52, 39), (56, 33), (60, 25), (63, 16)]
+    g, o = eif.Solver(**kw), Oracle(**kw)
+    unit = 0.5 * h * h / (np.pi * a * b)
+    zero = np.zeros(g.shapes["uy"])
+    for s in (g, o):
+        s.set_particles(**part)
+        s.reset_particle_increments()
+        if warm:
+            s.compute_inertia(1)
+            rec = s.particles()
+            rec[:, 6] = shift
+            s.set_particle_records(rec)
+    for k, (p, q) in enumerate(legs):
+        i, j = 513 + (5 * p if k & 1 else -5 * p), 257 + (q if k & 2 else -q)
+        ux = np.zeros(g.shapes["ux"])
+        ux[j, i - 1] = 1.0
+        got = []
+        for s in (g, o):
+            s.upload(ux, zero)
+            s.compute_inertia(1)
+            got.append(s.particles()[0, 19] / unit)
+        assert 0.4 < got[1] < 1.6
+        assert abs(got[0] - got[1]) <= 2 * 6e-13, (p, q)
+    g.close()
