@@ -1,7 +1,7 @@
 // eif_ellipse.hpp -- ellipse geometry on the device (src/ellipse.c:7-65): the
-// shape's constants, sine and cosine of bounded angles, roots and exponentials
-// of the range that occurs, and the foot of the normal by the reference's
-// iteration (foot_fp32 for the start, foot_fp64 to its stopping rule).
+// shape's constants, sine and cosine of bounded angles, and the foot of the
+// normal by the reference's iteration (foot_fp32 for the start, foot_fp64 to
+// its stopping rule).
 #pragma once
 #include <hip/hip_runtime.h>
 #include "eif_internal.hpp"
@@ -112,50 +112,6 @@ __device__ inline double rsqrt_nr(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-(x * y), y, 1.);
   return fma(0.5 * y, e, y);
-}
-
-// sqrt(x) for 0 <= x <= 1e300 (below 1e-300 as of 1e-300), correctly rounded
-// but for rare last bits: the hardware estimate and three Newton steps,
-// without the library's scaling
-__device__ inline double sqrt_pos(double x) {
-  x = x < 1e-300 ? 1e-300 : x;
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double r = fma(-h, g, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  return fma(fma(-g, g, x), h, g);
-}
-
-// a constant in scalar registers: as a plain operand of fma it would be
-// moved into two vector registers by vector instructions
-__device__ inline double scalar(double c) {
-  asm("" : "+s"(c));
-  return c;
-}
-
-// exp(y) for y >= 0 (above 700 as of 700): y less the nearest multiple of
-// ln 2 (in two doubles), the Taylor polynomial on |r| <= ln(2)/2 (truncation
-// below 5e-18), the power of two by ldexp
-__device__ inline double exp_pos(double y) {
-  y = y > 700. ? 700. : y;
-  const double n = __builtin_rint(y * 1.4426950408889634);
-  const double r = fma(-n, 0x1.abc9e3b39803fp-56, fma(-n, 0x1.62e42fefa39efp-1, y));
-  double p = scalar(1. / 6227020800.);
-  p = fma(p, r, scalar(1. / 479001600.));
-  p = fma(p, r, scalar(1. / 39916800.));
-  p = fma(p, r, scalar(1. / 3628800.));
-  p = fma(p, r, scalar(1. / 362880.));
-  p = fma(p, r, scalar(1. / 40320.));
-  p = fma(p, r, scalar(1. / 5040.));
-  p = fma(p, r, scalar(1. / 720.));
-  p = fma(p, r, scalar(1. / 120.));
-  p = fma(p, r, scalar(1. / 24.));
-  p = fma(p, r, scalar(1. / 6.));
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.);
-  p = fma(p, r, 1.);
-  return ldexp(p, (int)n);
 }
 
 // asin by its Maclaurin series, exact to rounding for |x| <= 2^-6; for

@@ -156,26 +156,17 @@ __device__ inline double signed_dist_from(const EllipseShape &e, const EllipseSh
   const double fx = x_ < 0. ? -(e.a * ct) : e.a * ct;
   const double fy = y_ < 0. ? -(e.b * st) : e.b * st;
   const double ex = fx - x_, ey = fy - y_;
-  const double dist = sign * sqrt_pos(+ex * ex + ey * ey);
+  const double dist = sign * sqrt(+ex * ex + ey * ey);
   return dist * inv_grid;
 }
 
 // src/suspensions/auxiliary.c:49-59.  tanh(x) as 1 - 2 / (exp(2|x|) + 1)
 // with the sign of x: like the libm routine it rounds to exactly +-1 once
 // 2 / (exp(2|x|) + 1) drops below half an ulp of 1, so the weights are
-// exactly 0 or 1 on the same cells.  The exponential, the quotient (the
-// hardware reciprocal and two Newton steps) and the distance's root are this
-// file's own, without the libm routines' range checks and scaling: the
-// largest error against long double stays 2.2e-16 (2e7 arguments), and
-// the block of a cell takes 87 vector instructions instead of 120: in a pass
-// with the search k_inertia_collide 31.6 -> 30.6 us at 1024 ellipses on 2048x4096,
-// 35.3 -> 34.2 at 4096 on 1024x2048
+// exactly 0 or 1 on the same cells.
 __device__ inline double tanh_w(double x) {
-  const double t = exp_pos(2. * fabs(x)) + 1.;
-  double y = __builtin_amdgcn_rcp(t);
-  y = fma(y, fma(-t, y, 1.), y);
-  y = fma(y, fma(-t, y, 1.), y);
-  return copysign(fma(-2., y, 1.), x);
+  const double th = 1. - 2. / (exp(2. * fabs(x)) + 1.);
+  return copysign(th, x);
 }
 // Both weights are functions of th = tanh(BETA d); the per-cell cache keeps
 // th, so a cached cell needs no exp.
