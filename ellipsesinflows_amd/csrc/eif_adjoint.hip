@@ -344,8 +344,7 @@ __global__ __launch_bounds__(256) void k_adj_ibm(IbmAdj a) {
   const double U = q[R_UX], V = q[R_UY], W = q[R_VZ];
   const double s0 = a.seed[3 * n], s1 = a.seed[3 * n + 1], s2 = a.seed[3 * n + 2];
   const double dxdy = a.dx * a.dy, h = a.grid_size;
-  double cth, sth;
-  sincos_angle(-paz, sth, cth);
+  const double cth = cos(-paz), sth = sin(-paz);
   const EllipseShape e = make_shape(pa, pb);
   const EllipseShape32 e32 = shape32(e);
   double acc[6] = {0., 0., 0., 0., 0., 0.};

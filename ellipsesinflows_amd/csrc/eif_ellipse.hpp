@@ -88,24 +88,6 @@ __device__ inline void sincos_q1(double t, double &s, double &c) {
   c = low ? pc : ps;
 }
 
-// sin and cos of a particle's orientation: |x| <= 64 (angles are kept in
-// [0, 2 pi]) reduced by multiples of pi/2 held in two doubles, the same
-// polynomials; other angles through the library
-__device__ inline void sincos_angle(double x, double &s, double &c) {
-  if (!(fabs(x) <= 64.)) {
-    sincos(x, &s, &c);
-    return;
-  }
-  constexpr double PIO2_HI = 1.5707963267948966, PIO2_LO = 6.123233995736766e-17;
-  const double q = rint(x * 0.63661977236758134);
-  const double u = fma(-q, PIO2_LO, fma(-q, PIO2_HI, x));
-  const int m = (int)q;
-  const double ps = sin_poly(u), pc = cos_poly(u);
-  const double a = m & 1 ? pc : ps, b = m & 1 ? ps : pc;
-  s = m & 2 ? -a : a;
-  c = (m + 1) & 2 ? -b : b;
-}
-
 // 1/sqrt(x) from the hardware estimate and one Newton step (relative error
 // near 1e-16); used where only the size of a step depends on it
 __device__ inline double rsqrt_nr(double x) {

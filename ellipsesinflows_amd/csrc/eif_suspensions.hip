@@ -466,7 +466,7 @@ __device__ inline void write_head(const IbmArgs &a, SliceHead *h, int lane, doub
   const bool same = __ballot(m.imin != prev.imin || m.jmin != prev.jmin) == 0ull &&
                     total == prev.total;
   double sr, cr;
-  sincos_angle(-paz, sr, cr);
+  sincos(-paz, &sr, &cr);
   if (lane < 3) (&h->bs.b0)[lane] = m;
   if (lane == 0) {
     h->px = px;
@@ -734,7 +734,7 @@ __global__ __launch_bounds__(IBM_THREADS) void k_ref_iterations(IbmArgs a,
   }
   __syncthreads();
   double cr, sr;
-  sincos_angle(-paz, sr, cr);
+  sincos(-paz, &sr, &cr);
   int iters = 0;
   for (long t = threadIdx.x; t < bs.total; t += IBM_THREADS) {
     int k, i, j;
@@ -1329,7 +1329,7 @@ __device__ bool contact_force(const CollArgs &a, int n0, int n1, int wall, int s
   const EllipseShape sh = make_shape(e.a, e.b);
   const EllipseShape32 f = shape32(sh);
   double cp, sp;
-  sincos_angle(e.angle, sp, cp);
+  sincos(e.angle, &sp, &cp);
   const double cm = cp, sm = -sp;
   double tw = -1.;
   double cx = e.x, cy = e.y, ct = 0., st = 0.;
