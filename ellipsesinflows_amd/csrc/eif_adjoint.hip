@@ -383,17 +383,18 @@ __global__ __launch_bounds__(256) void k_adj_ibm(IbmAdj a) {
       int its = 0;
       double tt = (double)foot_fp32(e32, fabs(xl), fabs(yl), its), ct, st;
       foot_fp64(e, fabs(xl), fabs(yl), tt, ct, st, its);
-      const double fx = copysign(pa * ct, xl), fy = copysign(pb * st, yl);
-      const double vx = xl - fx, vy = yl - fy;
-      const double dr = sqrt(vx * vx + vy * vy);
-      const double dist = sign * dr / h;
-      // tanh, exactly +-1 where the forward's weights saturate
-      const double th = copysign(1. - 2. / (exp(2. * BETA_W * fabs(dist)) + 1.), dist);
-      double gxl = 0., gyl = 0.;
-      if (dr > 0.) {
-        gxl = sign * vx / (dr * h);
-        gyl = sign * vy / (dr * h);
-      }
+      sincos(tt, &st, &ct);  // closer than the search's own
+      // the distance's gradient is the inward normal at the foot, and the
+      // distance the projection on it.  The vector from the foot to the cell
+      // centre loses its direction as the centre nears the boundary (by eps a
+      // over the distance; 0 / 0 on it): largest error of the weight's
+      // gradient 5e-11 down to 1e-6 cells, 3e-13 here
+      const double mx = pb * ct, my = pa * st, mm = sqrt(mx * mx + my * my);
+      const double ux = mx / mm, uy = my / mm;
+      const double vx = fabs(xl) - pa * ct, vy = fabs(yl) - pb * st;
+      const double dist = sign * fabs(vx * ux + vy * uy) / h;
+      const double th = tanh(BETA_W * dist);
+      const double gxl = -copysign(ux, xl) / h, gyl = -copysign(uy, yl) / h;
       double wb = 0.;  // cotangent of the weight
       double dwdd;     // d weight / d dist
       double w;

@@ -376,3 +376,41 @@ def test_weights_on_the_boundary_of_a_thin_ellipse(warm):
         assert 0.4 < got[1] < 1.6
         assert abs(got[0] - got[1]) <= 2 * 6e-13, (p, q)
     g.close()
+
+
+# a circle of 25 cells about a cell centre: twenty cell centres lie on its
+# boundary, where the distance's gradient is the normal though the cell centre
+# is its own foot.  The cotangent of the position against central differences,
+# h = 1e-6: h^2 J''' is (128 h)^2 = 2e-8 of the derivative for weights that
+# change over a cell of 1/128, round-off of the difference 1e-10 J
+@pytest.mark.parametrize("az", [0.0, np.pi / 2])
+def test_adjoint_of_a_body_with_cell_centres_on_its_boundary(az):
+    n, h = 128, 1e-6
+    kw = dict(itot=n, jtot=n, ly=1.0, Re=40.0, extfrcy=0.2)
+    ux, uy, p = cases.random_fields(n, n, 3, amp=0.3)
+    p[:] = 0.0
+    c = 64.5 / n
+
+    def solver(dx=0.0, dy=0.0):
+        s = eif.Solver(**kw)
+        s.upload(ux, uy, p)
+        s.update_boundaries()
+        s.set_particles(den=[1.3], a=[25.0 / n], b=[25.0 / n], x=[c + dx], y=[c + dy], az=[az],
+                        ux=[0.1], uy=[-0.2], vz=[0.3])
+        return s
+
+    dts = [2e-4]
+    fd = [(objective(solver(**{k: h}), dts) - objective(solver(**{k: -h}), dts)) / (2 * h)
+          for k in ("dx", "dy")]
+    s = solver()
+    s.tape_begin()
+    s.step_fixed_dt(dts[0], record=True)
+    rec = s.particles()
+    seed = np.zeros((1, 3))
+    seed[:, 1] = -rec[:, 0] * np.pi * rec[:, 1] * rec[:, 2]
+    s.adjoint_add_wall_shear(1.0)
+    s.adjoint_add(s.ADJ_FORCE, seed)
+    for _ in range(3):
+        s.stage_adjoint()
+    got = s.adjoint_get(s.ADJ_PARTICLES)[0, :2]
+    assert np.max(np.abs(got - fd)) <= 1e-6 * np.max(np.abs(fd)), (got, fd)
