@@ -414,3 +414,38 @@ def test_adjoint_of_a_body_with_cell_centres_on_its_boundary(az):
         s.stage_adjoint()
     got = s.adjoint_get(s.ADJ_PARTICLES)[0, :2]
     assert np.max(np.abs(got - fd)) <= 1e-6 * np.max(np.abs(fd)), (got, fd)
+
+
+# values that are no ordinary numbers, on a grid whose divisions are not by
+# powers of two: an infinite, an overflowing and an undefined velocity give
+# what the reference's divisions give (infinities stay infinite, and drive the
+# time step to zero), and zeros keep their signs
+@pytest.mark.parametrize("value", [np.inf, -np.inf, 1.7e308, np.nan, -0.0])
+def test_grid_divisions_of_special_values(value):
+    nx, ny = 48, 30
+    kw = dict(itot=nx, jtot=ny, ly=0.9, Re=70.0)
+    g, o = eif.Solver(**kw), Oracle(**kw)
+    ux, uy, p = cases.random_fields(nx, ny, 9)
+    psi = 0.1 * p
+    if value == 0.0:
+        for f in (ux, uy, p, psi):
+            f[:] = 0.0
+    for k, f in enumerate((ux, uy, p, psi)):
+        f[11 + 3 * k, 17 + 2 * k] = value
+    with np.errstate(all="ignore"):
+        for s in (g, o):
+            s.upload(ux, uy, p)
+            s.update_boundaries()
+        assert g.decide_dt() == o.decide_dt()
+        for s in (g, o):
+            s.set_dt(1e-3)
+            s.update_velocity(0)
+            s.set_field("psi", psi)
+            s.correct_velocity(0)
+            s.update_pressure()
+        a, b = g.download(), o.download()
+        for k in ("ux", "uy", "p"):
+            assert np.array_equal(a[k], b[k], equal_nan=True), k
+            there = ~np.isnan(a[k])
+            assert np.array_equal(np.signbit(a[k][there]), np.signbit(b[k][there])), k
+    g.close()
