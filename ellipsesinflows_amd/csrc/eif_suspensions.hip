@@ -2094,8 +2094,10 @@ int susp_init(Ctx *c) {
   }
   c->slice_len = IBM_SLICE;
   while (c->slice_len > 64 && all / c->slice_len < IBM_WAVES) c->slice_len /= 2;
+  // room for whole slices of IBM_SLICE whatever the length: bodies that grow
+  // by an upload of their records fit or do not at the same sizes
   for (int n = 0; n < c->np; n++)
-    first[n + 1] = first[n] + (int)((box[n] + c->slice_len - 1) / c->slice_len);
+    first[n + 1] = first[n] + (int)((box[n] + IBM_SLICE - 1) / IBM_SLICE) * (IBM_SLICE / c->slice_len);
   c->scratch_cells = off[c->np];
   c->nslices = first[c->np];
   TRY_S(coll_cells_setup(c, rec.data()));

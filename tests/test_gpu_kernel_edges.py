@@ -449,3 +449,34 @@ def test_grid_divisions_of_special_values(value):
             there = ~np.isnan(a[k])
             assert np.array_equal(np.signbit(a[k][there]), np.signbit(b[k][there])), k
     g.close()
+
+
+# bodies of 8.5 cells set to 10.9 cells by an upload of their records: their
+# boxes of up to 900 cells fit the four slices of 256 made for 837, and have to
+# fit shorter ones (14 of 64 cells would hold 896).  Sums of 4e5 terms against
+# the oracle's serial ones, as for the slice lengths
+@pytest.mark.parametrize("n", [1, 400])
+def test_bodies_grown_by_their_records(n):
+    nx, ny, h = 256, 512, 1.0 / 256
+    kw = dict(itot=nx, jtot=ny, ly=2.0, Re=100.0)
+    g, o = eif.Solver(**kw), Oracle(**kw)
+    ux, uy, p = cases.random_fields(nx, ny, 5)
+    rng = np.random.default_rng(n)
+    parts = dict(den=np.ones(n), a=np.full(n, 8.5 * h), b=np.full(n, 8.5 * h),
+                 x=rng.uniform(0.2, 0.8, n), y=rng.uniform(0.2, 1.8, n), az=rng.uniform(0, 3, n))
+    parts["x"][0] = parts["y"][0] = 100.5 * h  # a box of 30 by 30
+    for s in (g, o):
+        s.upload(ux, uy, p)
+        s.update_boundaries()
+        s.set_dt(1e-3)
+        s.set_particles(**parts)
+        rec = s.particles()
+        rec[:, 1:3] = 10.9 * h
+        s.set_particle_records(rec)
+        s.reset_particle_increments()
+        s.compute_inertia(0)
+        s.exchange_momentum()
+        s.res = s.particles()[:, 15:24]
+    g.synchronize()  # raises where a box did not fit
+    assert np.max(np.abs(g.res - o.res)) <= 1e-12 * np.max(np.abs(o.res))
+    g.close()
