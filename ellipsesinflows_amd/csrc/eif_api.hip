@@ -194,7 +194,7 @@ static void free_ctx(Ctx *c) {
                     c->sc_key, c->heads, c->cl_start, c->cl_items, c->cl_cell, c->cl_slot, c->cl_count};
   for (auto o : others)
     if (o) (void)hipFree(o);
-  staging_free(c);
+  staging_leave(c);
   if (c->hscal) (void)hipHostFree(c->hscal);
   if (c->hstat) (void)hipHostFree(c->hstat);
   if (c->gstat) (void)hipHostFree(c->gstat);
@@ -253,6 +253,7 @@ int fluid_gpu_create(const eif_config *cfg, eif_ctx **out) {
     return r;
   };
   if (hipGetDevice(&c->device) != hipSuccess) return fail(hip_fail(hipErrorUnknown, "hipGetDevice", __FILE__, __LINE__));
+  staging_join(c);
   {
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking);

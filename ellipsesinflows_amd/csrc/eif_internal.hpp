@@ -254,7 +254,7 @@ struct Ctx {
   // pass (one on 128x128) gains 0.1 of 3.7 ms
   bool capturing = false;
   Profiler *prof = nullptr;
-  struct Staging *staging = nullptr;  // pinned slots of the downloads
+  bool staging = false;  // counted among the users of the device's download slots
 };
 
 // error state
@@ -276,7 +276,8 @@ struct Download {
 constexpr int DOWNLOAD_PARTS = 5;  // at most
 int download(Ctx *c, const Download *parts, int n);
 int download(Ctx *c, void *host, const void *dev, size_t bytes);
-void staging_free(Ctx *c);
+void staging_join(Ctx *c);
+void staging_leave(Ctx *c);
 
 // profiling helpers (host)
 // prof_begin: whether this launch is timed (then prof_end closes it)

@@ -1,6 +1,9 @@
 """Sizes at the edges of the kernels' tiles and of their launch rules, against
 the oracle (bit for bit where the kernels perform the reference's operations
 in its order)."""
+import concurrent.futures
+import os
+
 import numpy as np
 import pytest
 import torch
@@ -480,3 +483,51 @@ def test_bodies_grown_by_their_records(n):
     g.synchronize()  # raises where a box did not fit
     assert np.max(np.abs(g.res - o.res)) <= 1e-12 * np.max(np.abs(o.res))
     g.close()
+
+
+# downloads at the same time by six threads, more than there are sets of slots:
+# from one context and from each thread's own, through one slot and in strips
+@pytest.mark.parametrize("nx,ny", [(64, 96), (300, 290), (500, 700)])
+@pytest.mark.parametrize("shared", [True, False])
+def test_downloads_by_several_threads(nx, ny, shared):
+    ss = [eif.Solver(nx, ny, ly=1.0) for _ in range(1 if shared else 6)]
+    want = []
+    for k, s in enumerate(ss):
+        want.append(cases.random_fields(nx, ny, 31 * k + nx))
+        s.upload(*want[-1])
+
+    def work(t):
+        s, w = ss[t % len(ss)], want[t % len(ss)]
+        same = True
+        for _ in range(6):
+            d = s.download()
+            same &= all(np.array_equal(d[k], f.reshape(d[k].shape)) for k, f in zip(("ux", "uy", "p"), w))
+        return same
+
+    with concurrent.futures.ThreadPoolExecutor(6) as pool:
+        assert all(pool.map(work, range(6)))
+    for s in ss:
+        s.close()
+
+
+# the slots are a device's, not a context's: downloads of 10 MB from 24 contexts
+# one after the other, which need 4 MiB of slots, map less than 24 MiB (a set
+# for each would be 96)
+def test_downloads_of_many_contexts_share_their_slots():
+    ss = [eif.Solver(512, 800, ly=1.0) for _ in range(24)]
+    out = [np.zeros(ss[0].shapes[k]) for k in ("ux", "uy", "p")]
+
+    def download(s):
+        s._check(s.lib.fluid_gpu_download(s.h, *[eif._ptr(a) for a in out]))
+
+    def mapped():
+        with open("/proc/self/statm") as f:
+            return int(f.read().split()[0]) * os.sysconf("SC_PAGE_SIZE")
+
+    download(ss[0])
+    before = mapped()
+    for s in ss:
+        download(s)
+    assert mapped() - before < 24 << 20
+    for s in ss:
+        s.close()
