@@ -1679,15 +1679,19 @@ int eif_gpu_autotune(eif_ctx *c, int flags, char *report, int report_len) {
   std::string rep;
   char buf[160];
   int rc = EIF_OK;
-  // predictor rows per workgroup (same operations per cell for each)
+  // predictor rows per workgroup (same operations per cell for each): 8, 16
+  // and 32, then the short marches that an untuned context takes on grids that
+  // do not fill the GPU (2, 4); the report has the best of the first three and
+  // the best of all
   {
     double best = 1e30;
     int pick = 0;
     rep += "predictor_rows:";
-    for (int rows : {8, 16, 32}) {
+    for (int rows : {8, 16, 32, 2, 4}) {
       c->pred_rows = rows;
       double ms = 0.;
       if ((rc = time_launches(c, [&] { return launch_predictor_probe(c); }, 10, &ms))) break;
+      if (rows == 2) rep += " -> " + std::to_string(pick) + " or";
       snprintf(buf, sizeof(buf), " %d=%.4fms", rows, ms);
       rep += buf;
       if (ms < best) {

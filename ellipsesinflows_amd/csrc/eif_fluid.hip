@@ -123,7 +123,7 @@ int launch_bc_p(Ctx *c, double *p) {
 // registers and more waves per SIMD.
 // ---------------------------------------------------------------------
 constexpr int PRED_BX = 256;
-constexpr int PRED_ROWS = 16;  // most rows per workgroup by default (the tuner may pick 8 or 32)
+constexpr int PRED_ROWS = 16;  // most rows per workgroup by default (the tuner times 2 to 32)
 // Default rows per workgroup: a workgroup's march is a chain of rows, each
 // waiting for its loads, so a grid that does not fill the GPU is as long as
 // the march.  The rows go down to 2 until there are PRED_GROUPS workgroups

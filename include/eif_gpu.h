@@ -212,7 +212,7 @@ int eif_gpu_graph_stats(eif_ctx *ctx, long out[4]);
 
 /* Autotuner (no counterpart in the reference): times the candidate launch
  * shapes on this context's grid and keeps the fastest.  Rows per workgroup
- * of the predictor (8, 16, 32) and of the projection (4, 8, 16) and the
+ * of the predictor (2 to 32) and of the projection (4, 8, 16) and the
  * register FFT's values per thread (4, 8, 16: the same butterflies) change
  * no result.  The chunk length of the partitioned y-solve (16, 32, 64 rows
  * where they divide jtot), and in partition mode the fused projection (see

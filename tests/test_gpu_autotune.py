@@ -83,3 +83,16 @@ def test_tuned_shapes_copied_to_a_case_of_the_same_grid():
         other.tune_copy(src)
     for g in (src, dst, other):
         g.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 96), (256, 512)])
+def test_tuner_times_the_shapes_of_small_grids(nx, ny):
+    """The predictor's rows that an untuned context takes on a small grid are
+    among those timed, and the fastest of all is kept."""
+    g = eif.Solver(nx, ny, ly=2.0, Re=100.0)
+    rep = g.autotune()
+    g.close()
+    text = re.search(r"predictor_rows:(.*?);", rep).group(1)
+    times = {int(r): float(t) for r, t in re.findall(r" (\d+)=([\d.]+)ms", text)}
+    assert sorted(times) == [2, 4, 8, 16, 32], rep
+    assert times[int(text.split("->")[-1])] == min(times.values()), rep
