@@ -531,3 +531,51 @@ def test_downloads_of_many_contexts_share_their_slots():
     assert mapped() - before < 24 << 20
     for s in ss:
         s.close()
+
+
+def slice_length(nx, ny, ly, radii):
+    """cells a slice, by the library's rule: 256, halved to 64 at least while
+    the boxes make fewer than 2048 slices"""
+    dx, dy = 1.0 / nx, ly / ny
+    cells = 0
+    for r in radii:
+        wx, wy = min(int(2 * r / dx) + 10, nx), min(int(2 * r / dy) + 10, ny)
+        cells += wx * (wy + 4) if ly > 2 * r + 16 * dy else 3 * wx * wy
+    length = 256
+    while length > 64 and cells // length < 2048:
+        length //= 2
+    return length
+
+
+# slices of each length (100, 300 and 400 bodies of 1440 box cells), the
+# distances searched from a cold start, served from the cache and searched from
+# the last foot; sums of up to 6e5 terms against the oracle's serial ones:
+# 1e-12 of the largest member
+@pytest.mark.parametrize("n,length", [(100, 64), (300, 128), (400, 256)])
+def test_slices_of_each_length(n, length):
+    nx, ny, ly, a = 512, 1024, 2.0, 0.026
+    assert slice_length(nx, ny, ly, [a] * n) == length
+    kw = dict(itot=nx, jtot=ny, ly=ly, Re=100.0)
+    g, o = eif.Solver(**kw), Oracle(**kw)
+    ux, uy, p = cases.random_fields(nx, ny, 5)
+    rng = np.random.default_rng(n)
+    y = rng.uniform(0, 2, n)
+    y[0] = 1.999
+    parts = dict(den=np.ones(n), a=np.full(n, a), b=np.full(n, 0.6 * a), x=rng.uniform(0.2, 0.8, n),
+                 y=y, az=rng.uniform(0, 3, n))
+    for s in (g, o):
+        s.upload(ux, uy, p)
+        s.update_boundaries()
+        s.set_dt(1e-3)
+        s.set_particles(**parts)
+        s.reset_particle_increments()
+        s.compute_inertia(0)
+        s.exchange_momentum()
+        rec = s.particles()
+        rec[:, 6:9] = [2e-4, -1e-4, 1e-3]
+        s.set_particle_records(rec)
+        s.compute_inertia(1)
+    x, y = g.particles()[:, 15:24], o.particles()[:, 15:24]
+    assert np.max(np.abs(x - y)) <= 1e-12 * np.max(np.abs(y))
+    g.synchronize()
+    g.close()
