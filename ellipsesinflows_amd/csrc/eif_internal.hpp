@@ -57,7 +57,7 @@ constexpr int TILE_CAP = 48;     // boxes registered per tile
 constexpr int CONTACT_CAP = 64;  // colliding partners per particle
 constexpr int COLL_CELLS_MIN = 4096;  // particles from which the cell list is chosen
 constexpr int CELL_BUILD_MAX = 8192;  // particles up to which one workgroup builds the cell list
-constexpr int COLL_CELLS_CAP = 14336; // cells at most: their counts and a scan in 60 KiB of LDS
+constexpr int COLL_CELLS_CAP = 14336; // cells at most: their counts and a scan in 57 KiB of LDS
 constexpr int EQC_ITER_CAP = 100000;  // guard of the uncapped fixed point
 constexpr int DT_PARTS_CAP = 16384;   // workgroups of the projection with fused dt
 constexpr int RES_SLOTS = 128;        // sub-iterations of one stage queued at most
@@ -371,7 +371,7 @@ int launch_collision(Ctx *c, int cnstep, hipStream_t st = nullptr, bool packed =
 int launch_increment(Ctx *c, int rk, int sub = -1);
 // inertia(1) and collision(1) of sub-iteration `sub`, gated, in one launch
 int launch_substep_forces(Ctx *c, int sub);
-int launch_update_particles(Ctx *c, hipStream_t st = nullptr);
+int launch_update_particles(Ctx *c);
 // clear_tiles: also clear the IBM tile registrations for the next exchange;
 // update: the particle update first, in the same launch
 int launch_reset(Ctx *c, hipStream_t st = nullptr, bool clear_tiles = false,

@@ -25,8 +25,9 @@
 //     tiles then adds the contributions cell by cell in the reference's
 //     particle/image order and applies them to ux/uy (no atomics, no
 //     full-field pass);
-//   * collisions: one thread per particle pair finds the colliding pairs,
-//     one thread per particle gathers its partners' forces in the
+//   * collisions: one wave per particle finds the partners whose bounding
+//     circles reach it (all others, or the neighbours of a cell list), solves
+//     the contacts with two lanes each and adds their forces in the
 //     reference's pair order.
 #include "eif_ellipse.hpp"
 #include "eif_internal.hpp"
@@ -210,17 +211,13 @@ __device__ inline bool sub_open(const double *res, int sub) {
 }
 
 // The IBM, deposit and collision kernels give each wave its own slice, tile or
-// particle.  The waves of a workgroup (WG_WAVES) share nothing, so LDS is per
-// wave and ordered within the wave.  One wave a workgroup: four made the
-// collision launch 28 -> 41 us and left the others as they were (2048x4096,
-// 1024 ellipses; the dispatch of 11600 one-wave workgroups takes 3.6 us).
-constexpr int WG_WAVES = 1;
+// particle, one wave a workgroup: four made the collision launch 28 -> 41 us
+// and left the others as they were (2048x4096, 1024 ellipses; the dispatch of
+// 11600 one-wave workgroups takes 3.6 us).
+constexpr int WAVE = 64;
 __device__ inline int wave_lane() { return threadIdx.x & 63; }
 // the wave's place in the launch, known uniform
-__device__ inline int wave_index(const VB &vb) {
-  return __builtin_amdgcn_readfirstlane(vb.bx * WG_WAVES + (threadIdx.x >> 6));
-}
-__device__ inline int wave_in_group() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+__device__ inline int wave_index(const VB &vb) { return __builtin_amdgcn_readfirstlane(vb.bx); }
 // LDS written by the wave's lanes is visible to its other lanes
 __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -253,7 +250,7 @@ struct IbmArgs {
   unsigned long long *stats;  // per particle: cells, cells evaluated, FP64 and FP32 iterations
   double *cpos;               // np x 4: the broad phase's packed positions and radii
   int np;
-  int nslices, slice;      // slices, and box cells of each
+  int slice;               // box cells of each slice
   const int *slice_first;  // np+1: first slice of each particle
   const int4 *slice_rec;   // of each slice: its particle, the particle's first slice and slices
   long *slice_info;        // np x 2: box cells, cells evaluated (this call)
@@ -265,7 +262,7 @@ struct IbmArgs {
   double *slice_part0;
   double *slice_part;
   const int *halt;   // graph-step stop flag
-  SliceHead *heads;  // per particle: the pass's position, shape, boxes, cache state      // per-slice partial sums (3 each)
+  SliceHead *heads;  // per particle: the pass's position, shape, boxes, cache state
 };
 
 // x of lane i + n of the same row of 16 lanes (DPP row_shl:n, CTRL = 0x100 + n);
@@ -603,15 +600,14 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
 // U: cells a lane, slices of 64 U
 template <int U>
 struct InertiaB {
-  static constexpr int T = 64 * WG_WAVES, M = 4;
+  static constexpr int T = WAVE, M = 4;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, int cnstep) {
   if (halted(a.halt)) return;
-  const int slice = wave_index(vb);
-  if (slice < a.nslices) inertia_slice<U>(a, cnstep, slice, sub_open(a.res, a.sub));
+  inertia_slice<U>(a, cnstep, wave_index(vb), sub_open(a.res, a.sub));
 }
 };
 template <int U>
-__global__ __launch_bounds__(64 * WG_WAVES, 4) void k_inertia(IbmArgs a, int cnstep) {
+__global__ __launch_bounds__(WAVE, 4) void k_inertia(IbmArgs a, int cnstep) {
   InertiaB<U>::run(VB::here(), a, cnstep);
 }
 
@@ -782,12 +778,11 @@ __device__ inline void register_tile(const IbmArgs &a, int tile, int box_id) {
 // already hold them; sliced like k_inertia.  Used before k_exchange when
 // the cache may be stale.
 struct IbmDistB {
-  static constexpr int T = 64 * WG_WAVES, M = 0;
+  static constexpr int T = WAVE, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a) {
   if (halted(a.halt)) return;
   if (!sub_open(a.res, a.sub)) return;
   const int slice = wave_index(vb), lane = wave_lane();
-  if (slice >= a.nslices) return;
   const int4 rec = a.slice_rec[slice];
   const int n = rec.x, s0 = rec.y, nsl = rec.z;
   const SliceHead &hd = a.heads[n];
@@ -828,7 +823,7 @@ struct IbmDistB {
   }
 }
 };
-__global__ __launch_bounds__(64 * WG_WAVES) void k_ibm_dist(IbmArgs a) {
+__global__ __launch_bounds__(WAVE) void k_ibm_dist(IbmArgs a) {
   IbmDistB::run(VB::here(), a);
 }
 
@@ -841,11 +836,10 @@ __global__ __launch_bounds__(64 * WG_WAVES) void k_ibm_dist(IbmArgs a) {
 // The heads hold the particles' positions without increments.
 template <int U>
 struct ExchangeB {
-  static constexpr int T = 64 * WG_WAVES, M = 0;
+  static constexpr int T = WAVE, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, int own_counts) {
   if (halted(a.halt)) return;
   const int slice = wave_index(vb), lane = wave_lane();
-  if (slice >= a.nslices) return;
   const int4 rec = a.slice_rec[slice];
   const int n = rec.x, s0 = rec.y, nsl = rec.z;
   const double *q = a.prt + (long)n * R_N;
@@ -1001,7 +995,7 @@ struct ExchangeB {
 }
 };
 template <int U>
-__global__ __launch_bounds__(64 * WG_WAVES) void k_exchange(IbmArgs a, int own_counts) {
+__global__ __launch_bounds__(WAVE) void k_exchange(IbmArgs a, int own_counts) {
   ExchangeB<U>::run(VB::here(), a, own_counts);
 }
 
@@ -1010,7 +1004,7 @@ __global__ __launch_bounds__(64 * WG_WAVES) void k_exchange(IbmArgs a, int own_c
 // ---------------------------------------------------------------------
 struct TileArgs {
   Layout L;
-  int nx, ny, ntx, ntiles;
+  int nx, ny, ntx;
   const Box *boxes;
   const double *sc_fx, *sc_fy;
   const int *tile_cnt, *tile_list;
@@ -1032,18 +1026,13 @@ __device__ inline double box_value(const Box &b, const double *sc, int i, int j)
 // (particle index, then image; a box registered twice counts once), the
 // boxes are staged in LDS, and every cell sums its boxes' values in that
 // order.
-constexpr int TILE_THREADS = 64 * WG_WAVES;
 static_assert(TILE_X == 64, "one lane per tile column");
 static_assert(TILE_CAP <= 64, "one lane per registration");
 
 __device__ __forceinline__ void tile_body(const TileArgs &a, int tile) {
-  __shared__ int raw_[WG_WAVES][TILE_CAP];
-  __shared__ bool rep_[WG_WAVES][TILE_CAP];
-  __shared__ Box sbox_[WG_WAVES][TILE_CAP];
-  const int wv = wave_in_group();
-  int *raw = raw_[wv];
-  bool *rep = rep_[wv];
-  Box *sbox = sbox_[wv];
+  __shared__ int raw[TILE_CAP];
+  __shared__ bool rep[TILE_CAP];
+  __shared__ Box sbox[TILE_CAP];
   // tiles in grid order, so neighbouring workgroups touch neighbouring
   // memory; tiles no box reaches return at once
   const int cnt = min(a.tile_cnt[tile], TILE_CAP);
@@ -1135,14 +1124,13 @@ __device__ __forceinline__ void tile_body(const TileArgs &a, int tile) {
 }
 
 struct TilesB {
-  static constexpr int T = TILE_THREADS, M = 0;
+  static constexpr int T = WAVE, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, TileArgs a) {
   if (halted(a.halt)) return;
-  const int tile = wave_index(vb);
-  if (tile < a.ntiles) tile_body(a, tile);
+  tile_body(a, wave_index(vb));
 }
 };
-__global__ __launch_bounds__(TILE_THREADS) void k_tiles(TileArgs a) {
+__global__ __launch_bounds__(WAVE) void k_tiles(TileArgs a) {
   TilesB::run(VB::here(), a);
 }
 
@@ -1151,17 +1139,17 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tiles(TileArgs a) {
 // particle each, the rest are the tiles.  Neither reads what the other
 // writes.
 struct TilesX0B {
-  static constexpr int T = TILE_THREADS, M = 0;
+  static constexpr int T = WAVE, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, TileArgs t, IbmArgs a) {
   if (halted(a.halt)) return;
   const int k = wave_index(vb);
   if (k < a.np)
     finalize_x0_particle(a, k);
-  else if (k - a.np < t.ntiles)
+  else
     tile_body(t, k - a.np);
 }
 };
-__global__ __launch_bounds__(TILE_THREADS) void k_tiles_x0(TileArgs t, IbmArgs a) {
+__global__ __launch_bounds__(WAVE) void k_tiles_x0(TileArgs t, IbmArgs a) {
   TilesX0B::run(VB::here(), t, a);
 }
 
@@ -1437,9 +1425,8 @@ __device__ inline bool candidate(const CollArgs &a, int n, const Circle &me, int
 }
 
 __device__ void collide_particle(const CollArgs &a, int n) {
-  __shared__ int s_cand_[WG_WAVES][COLL_CAND_CAP];
-  __shared__ int s_sorted_[WG_WAVES][COLL_CAND_CAP];
-  int *s_cand = s_cand_[wave_in_group()], *s_sorted = s_sorted_[wave_in_group()];
+  __shared__ int s_cand[COLL_CAND_CAP];
+  __shared__ int s_sorted[COLL_CAND_CAP];
   // a long chain of dependent operations beside waves of short ones
   __builtin_amdgcn_s_setprio(3);
   const int lane = wave_lane();
@@ -1549,15 +1536,14 @@ __device__ void collide_particle(const CollArgs &a, int n) {
 
 // one wave per particle
 struct CollideB {
-  static constexpr int T = 64 * WG_WAVES, M = 0;
+  static constexpr int T = WAVE, M = 0;
   static __device__ __forceinline__ void run(const VB &vb, CollArgs a) {
   if (halted(a.halt)) return;
   if (!sub_open(a.res, a.sub)) return;
-  const int n = wave_index(vb);
-  if (n < a.np) collide_particle(a, n);
+  collide_particle(a, wave_index(vb));
 }
 };
-__global__ __launch_bounds__(64 * WG_WAVES) void k_collide(CollArgs a) {
+__global__ __launch_bounds__(WAVE) void k_collide(CollArgs a) {
   CollideB::run(VB::here(), a);
 }
 
@@ -1584,6 +1570,9 @@ __device__ inline int cell_of(const CollArgs &a, double x, double y) {
   const int cy = min(max((int)floor(yw * (1. / a.hy)), 0), a.ncy - 1);
   return cy * a.ncx + cx;
 }
+
+// sums of up to 16 waves at part[0] and their scan at part[32]
+constexpr int CELL_SCAN = 64;
 
 // cnt (nc counts in LDS) turned into exclusive offsets by the workgroup's
 // threads, part their partial sums; returns the total.  Each thread sums a
@@ -1685,7 +1674,7 @@ struct CellScanB {
     extern __shared__ int cl_lds[];
     const int nc = a.ncx * a.ncy;
     int *cnt = cl_lds;          // nc counts
-    int *part = cl_lds + nc;    // blockDim.x partial sums
+    int *part = cl_lds + nc;    // CELL_SCAN sums of the waves
     for (int k = threadIdx.x; k < nc; k += blockDim.x) {
       cnt[k] = counts[k];
       counts[k] = 0;
@@ -1722,20 +1711,20 @@ __global__ __launch_bounds__(256) void k_cell_place(CollArgs a) {
 // occupancy its registers would take from the slices.
 template <int U>
 struct InertiaCollideB {
-  static constexpr int T = 64 * WG_WAVES, M = 4;
+  static constexpr int T = WAVE, M = 4;
   static __device__ __forceinline__ void run(const VB &vb, IbmArgs a, CollArgs ca, int cnstep) {
   if (halted(a.halt)) return;
   const bool open = sub_open(a.res, a.sub);
   const int k = wave_index(vb);
   if (k < ca.np) {
     if (open) collide_particle(ca, k);
-  } else if (k - ca.np < a.nslices) {
+  } else {
     inertia_slice<U>(a, cnstep, k - ca.np, open);
   }
 }
 };
 template <int U>
-__global__ __launch_bounds__(64 * WG_WAVES, 4) void k_inertia_collide(IbmArgs a, CollArgs ca,
+__global__ __launch_bounds__(WAVE, 4) void k_inertia_collide(IbmArgs a, CollArgs ca,
                                                                       int cnstep) {
   InertiaCollideB<U>::run(VB::here(), a, ca, cnstep);
 }
@@ -2023,7 +2012,6 @@ static IbmArgs ibm_args(Ctx *c) {
   a.stats = c->ibm_pp;
   a.cpos = c->cpos;
   a.np = c->np;
-  a.nslices = c->nslices;
   a.slice = c->slice_len;
   a.slice_first = c->slice_first;
   a.slice_rec = c->slice_rec;
@@ -2038,9 +2026,6 @@ static IbmArgs ibm_args(Ctx *c) {
   return a;
 }
 
-// workgroups of n waves
-static dim3 wave_grid(long n) { return dim3((unsigned)((n + WG_WAVES - 1) / WG_WAVES)); }
-
 // f(cells a lane) for the context's slices
 template <class F>
 static void by_slice(const Ctx *c, F f) {
@@ -2053,13 +2038,13 @@ static void by_slice(const Ctx *c, F f) {
 static void go_inertia(Ctx *c, const IbmArgs &a, int cnstep, hipStream_t st) {
   by_slice(c, [&](auto u) {
     constexpr int U = decltype(u)::value;
-    go<InertiaB<U>>(k_inertia<U>, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, st, a, cnstep);
+    go<InertiaB<U>>(k_inertia<U>, dim3(c->nslices), dim3(WAVE), 0, st, a, cnstep);
   });
 }
 static void go_exchange(Ctx *c, const IbmArgs &a, int own_counts) {
   by_slice(c, [&](auto u) {
     constexpr int U = decltype(u)::value;
-    go<ExchangeB<U>>(k_exchange<U>, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a,
+    go<ExchangeB<U>>(k_exchange<U>, dim3(c->nslices), dim3(WAVE), 0, c->stream, a,
                      own_counts);
   });
 }
@@ -2186,7 +2171,7 @@ int launch_exchange(Ctx *c, bool cached_known, bool tiles_clear, bool defer_fina
   IbmArgs a = ibm_args(c);
   go<HeadsB>(k_heads, dim3((c->np + 3) / 4), dim3(256), 0, c->stream, a, 0);
   if (!cached_known)
-    go<IbmDistB>(k_ibm_dist, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, c->stream, a);
+    go<IbmDistB>(k_ibm_dist, dim3(c->nslices), dim3(WAVE), 0, c->stream, a);
   go_exchange(c, a, cached_known ? 1 : 0);
   EIF_HIP(hipGetLastError());
   if (!defer_finalize) return launch_exchange_finalize(c, c->stream);
@@ -2197,7 +2182,7 @@ int launch_exchange(Ctx *c, bool cached_known, bool tiles_clear, bool defer_fina
 // positions without increments, into the per-cell cache
 int launch_ibm_dist(Ctx *c, hipStream_t st) {
   if (c->np == 0) return EIF_OK;
-  go<IbmDistB>(k_ibm_dist, wave_grid(c->nslices), dim3(64 * WG_WAVES), 0, st ? st : c->stream,
+  go<IbmDistB>(k_ibm_dist, dim3(c->nslices), dim3(WAVE), 0, st ? st : c->stream,
                      ibm_args(c));
   EIF_HIP(hipGetLastError());
   return EIF_OK;
@@ -2218,7 +2203,7 @@ int launch_exchange_inertia0(Ctx *c, const double *us_x, const double *us_y) {
   return EIF_OK;
 }
 
-// the exchange's per-particle sums (slice order); nothing on the fluid side
+// the exchange's per-particle sums; nothing on the fluid side
 // reads them, so this may run on another stream after the exchange
 int launch_exchange_finalize(Ctx *c, hipStream_t st) {
   if (c->np == 0) return EIF_OK;
@@ -2233,7 +2218,6 @@ static TileArgs tile_args(Ctx *c, int apply) {
   t.nx = c->nx;
   t.ny = c->ny;
   t.ntx = c->ntx;
-  t.ntiles = c->ntx * c->nty;
   t.boxes = c->boxes;
   t.sc_fx = c->sc_fx;
   t.sc_fy = c->sc_fy;
@@ -2254,7 +2238,7 @@ int launch_update_momentum(Ctx *c) {
   if (c->np == 0) return EIF_OK;
   ProfScope ps(c, "ibm_apply");
   TileArgs t = tile_args(c, 1);
-  go<TilesB>(k_tiles, wave_grid(tile_count(c)), dim3(TILE_THREADS), 0, c->stream, t);
+  go<TilesB>(k_tiles, dim3((unsigned)tile_count(c)), dim3(WAVE), 0, c->stream, t);
   EIF_HIP(hipGetLastError());
   return EIF_OK;
 }
@@ -2264,7 +2248,7 @@ int launch_update_momentum_x0(Ctx *c) {
   if (c->np == 0) return EIF_OK;
   ProfScope ps(c, "ibm_apply");
   TileArgs t = tile_args(c, 1);
-  go<TilesX0B>(k_tiles_x0, wave_grid(c->np + tile_count(c)), dim3(TILE_THREADS), 0, c->stream,
+  go<TilesX0B>(k_tiles_x0, dim3((unsigned)(c->np + tile_count(c))), dim3(WAVE), 0, c->stream,
                      t, ibm_args(c));
   EIF_HIP(hipGetLastError());
   return EIF_OK;
@@ -2276,7 +2260,7 @@ int launch_materialise_du(Ctx *c) {
   EIF_HIP(hipMemsetAsync(c->duy, 0, bytes, c->stream));
   if (c->np > 0) {
     TileArgs t = tile_args(c, 0);
-    go<TilesB>(k_tiles, wave_grid(tile_count(c)), dim3(TILE_THREADS), 0, c->stream,
+    go<TilesB>(k_tiles, dim3((unsigned)tile_count(c)), dim3(WAVE), 0, c->stream,
                        t);
     EIF_HIP(hipGetLastError());
   }
@@ -2372,7 +2356,7 @@ static CollArgs coll_args(Ctx *c, int cnstep) {
 // the cell list for a collision launch with these (gated) arguments
 static void launch_cell_list(Ctx *c, const CollArgs &a, hipStream_t st) {
   if (!a.use_cells) return;
-  const size_t lds = ((size_t)c->cl_ncx * c->cl_ncy + 1024) * sizeof(int);
+  const size_t lds = ((size_t)c->cl_ncx * c->cl_ncy + CELL_SCAN) * sizeof(int);
   if (c->np <= CELL_BUILD_MAX) {
     go<CellBuildB>(k_cell_build, dim3(1), dim3(CellBuildB::T), lds, st, a);
     return;
@@ -2390,7 +2374,7 @@ int launch_collision(Ctx *c, int cnstep, hipStream_t st, bool packed) {
   const CollArgs a = coll_args(c, cnstep);
   if (!packed) go<CollPackB>(k_coll_pack, dim3((c->np + 255) / 256), dim3(256), 0, st, a);
   launch_cell_list(c, a, st);
-  go<CollideB>(k_collide, wave_grid(c->np), dim3(64 * WG_WAVES), 0, st, a);
+  go<CollideB>(k_collide, dim3(c->np), dim3(WAVE), 0, st, a);
   EIF_HIP(hipGetLastError());
   return EIF_OK;
 }
@@ -2417,7 +2401,7 @@ int launch_substep_forces(Ctx *c, int sub) {
   const bool timed = prof_kernel_events(c, "ibm_substep", &e0, &e1);
   by_slice(c, [&](auto u) {
     constexpr int U = decltype(u)::value;
-    const dim3 grid = wave_grid(c->np + c->nslices), block(64 * WG_WAVES);
+    const dim3 grid(c->np + c->nslices), block(WAVE);
     if (timed)  // a sampled launch stamps its events
       hipExtLaunchKernelGGL(k_inertia_collide<U>, grid, block, 0, c->stream, e0, e1, 0, a, ca, 1);
     else
@@ -2538,10 +2522,10 @@ int launch_graph_status(Ctx *c) {
   return EIF_OK;
 }
 
-int launch_update_particles(Ctx *c, hipStream_t st) {
+int launch_update_particles(Ctx *c) {
   if (c->np == 0) return EIF_OK;
   go<UpdateParticlesB>(k_update_particles, dim3((c->np + 255) / 256), dim3(256), 0,
-                     st ? st : c->stream, c->prt, c->np, c->ly, c->halt);
+                     c->stream, c->prt, c->np, c->ly, c->halt);
   EIF_HIP(hipGetLastError());
   return EIF_OK;
 }
