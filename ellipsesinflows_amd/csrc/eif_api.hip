@@ -838,7 +838,7 @@ static int stage_start(Ctx *c, int rk, bool pred_queued, bool side_start) {
     EIF_HIP(hipStreamWaitEvent(c->side, c->ev_fork, 0));
     TRY(launch_ibm_dist(c, c->side));
     EIF_HIP(hipEventRecord(c->ev_i0, c->side));
-    TRY(launch_collision(c, 0, c->side, !c->capturing));
+    TRY(launch_collision(c, 0, c->side, true));
     EIF_HIP(hipEventRecord(c->ev_c0, c->side));
     EIF_HIP(hipStreamWaitEvent(c->stream, c->ev_i0, 0));
   } else if (side_start) {
@@ -853,7 +853,7 @@ static int stage_start(Ctx *c, int rk, bool pred_queued, bool side_start) {
     TRY(launch_reset(c, c->side, true, true));
     TRY(launch_ibm_dist(c, c->side));
     EIF_HIP(hipEventRecord(c->ev_i0, c->side));
-    TRY(launch_collision(c, 0, c->side, !c->capturing));
+    TRY(launch_collision(c, 0, c->side, true));
     EIF_HIP(hipEventRecord(c->ev_c0, c->side));
     EIF_HIP(hipStreamWaitEvent(c->stream, c->ev_i0, 0));
   } else {
@@ -868,7 +868,7 @@ static int stage_start(Ctx *c, int rk, bool pred_queued, bool side_start) {
     TRY(launch_ibm_dist(c));
     EIF_HIP(hipEventRecord(c->ev_fork, c->stream));
     EIF_HIP(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-    TRY(launch_collision(c, 0, c->side, !c->capturing));
+    TRY(launch_collision(c, 0, c->side, true));
     EIF_HIP(hipEventRecord(c->ev_c0, c->side));
   }
   // the exchange with the predicted velocity and, in the same pass,
@@ -1045,9 +1045,7 @@ static int capture_step(Ctx *c, const int K[3], GraphEntry *out) {
   hipGraph_t graph = nullptr;
   EIF_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   out->dt_parts = 0;
-  c->capturing = true;
   const int rc = queue_graph_step(c, K, out->at_gate);
-  c->capturing = false;
   const hipError_t e = hipStreamEndCapture(c->stream, &graph);
   c->prof->on = prof_was;
   const PtrState end = save_ptrs(c);

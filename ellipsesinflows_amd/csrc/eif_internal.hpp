@@ -248,11 +248,6 @@ struct Ctx {
   double *st_ux1 = nullptr, *st_ux2 = nullptr;                   // like ux
   double *st_uy1 = nullptr, *st_uy2 = nullptr, *st_phi = nullptr;  // like uy
   int st_num = 0;
-  // a single case's step is being captured.  Its collision(0) keeps the launch
-  // that packs the positions (k_reset has packed them): replayed without it,
-  // 64 ellipses on 512x1024 took 10.27 ms instead of 9.91, while an eager
-  // pass (one on 128x128) gains 0.1 of 3.7 ms
-  bool capturing = false;
   Profiler *prof = nullptr;
   bool staging = false;  // counted among the users of the device's download slots
 };
