@@ -544,48 +544,63 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
   int it64 = 0, it32 = 0;
   const int t0 = (slice - s0) * (64 * U);
   const int t1 = t0 + 64 * U < total ? t0 + 64 * U : total;
-  // all loads of the lane's cells first (a cell past t1 loads the last cell
-  // instead and is not added), then the weights and the sums in cell order
-  if (t0 < t1) {
-    double th_[U] = {}, x_[U], y_[U], vx0[U], vx1[U], vy0[U], vy1[U];
-    int k_[U], i_[U], j_[U];
-    lane_cells<U>(bs, t0, t1, lane, k_, i_, j_);
+  auto add = [&](int k, double x, double y, double th, double vx0, double vx1, double vy0,
+                 double vy1) {
+    const double py_ = py + a.ly * (k - 1);
+    const double w = v_weight_th(th);
+    const double valx = w * 0.5 * (vx0 + vx1) * dxdy;
+    const double valy = w * 0.5 * (vy0 + vy1) * dxdy;
+    acc[0] += valx * inv_pm;
+    acc[2] += -(y - py_) * valx * inv_pim;
+    acc[1] += valy * inv_pm;
+    acc[2] += +(x - px) * valy * inv_pim;
+  };
+  if (cached) {
+    // all loads of the lane's cells first (a cell past t1 loads the last cell
+    // instead and is not added), then the sums in cell order
+    if (t0 < t1) {
+      double th_[U], x_[U], y_[U], vx0[U], vx1[U], vy0[U], vy1[U];
+      int k_[U], i_[U], j_[U];
+      lane_cells<U>(bs, t0, t1, lane, k_, i_, j_);
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const unsigned fx = face_x(a.L, i_[u], j_[u]), fy = face_y(a.L, i_[u], j_[u]);
-      x_[u] = a.xc[i_[u]];
-      y_[u] = a.yc[j_[u] - 1];
-      vx0[u] = a.ux[fx];
-      vx1[u] = a.ux[fx + 1];
-      vy0[u] = a.uy[fy];
-      vy1[u] = a.uy[fy + (unsigned)(a.nx + 2)];
+      for (int u = 0; u < U; u++) {
+        const unsigned fx = face_x(a.L, i_[u], j_[u]), fy = face_y(a.L, i_[u], j_[u]);
+        x_[u] = a.xc[i_[u]];
+        y_[u] = a.yc[j_[u] - 1];
+        th_[u] = dist[min(t0 + lane + 64 * u, t1 - 1)];
+        vx0[u] = a.ux[fx];
+        vx1[u] = a.ux[fx + 1];
+        vy0[u] = a.uy[fy];
+        vy1[u] = a.uy[fy + (unsigned)(a.nx + 2)];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (t0 + lane + 64 * u < t1)
+          add(k_[u], x_[u], y_[u], th_[u], vx0[u], vx1[u], vy0[u], vy1[u]);
     }
-    // th, or the foot's parameter that its search starts from
-    if (cached || warm) {
-      const double *from = cached ? dist : tcell;
-#pragma unroll
-      for (int u = 0; u < U; u++) th_[u] = from[min(t0 + lane + 64 * u, t1 - 1)];
-    }
-#pragma unroll
+  } else {
+    // a cell at a time: the loads of U = 4 cells held through four searches
+    // took more than the 128 VGPRs there are, and 60 steps at 2048x4096 with
+    // 1024 ellipses 127.4 ms instead of 124.3
+    const bool single = single_image(bs);
+#pragma nounroll
     for (int u = 0; u < U; u++) {
       const int t = t0 + lane + 64 * u;
-      if (t >= t1) continue;
-      const double py_ = py + a.ly * (k_[u] - 1);
-      const double x = x_[u], y = y_[u];
-      if (!cached) {
-        double tf = th_[u];
-        th_[u] = weight_th(signed_dist_from(e, f, 1. / a.grid_size, px, py_, cr, sr, x, y, warm,
-                                            tf, it32, it64));
-        tcell[t] = tf;
-        dist[t] = th_[u];
-      }
-      const double w = v_weight_th(th_[u]);
-      const double valx = w * 0.5 * (vx0[u] + vx1[u]) * dxdy;
-      const double valy = w * 0.5 * (vy0[u] + vy1[u]) * dxdy;
-      acc[0] += valx * inv_pm;
-      acc[2] += -(y - py_) * valx * inv_pim;
-      acc[1] += valy * inv_pm;
-      acc[2] += +(x - px) * valy * inv_pim;
+      if (t >= t1) break;
+      int k, i, j;
+      cell_of(bs, t, k, i, j, single);
+      const double x = a.xc[i], y = a.yc[j - 1];
+      // the velocities do not depend on the distance: loaded first
+      const unsigned fx = face_x(a.L, i, j), fy = face_y(a.L, i, j);
+      const double vx0 = a.ux[fx], vx1 = a.ux[fx + 1];
+      const double vy0 = a.uy[fy], vy1 = a.uy[fy + (unsigned)(a.nx + 2)];
+      double tf = warm ? tcell[t] : 0.;
+      const double th = weight_th(signed_dist_from(e, f, 1. / a.grid_size, px,
+                                                   py + a.ly * (k - 1), cr, sr, x, y, warm, tf,
+                                                   it32, it64));
+      tcell[t] = tf;
+      dist[t] = th;
+      add(k, x, y, th, vx0, vx1, vy0, vy1);
     }
   }
   double part[SLICE_VALS] = {wave_sum(acc[0]), wave_sum(acc[1]), wave_sum(acc[2])};
