@@ -579,28 +579,44 @@ __device__ __forceinline__ void inertia_slice(const IbmArgs &a, int cnstep, int 
           add(k_[u], x_[u], y_[u], th_[u], vx0[u], vx1[u], vy0[u], vy1[u]);
     }
   } else {
-    // a cell at a time: the loads of U = 4 cells held through four searches
-    // took more than the 128 VGPRs there are, and 60 steps at 2048x4096 with
-    // 1024 ellipses 127.4 ms instead of 124.3
-    const bool single = single_image(bs);
+    // G cells at a time, their loads first (they do not depend on the
+    // distance).  Of U = 4 one: four cells' loads held through four searches
+    // take more than the 128 VGPRs there are, and 60 steps at 2048x4096 with
+    // 1024 ellipses 127.4 ms instead of 124.3.  Of U = 2 both: eight cases
+    // advanced together take 34.3 ms, 35.0 one at a time
+    constexpr int G = U > 2 ? 1 : U;
 #pragma nounroll
-    for (int u = 0; u < U; u++) {
-      const int t = t0 + lane + 64 * u;
-      if (t >= t1) break;
-      int k, i, j;
-      cell_of(bs, t, k, i, j, single);
-      const double x = a.xc[i], y = a.yc[j - 1];
-      // the velocities do not depend on the distance: loaded first
-      const unsigned fx = face_x(a.L, i, j), fy = face_y(a.L, i, j);
-      const double vx0 = a.ux[fx], vx1 = a.ux[fx + 1];
-      const double vy0 = a.uy[fy], vy1 = a.uy[fy + (unsigned)(a.nx + 2)];
-      double tf = warm ? tcell[t] : 0.;
-      const double th = weight_th(signed_dist_from(e, f, 1. / a.grid_size, px,
-                                                   py + a.ly * (k - 1), cr, sr, x, y, warm, tf,
-                                                   it32, it64));
-      tcell[t] = tf;
-      dist[t] = th;
-      add(k, x, y, th, vx0, vx1, vy0, vy1);
+    for (int c0 = 0; c0 < U; c0 += G) {
+      const int b0 = t0 + 64 * c0;
+      if (b0 >= t1) break;
+      double tf[G] = {}, x_[G], y_[G], vx0[G], vx1[G], vy0[G], vy1[G];
+      int k_[G], i_[G], j_[G];
+      lane_cells<G>(bs, b0, t1, lane, k_, i_, j_);
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const unsigned fx = face_x(a.L, i_[u], j_[u]), fy = face_y(a.L, i_[u], j_[u]);
+        x_[u] = a.xc[i_[u]];
+        y_[u] = a.yc[j_[u] - 1];
+        vx0[u] = a.ux[fx];
+        vx1[u] = a.ux[fx + 1];
+        vy0[u] = a.uy[fy];
+        vy1[u] = a.uy[fy + (unsigned)(a.nx + 2)];
+      }
+      if (warm) {
+#pragma unroll
+        for (int u = 0; u < G; u++) tf[u] = tcell[min(b0 + lane + 64 * u, t1 - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const int t = b0 + lane + 64 * u;
+        if (t >= t1) continue;
+        const double th = weight_th(signed_dist_from(e, f, 1. / a.grid_size, px,
+                                                     py + a.ly * (k_[u] - 1), cr, sr, x_[u], y_[u],
+                                                     warm, tf[u], it32, it64));
+        tcell[t] = tf[u];
+        dist[t] = th;
+        add(k_[u], x_[u], y_[u], th, vx0[u], vx1[u], vy0[u], vy1[u]);
+      }
     }
   }
   double part[SLICE_VALS] = {wave_sum(acc[0]), wave_sum(acc[1]), wave_sum(acc[2])};
