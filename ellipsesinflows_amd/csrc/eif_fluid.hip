@@ -128,7 +128,8 @@ constexpr int PRED_ROWS = 16;  // most rows per workgroup by default (the tuner 
 // waiting for its loads, so a grid that does not fill the GPU is as long as
 // the march.  The rows go down to 2 until there are PRED_GROUPS workgroups
 // (two a CU): 16.7 -> 4.8 us at 128x128 (2 rows), 18.4 -> 10.3 at 512x1024 (4),
-// 28.4 -> 23.1 at 768x1536 (8); from 1024x2048 on 16 rows are the fastest.
+// 28.4 -> 23.1 at 768x1536 (8; 25.9 since qdiv looks for special quotients);
+// from 1024x2048 on 16 rows are the fastest.
 constexpr int PRED_GROUPS = 512;
 enum { PRED_STORE = 0, PRED_PREV = 1, PRED_SRC = 2, PRED_NOB = 3 };
 // bit MODE set: that mode loads a row ahead.  The row loop is unrolled

@@ -194,8 +194,9 @@ constexpr int IBM_THREADS = 256;
 // its cells four, two or one a lane in turn, so a launch too small to fill
 // the GPU is as long as that turn: with 64 cells k_inertia_collide took 10.0
 // -> 7.0 us and k_ibm_dist 10.2 -> 6.1 at 64 ellipses on 512x1024 (2600
-// waves), 8.5 -> 5.1 and 10.7 -> 5.2 at one on 128x128; at 11600 waves (1024
-// ellipses on 2048x4096) shorter slices only repeat the waves' prologue.
+// waves), 8.5 -> 5.1 and 10.7 -> 5.2 at one on 128x128 (with a shorter foot
+// search than now, when the launches take 7.4, 6.1, 5.0 and 5.2); at 11600 waves
+// (1024 ellipses on 2048x4096) shorter slices only repeat the waves' prologue.
 constexpr int IBM_SLICE = 256;
 constexpr int IBM_WAVES = 2048;
 constexpr int SLICE_VALS = 5;   // per-slice partials: 3 sums, FP64 and FP32 iterations
@@ -1435,8 +1436,9 @@ __device__ bool contact_force(const CollArgs &a, int n0, int n1, int wall, int s
 // The launch is as long as one wave's chain of dependent loads and FP64
 // operations, so loads are taken together (four partners a lane; the nine
 // cells as three runs), the wave goes before others on its SIMD, and what
-// only the last fit or an overlap needs is left to the end: k_inertia_collide 38.2 ->
-// 35.3 us at 4096 ellipses on 1024x2048, 33.0 -> 31.6 at 1024 on 2048x4096.
+// only the last fit or an overlap needs is left to the end: k_inertia_collide
+// 38.2 -> 35.3 us at 4096 ellipses on 1024x2048, 33.0 -> 31.6 at 1024 on
+// 2048x4096 (with a shorter foot search than now: 43 and 46 us).
 constexpr int COLL_CAND_CAP = 256;  // candidate partners per particle
 
 // the lanes' partners that hit, appended to s_cand
